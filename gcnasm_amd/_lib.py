@@ -196,6 +196,7 @@ SIGNATURES = {
     "ga_quant_fp8_1x128": (_i, [_vp, _i, _i, _i, _i, _vp, _i, _vp, _i, _vp]),
     "ga_quant_fp8_128x128": (_i, [_vp, _i, _i, _i, _i, _vp, _i, _vp, _i, _vp]),
     "ga_quant_fp8_per_tensor": (_i, [_vp, _i, _sz, _vp, _vp, _vp, _vp]),
+    "ga_quant_fp8_per_tensor_ws": (_i, [_vp, _i, _sz, _vp, _vp, _vp, _sz, _vp]),
     "ga_kernel_find": (_i, [ctypes.c_char_p, ctypes.POINTER(_i)]),
     "ga_kernel_workspace_bytes": (_sz, [_i, ctypes.POINTER(LaunchDesc), _i, _i]),
     "ga_kernel_launch": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, _i, _vp, _sz, _vp]),

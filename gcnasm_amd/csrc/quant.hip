@@ -352,75 +352,117 @@ __global__ __launch_bounds__(kTileThreads) void quant_128x128_kernel(
         sfb[(size_t)rb * ld_s + g] = sc;
 }
 
-// ---- per-tensor: zero, amax (atomicMax on the bits of |x|), quantise --------
-// Both passes stream x with U loads of 16 bytes (f32) or 8 bytes (bf16) in
-// flight per lane; the scalar tail (n % 4) is handled by block 0.
+// ---- per-tensor: amax, quantise -------------------------------------------------
+// Both passes stream x with U loads of 16 bytes (bf16 8 bytes where x or q
+// does not allow 16) in flight per lane; the scalar tail (n % EPL) is handled
+// by block 0. The maximum is reduced over the workgroup first: one word per
+// workgroup leaves the first pass, either to its place among at most kAmaxParts
+// partial maxima, which every workgroup of the second pass reduces again (4 KB
+// from L2), or, where the caller's scratch is one word, by an atomic that is
+// skipped when the word already holds as much. One atomic per wave (8192 on
+// one word, each a round trip to memory from its XCD) took 98 us at 4096x4096
+// bf16, whose bytes take 5. Measured on MI355X, these two passes and a 4096^3
+// product (54 us): 160.8 us then, 69.0 with the partial maxima.
 constexpr int kTensorU = 4;
+constexpr int kAmaxParts = 1024;
 
 __global__ void zero_u32_kernel(uint32_t* p) { *p = 0u; }
 
-template <int IN>
-__global__ __launch_bounds__(256) void amax_kernel(const void* __restrict__ x, size_t n,
-                                                   uint32_t* __restrict__ amax_bits)
+// Maximum over the 256 threads of a workgroup, in every thread.
+__device__ __forceinline__ uint32_t block_max(uint32_t a)
 {
-    uint32_t a = 0u;
-    const size_t n4 = n / 4;
-    const size_t stride = (size_t)gridDim.x * 256;
-    for (size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x; i0 < n4; i0 += stride * kTensorU) {
-        float v[kTensorU][4];
-#pragma unroll
-        for (int u = 0; u < kTensorU; u++) {
-            const size_t i = i0 + u * stride;
-            load_elems<IN, 4>(x, i * 4, i < n4, v[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < kTensorU; u++)
-            a = max(a, amax_n<4>(v[u]));
-    }
-    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
-        size_t i = n4 * 4 + threadIdx.x;
-        float v = IN == GA_IN_F32 ? ((const float*)x)[i] : bf16_to_f32(((const uint16_t*)x)[i]);
-        a = max(a, abs_key(v));
-    }
+    __shared__ uint32_t wmax[4];
     a = group_max_dpp<32>(a);
     a = max(a, (uint32_t)__shfl_xor((int)a, 32, 64));
-    if ((threadIdx.x & 63) == 0 && a > 0u)
-        atomicMax(amax_bits, a);
+    if ((threadIdx.x & 63) == 0)
+        wmax[threadIdx.x >> 6] = a;
+    __syncthreads();
+    return max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
 }
 
 template <int IN>
+__device__ __forceinline__ float load_one(const void* x, size_t i)
+{
+    return IN == GA_IN_F32 ? ((const float*)x)[i] : bf16_to_f32(((const uint16_t*)x)[i]);
+}
+
+// PARTS: out[blockIdx.x] = this workgroup's maximum, else atomicMax on out[0].
+template <int IN, int EPL, bool PARTS>
+__global__ __launch_bounds__(256) void amax_kernel(const void* __restrict__ x, size_t n,
+                                                   uint32_t* __restrict__ out)
+{
+    uint32_t a = 0u;
+    const size_t nv = n / EPL;
+    const size_t stride = (size_t)gridDim.x * 256;
+    for (size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x; i0 < nv; i0 += stride * kTensorU) {
+        float v[kTensorU][EPL];
+#pragma unroll
+        for (int u = 0; u < kTensorU; u++) {
+            const size_t i = i0 + u * stride;
+            load_elems<IN, EPL>(x, i * EPL, i < nv, v[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kTensorU; u++)
+            a = max(a, amax_n<EPL>(v[u]));
+    }
+    if (blockIdx.x == 0 && threadIdx.x < n % EPL)
+        a = max(a, abs_key(load_one<IN>(x, nv * EPL + threadIdx.x)));
+    a = block_max(a);
+    if (threadIdx.x == 0) {
+        if constexpr (PARTS)
+            out[blockIdx.x] = a;
+        else if (a > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax(out, a);
+    }
+}
+
+template <int IN, int EPL>
 __global__ __launch_bounds__(256) void quant_tensor_kernel(const void* __restrict__ x, size_t n,
                                                            const uint32_t* __restrict__ amax_bits,
-                                                           uint8_t* __restrict__ q,
+                                                           int nparts, uint8_t* __restrict__ q,
                                                            float* __restrict__ scale)
 {
-    const float sc = ds_scale(__uint_as_float(*amax_bits));
+    uint32_t am = 0u;
+    if (nparts == 1) {
+        am = *amax_bits;
+    } else {
+        for (int i = threadIdx.x; i < nparts; i += 256)
+            am = max(am, amax_bits[i]);
+        am = block_max(am);
+    }
+    const float sc = ds_scale(__uint_as_float(am));
     const ScaleDiv d(sc);
     if (blockIdx.x == 0 && threadIdx.x == 0)
         *scale = sc;
-    const size_t n4 = n / 4;
+    const size_t nv = n / EPL;
     const size_t stride = (size_t)gridDim.x * 256;
-    for (size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x; i0 < n4; i0 += stride * kTensorU) {
-        float v[kTensorU][4];
+    for (size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x; i0 < nv; i0 += stride * kTensorU) {
+        float v[kTensorU][EPL];
 #pragma unroll
         for (int u = 0; u < kTensorU; u++) {
             const size_t i = i0 + u * stride;
-            load_elems<IN, 4>(x, i * 4, i < n4, v[u]);
+            load_elems<IN, EPL>(x, i * EPL, i < nv, v[u]);
         }
 #pragma unroll
         for (int u = 0; u < kTensorU; u++) {
             const size_t i = i0 + u * stride;
-            if (i < n4) {
-                float t[4];
+            if (i < nv) {
+                float t[EPL];
                 d.div(v[u], t);
-                *(uint32_t*)(q + i * 4) = e4m3_encode4(t[0], t[1], t[2], t[3]);
+                if constexpr (EPL == 8) {
+                    uint2 w;
+                    w.x = e4m3_encode4(t[0], t[1], t[2], t[3]);
+                    w.y = e4m3_encode4(t[4], t[5], t[6], t[7]);
+                    *(uint2*)(q + i * 8) = w;
+                } else {
+                    *(uint32_t*)(q + i * 4) = e4m3_encode4(t[0], t[1], t[2], t[3]);
+                }
             }
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
-        size_t i = n4 * 4 + threadIdx.x;
-        float v = IN == GA_IN_F32 ? ((const float*)x)[i] : bf16_to_f32(((const uint16_t*)x)[i]);
-        const float vv[1] = {v};
+    if (blockIdx.x == 0 && threadIdx.x < n % EPL) {
+        const size_t i = nv * EPL + threadIdx.x;
+        const float vv[1] = {load_one<IN>(x, i)};
         float t[1];
         d.div(vv, t);
         q[i] = (uint8_t)e4m3_encode(t[0]);
@@ -486,14 +528,6 @@ static inline unsigned grid1d(long long work, int per_block)
 
 using namespace ga;
 
-#define GA_DISPATCH_IN(in_dtype, KERNEL, ...)                                      \
-    do {                                                                           \
-        if ((in_dtype) == GA_IN_F32)                                               \
-            hipLaunchKernelGGL(KERNEL<GA_IN_F32>, __VA_ARGS__);                    \
-        else                                                                       \
-            hipLaunchKernelGGL(KERNEL<GA_IN_BF16>, __VA_ARGS__);                   \
-    } while (0)
-
 // 1x32 / 1x128 blocks per lane: two for fp32 and 8-byte bf16 loads, one for
 // 16-byte bf16 loads (16-32 bytes in flight per lane). Measured on MI355X at
 // 8192x8192 (fraction of 8 TB/s, 4 blocks -> this): MX E4M3 fp32 0.70 -> 0.73,
@@ -528,6 +562,29 @@ static void launch_quant_mx(int in_dtype, bool wide, long long blocks, hipStream
     else
         hipLaunchKernelGGL((quant_mx_kernel<GA_IN_BF16, 4, FP4, kQU, E5>), dim3(grid), dim3(256),
                            0, st, x, rows, K, ld_x, q, ld_q, s, ld_s, rule);
+}
+
+// The partial maxima take one word per workgroup of the first pass, so its
+// grid is what the scratch holds, at most kAmaxParts; a scratch of fewer words
+// than the workgroups that keep every CU streaming (kAmaxParts, or one per
+// 256 * EPL elements) is used as one word.
+template <int IN, int EPL>
+static void launch_quant_tensor(const void* x, size_t n, uint8_t* q, float* scale, uint32_t* ws,
+                                size_t ws_bytes, hipStream_t s)
+{
+    const size_t runs = (n + 256 * EPL - 1) / (256 * EPL);
+    const unsigned parts = (unsigned)std::min<size_t>(runs, kAmaxParts);
+    const unsigned blocks = (unsigned)std::min<size_t>(runs, 2048);
+    if (ws_bytes / 4 >= parts) {
+        hipLaunchKernelGGL((amax_kernel<IN, EPL, true>), dim3(parts), dim3(256), 0, s, x, n, ws);
+        hipLaunchKernelGGL((quant_tensor_kernel<IN, EPL>), dim3(blocks), dim3(256), 0, s, x, n, ws,
+                           (int)parts, q, scale);
+    } else {
+        hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, s, ws);
+        hipLaunchKernelGGL((amax_kernel<IN, EPL, false>), dim3(parts), dim3(256), 0, s, x, n, ws);
+        hipLaunchKernelGGL((quant_tensor_kernel<IN, EPL>), dim3(blocks), dim3(256), 0, s, x, n, ws,
+                           1, q, scale);
+    }
 }
 
 static ga_status check_in(int in_dtype)
@@ -637,17 +694,29 @@ ga_status ga_quant_fp8_128x128(const void* x, int in_dtype, int rows, int K, int
 ga_status ga_quant_fp8_per_tensor(const void* x, int in_dtype, size_t n, void* q, float* scale,
                                   void* amax_ws, void* stream)
 {
+    return ga_quant_fp8_per_tensor_ws(x, in_dtype, n, q, scale, amax_ws, 4, stream);
+}
+
+ga_status ga_quant_fp8_per_tensor_ws(const void* x, int in_dtype, size_t n, void* q, float* scale,
+                                     void* amax_ws, size_t ws_bytes, void* stream)
+{
     if (check_in(in_dtype) != GA_OK)
         return GA_ERR_ARG;
     if (!x || !q || !scale || !amax_ws || n == 0)
         return fail(GA_ERR_ARG, "quant_fp8_per_tensor: bad argument");
+    if (ws_bytes < 4)
+        return fail(GA_ERR_WORKSPACE, "quant_fp8_per_tensor: scratch holds %zu bytes, need 4",
+                    ws_bytes);
     hipStream_t s = (hipStream_t)stream;
-    const unsigned blocks = (unsigned)std::min<long long>(grid1d((long long)(n / 4) + 1, 256), 2048);
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, s, (uint32_t*)amax_ws);
-    GA_DISPATCH_IN(in_dtype, amax_kernel, dim3(blocks), dim3(256), 0, s, x, n,
-                   (uint32_t*)amax_ws);
-    GA_DISPATCH_IN(in_dtype, quant_tensor_kernel, dim3(blocks), dim3(256), 0, s, x, n,
-                   (const uint32_t*)amax_ws, (uint8_t*)q, scale);
+    if (in_dtype == GA_IN_F32)
+        launch_quant_tensor<GA_IN_F32, 4>(x, n, (uint8_t*)q, scale, (uint32_t*)amax_ws, ws_bytes,
+                                          s);
+    else if (((uintptr_t)x & 15) == 0 && ((uintptr_t)q & 7) == 0)
+        launch_quant_tensor<GA_IN_BF16, 8>(x, n, (uint8_t*)q, scale, (uint32_t*)amax_ws, ws_bytes,
+                                           s);
+    else
+        launch_quant_tensor<GA_IN_BF16, 4>(x, n, (uint8_t*)q, scale, (uint32_t*)amax_ws, ws_bytes,
+                                           s);
     GA_HIP_CHECK(hipGetLastError());
     return GA_OK;
 }

@@ -90,10 +90,10 @@ def quant_fp8_per_tensor(x, stream=None):
     x = x.contiguous()
     q = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
     scale = torch.empty((1,), dtype=torch.float32, device=x.device)
-    ws = torch.empty((1,), dtype=torch.int32, device=x.device)
-    check(lib().ga_quant_fp8_per_tensor(x.data_ptr(), _in_dtype(x), x.numel(), q.data_ptr(),
-                                        scale.data_ptr(), ws.data_ptr(),
-                                        _stream_handle(stream)))
+    ws = torch.empty((1024,), dtype=torch.int32, device=x.device)
+    check(lib().ga_quant_fp8_per_tensor_ws(x.data_ptr(), _in_dtype(x), x.numel(), q.data_ptr(),
+                                           scale.data_ptr(), ws.data_ptr(), 4096,
+                                           _stream_handle(stream)))
     return q, scale
 
 

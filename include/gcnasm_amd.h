@@ -309,6 +309,12 @@ ga_status ga_quant_fp8_128x128(const void* x, int in_dtype, int rows, int K, int
  * least 4 bytes. */
 ga_status ga_quant_fp8_per_tensor(const void* x, int in_dtype, size_t n, void* q,
                                   float* scale, void* amax_ws, void* stream);
+/* The same with the scratch's size: from 4096 bytes on (or 4 bytes per 1024
+ * fp32 / bf16 elements, whichever is less) the maximum is reduced through
+ * partial maxima there, without the clearing launch and the atomics that a
+ * scratch of one word takes. The scratch need not be cleared. Same bytes. */
+ga_status ga_quant_fp8_per_tensor_ws(const void* x, int in_dtype, size_t n, void* q,
+                                     float* scale, void* amax_ws, size_t ws_bytes, void* stream);
 
 /* ------------------------------------------------------------------------- */
 /* GEMM entry points.                                                         */

@@ -302,3 +302,37 @@ def test_e5m2_encoder_every_bf16_value(dev):
     np.testing.assert_array_equal(q.cpu().numpy(), oracle.quant_mx8(xf, 1, 0)[0])
     np.testing.assert_array_equal(q.cpu().numpy().reshape(-1, 32)[:nblk, 1:].reshape(-1)[:len(v)],
                                   oracle.e5m2_encode(v))
+
+
+@pytest.mark.parametrize("in_bf16", [False, True])
+@pytest.mark.parametrize("n", [1, 3, 7, 8, 2047, 2049, 262147, 9000011])
+def test_quant_per_tensor_scratch_sizes(dev, n, in_bf16):
+    """One word of scratch (atomics), partial maxima, and pointers that do not
+    allow 16-byte loads write the same bytes; the scratch starts dirty. The
+    maximum sits in the last element (the scalar tail where there is one)."""
+    import ctypes
+
+    from gcnasm_amd import _lib
+    x = oracle.randn(n + 1, 11)
+    x[n // 2] = np.float32("nan")
+    x[n - 1] = -37.5
+    if in_bf16:
+        xb = oracle.to_bf16_bits(x)
+        x = oracle.bf16_bits_to_f32(xb)
+        xt = torch.from_numpy(xb.view(np.int16)).to(dev).view(torch.bfloat16)
+    else:
+        xt = torch.from_numpy(x).to(dev)
+    for first in (0, 1):
+        src = xt[first:first + n]
+        want, scale = oracle.quant_fp8_per_tensor(x[first:first + n])
+        for words in (1, 1024):
+            q = torch.full((n,), 0xAA, dtype=torch.uint8, device=dev)
+            s = torch.zeros(1, dtype=torch.float32, device=dev)
+            ws = torch.full((words,), -1, dtype=torch.int32, device=dev)
+            _lib.check(_lib.lib().ga_quant_fp8_per_tensor_ws(
+                src.data_ptr(), 1 if in_bf16 else 0, n, q.data_ptr(), s.data_ptr(),
+                ws.data_ptr(), words * 4, ctypes.c_void_p(0)))
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32),
+                                          np.asarray(scale, np.float32).reshape(1).view(np.uint32))
+            np.testing.assert_array_equal(q.cpu().numpy(), want.reshape(-1))
