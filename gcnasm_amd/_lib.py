@@ -193,6 +193,7 @@ SIGNATURES = {
     "ga_quant_mxfp8": (_i, [_vp, _i, _i, _i, _i, _vp, _i, _vp, _i, _i, _vp]),
     "ga_quant_mx8": (_i, [_vp, _i, _i, _i, _i, _vp, _i, _vp, _i, _i, _i, _vp]),
     "ga_quant_mxfp4": (_i, [_vp, _i, _i, _i, _i, _vp, _i, _vp, _i, _i, _vp]),
+    "ga_prepare_mx_a": (_i, [_vp, _i, _i, _i, _i, _i, _vp, _vp, _i, _vp]),
     "ga_quant_fp8_1x128": (_i, [_vp, _i, _i, _i, _i, _vp, _i, _vp, _i, _vp]),
     "ga_quant_fp8_128x128": (_i, [_vp, _i, _i, _i, _i, _vp, _i, _vp, _i, _vp]),
     "ga_quant_fp8_per_tensor": (_i, [_vp, _i, _sz, _vp, _vp, _vp, _vp]),

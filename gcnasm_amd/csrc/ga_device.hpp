@@ -210,19 +210,21 @@ __device__ __forceinline__ uint32_t e4m3_encode(float x)
 
 // Four E4M3 codes packed little-endian, same results as e4m3_encode: the
 // hardware converter (v_cvt_pk_fp8_f32: OCP E4M3, round to nearest even) on
-// inputs clamped to +-448 (saturation), NaN inputs replaced by 0x7F after.
+// inputs clamped to +-448 (saturation), NaN inputs replaced by 0x7F after
+// (NAN_RULE false: the caller knows that there are none).
+template <bool NAN_RULE = true>
 __device__ __forceinline__ uint32_t e4m3_encode4(float a, float b, float c, float d)
 {
     const float x[4] = {a, b, c, d};
     float y[4];
 #pragma unroll
     for (int j = 0; j < 4; j++)
-        y[j] = __builtin_fminf(__builtin_fmaxf(x[j], -448.0f), 448.0f);
+        y[j] = __builtin_amdgcn_fmed3f(x[j], -448.0f, 448.0f);
     const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false);
     uint32_t r = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], lo, true);
 #pragma unroll
     for (int j = 0; j < 4; j++)
-        if (x[j] != x[j])
+        if (NAN_RULE && x[j] != x[j])
             r = (r & ~(0xFFu << (8 * j))) | (0x7Fu << (8 * j));
     return r;
 }
@@ -230,106 +232,39 @@ __device__ __forceinline__ uint32_t e4m3_encode4(float a, float b, float c, floa
 // Four E5M2 (bf8) codes as one dword, same results as the oracle's E5M2
 // encode: the hardware converter on inputs clamped to +-57344 (saturation;
 // the converter alone would round past the maximum to inf), NaN -> 0x7F.
+template <bool NAN_RULE = true>
 __device__ __forceinline__ uint32_t e5m2_encode4(float a, float b, float c, float d)
 {
     const float x[4] = {a, b, c, d};
     float y[4];
 #pragma unroll
     for (int j = 0; j < 4; j++)
-        y[j] = __builtin_fminf(__builtin_fmaxf(x[j], -57344.0f), 57344.0f);
+        y[j] = __builtin_amdgcn_fmed3f(x[j], -57344.0f, 57344.0f);
     const int lo = __builtin_amdgcn_cvt_pk_bf8_f32(y[0], y[1], 0, false);
     uint32_t r = (uint32_t)__builtin_amdgcn_cvt_pk_bf8_f32(y[2], y[3], lo, true);
 #pragma unroll
     for (int j = 0; j < 4; j++)
-        if (x[j] != x[j])
+        if (NAN_RULE && x[j] != x[j])
             r = (r & ~(0xFFu << (8 * j))) | (0x7Fu << (8 * j));
     return r;
 }
 
-// Four e2m1 codes as 16 bits (element j in bits 4j..4j+3), same results as
-// e2m1_encode: the hardware converter (v_cvt_scalef32_pk_fp4_f32, scale 1)
-// on inputs clamped to +-6, NaN inputs replaced by a zero of their sign.
+// Four OCP e2m1 codes as 16 bits (element j in bits 4j..4j+3; values 0, .5, 1,
+// 1.5, 2, 3, 4, 6, sign in bit 3): round to nearest, ties to the even code,
+// saturate to +-6. The hardware converter (v_cvt_scalef32_pk_fp4_f32, scale 1)
+// on inputs clamped to +-6, NaN inputs replaced by a zero of their sign (e2m1 has no NaN).
+template <bool NAN_RULE = true>
 __device__ __forceinline__ uint32_t e2m1_encode4(float a, float b, float c, float d)
 {
     const float x[4] = {a, b, c, d};
     float y[4];
 #pragma unroll
     for (int j = 0; j < 4; j++)
-        y[j] = x[j] != x[j] ? __builtin_copysignf(0.0f, x[j])
-                            : __builtin_fminf(__builtin_fmaxf(x[j], -6.0f), 6.0f);
+        y[j] = NAN_RULE && x[j] != x[j] ? __builtin_copysignf(0.0f, x[j])
+                                        : __builtin_amdgcn_fmed3f(x[j], -6.0f, 6.0f);
     uint32_t r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, y[0], y[1], 1.0f, 0);
     r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, y[2], y[3], 1.0f, 1);
     return r & 0xFFFFu;
-}
-
-// Exact floor(log2 a) and 23 fraction bits for a finite a > 0.
-__device__ __forceinline__ void log2_parts(float a, int& E, uint32_t& frac)
-{
-    uint32_t u = __float_as_uint(a) & 0x7FFFFFFFu;
-    int ef = (int)(u >> 23);
-    if (ef > 0) {
-        E = ef - 127;
-        frac = u & 0x7FFFFFu;
-    } else {
-        uint32_t mant = u & 0x7FFFFFu;
-        int msb = 31 - __clz(mant);
-        E = msb - 149;
-        frac = (mant << (23 - msb)) & 0x7FFFFFu;
-    }
-}
-
-// E8M0 exponent of an MX block whose element format has largest value
-// (1 + FRAC/2^23) * 2^EMAX: rule 0: floor(log2(amax/max)), 1: ceil, 2: OCP
-// floor(log2 amax) - EMAX. Zero block -> -127.
-template <uint32_t FRAC, int EMAX>
-__device__ __forceinline__ int mx_scale_exp_t(float amax, int rule)
-{
-    if (!(amax > 0.0f))
-        return -127;
-    if (__float_as_uint(amax) == 0x7F800000u)
-        return 127;
-    int E;
-    uint32_t f;
-    log2_parts(amax, E, f);
-    int e;
-    if (rule == 0)
-        e = (f >= FRAC) ? E - EMAX : E - EMAX - 1;
-    else if (rule == 1)
-        e = (f <= FRAC) ? E - EMAX : E - EMAX + 1;
-    else
-        e = E - EMAX;
-    return e < -127 ? -127 : (e > 127 ? 127 : e);
-}
-
-// E4M3: 448 = 1.75 * 2^8.
-__device__ __forceinline__ int mx_scale_exp(float amax, int rule)
-{
-    return mx_scale_exp_t<0x600000u, 8>(amax, rule);
-}
-
-// E5M2: 57344 = 1.75 * 2^15.
-__device__ __forceinline__ int mx5_scale_exp(float amax, int rule)
-{
-    return mx_scale_exp_t<0x600000u, 15>(amax, rule);
-}
-
-// E2M1: 6 = 1.5 * 2^2.
-__device__ __forceinline__ int mx4_scale_exp(float amax, int rule)
-{
-    return mx_scale_exp_t<0x400000u, 2>(amax, rule);
-}
-
-// OCP E2M1 encode (MXFP4 element; values 0, .5, 1, 1.5, 2, 3, 4, 6, sign in
-// bit 3): round to nearest, ties to the even code, saturate to +-6. E2M1 has
-// no NaN: NaN gives a zero with its sign bit.
-__device__ __forceinline__ uint32_t e2m1_encode(float x)
-{
-    const uint32_t u = __float_as_uint(x);
-    const float a = __uint_as_float(u & 0x7FFFFFFFu);
-    const uint32_t c = (uint32_t)(a > 0.25f) + (uint32_t)(a >= 0.75f) + (uint32_t)(a > 1.25f) +
-                       (uint32_t)(a >= 1.75f) + (uint32_t)(a > 2.5f) + (uint32_t)(a >= 3.5f) +
-                       (uint32_t)(a > 5.0f);
-    return ((u >> 28) & 8u) | c;
 }
 
 // Linear tile id -> (tile_m, tile_n) on a gdx x gdy tile grid. Workgroup ids

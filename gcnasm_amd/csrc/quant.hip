@@ -7,8 +7,9 @@
 //                     written transposed [K/128, rows] (opus SFA layout)
 //   * DeepSeek 128x128: fp32 s per 128x128 tile [ceil(rows/128), K/128]
 //   * per-tensor:     one fp32 s = amax/448
-// Encoding is the exact integer RNE/saturating E4M3 encode of ga_device.hpp;
-// x/s uses IEEE fp32 division (correctly rounded; built without fast-math).
+// Encoding is the hardware converters behind a clamp to the format's maximum
+// (ga_device.hpp), bit-exact with round to nearest even and saturation; x/s is
+// the correctly rounded fp32 quotient wherever it decides a code.
 // All kernels are HBM streaming kernels: 16-byte loads per lane (8-byte for
 // bf16 rows whose stride does not allow 16), several independent loads in
 // flight per lane, cross-lane amax over DPP row exchanges, coalesced stores.
@@ -17,42 +18,49 @@
 
 namespace ga {
 
-__device__ __forceinline__ uint32_t pack4(uint32_t a, uint32_t b, uint32_t c, uint32_t d)
-{
-    return a | (b << 8) | (c << 16) | (d << 24);
-}
-
-// Up to 8 elements per lane from one 16-byte (f32: 4) or 8/16-byte (bf16: 4/8)
-// load; lanes that are out of range read zeros.
+// EPL elements of a lane as they lie in memory: one 16-byte load (f32: 4,
+// bf16: 8 elements) or one 8-byte load (bf16: 4). A kernel issues all its
+// loads first, those of out-of-range lanes from element 0, and unpack() turns
+// those into zeros: a load under a branch is waited for inside it, so several
+// such loads of a lane ran one after the other (measured on MI355X together
+// with the encoders' NaN rule out of the common path, prepare_mx_a_kernel:
+// 8192x8192 bf16 MXFP8 43.7 -> 32.9 us, 2048x8192 MXFP4 14.3 -> 9.2).
 template <int IN, int EPL>
-__device__ __forceinline__ void load_elems(const void* x, size_t idx, bool ok, float (&v)[EPL])
-{
+struct Raw {
+    static_assert(IN == GA_IN_BF16 || EPL == 4, "f32: 4 elements per 16-byte load");
+    static constexpr int kDwords = IN == GA_IN_F32 ? 4 : EPL / 2;
+    uint32_t w[kDwords];
+
+    __device__ __forceinline__ void load(const void* x, size_t idx, bool ok)
+    {
+        const size_t i = ok ? idx : 0;
+        if constexpr (kDwords == 4) {
+            const v4i t = IN == GA_IN_F32 ? *(const v4i*)((const float*)x + i)
+                                          : *(const v4i*)((const uint16_t*)x + i);
 #pragma unroll
-    for (int j = 0; j < EPL; j++)
-        v[j] = 0.0f;
-    if (!ok)
-        return;
-    if constexpr (IN == GA_IN_F32) {
-        static_assert(EPL == 4, "f32: 4 elements per 16-byte load");
-        const v4f t = *(const v4f*)((const float*)x + idx);
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            v[j] = t[j];
-    } else if constexpr (EPL == 8) {
-        const v4i t = *(const v4i*)((const uint16_t*)x + idx);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            v[2 * j] = bf16_to_f32((uint16_t)((uint32_t)t[j] & 0xFFFF));
-            v[2 * j + 1] = bf16_to_f32((uint16_t)((uint32_t)t[j] >> 16));
+            for (int j = 0; j < 4; j++)
+                w[j] = (uint32_t)t[j];
+        } else {
+            const uint2 t = *(const uint2*)((const uint16_t*)x + i);
+            w[0] = t.x;
+            w[1] = t.y;
         }
-    } else {
-        const uint2 t = *(const uint2*)((const uint16_t*)x + idx);
-        v[0] = bf16_to_f32((uint16_t)(t.x & 0xFFFF));
-        v[1] = bf16_to_f32((uint16_t)(t.x >> 16));
-        v[2] = bf16_to_f32((uint16_t)(t.y & 0xFFFF));
-        v[3] = bf16_to_f32((uint16_t)(t.y >> 16));
     }
-}
+
+    __device__ __forceinline__ void unpack(bool ok, float (&v)[EPL]) const
+    {
+#pragma unroll
+        for (int j = 0; j < kDwords; j++) {
+            const uint32_t u = ok ? w[j] : 0u;
+            if constexpr (IN == GA_IN_F32) {
+                v[j] = __uint_as_float(u);
+            } else {
+                v[2 * j] = __uint_as_float(u << 16);
+                v[2 * j + 1] = __uint_as_float(u & 0xFFFF0000u);
+            }
+        }
+    }
+};
 
 // Block maxima of |x| are taken on the bit patterns: for x >= 0 the IEEE bit
 // order is the value order, and every NaN (quiet or signalling) maps to 0, so
@@ -114,21 +122,94 @@ __device__ __forceinline__ uint32_t amax_raw(const float (&v)[EPL])
 // recomputation is taken by the whole wave when any of its blocks holds a
 // NaN (a ballot makes the branch uniform), so the lane exchanges always run
 // with every lane active.
+// nan says so (the same in every lane): the encoders' NaN rule is then needed.
 template <int W, int EPL>
-__device__ __forceinline__ uint32_t block_amax(const float (&v)[EPL])
+__device__ __forceinline__ uint32_t block_amax(const float (&v)[EPL], bool& nan)
 {
     uint32_t a = group_max_dpp<W>(amax_raw<EPL>(v));
-    if (__builtin_amdgcn_ballot_w64(a > 0x7F800000u) != 0)
+    nan = __builtin_amdgcn_ballot_w64(a > 0x7F800000u) != 0;
+    if (nan)
         a = group_max_dpp<W>(amax_n<EPL>(v));
     return a;
+}
+
+// E8M0 exponent of an MX block whose element format (elem 0 E4M3, 1 E5M2, 2
+// e2m1) has the largest value max = (1 + frac / 2^23) * 2^emax, from the bit
+// pattern u of the block's maximum (no NaN). Rule 0: floor(log2(amax / max)),
+// 1: ceil, 2: floor(log2 amax) - emax; within -127 .. 127, a zero block -127,
+// an infinite one 127. Adding `add` carries into the exponent field where the
+// rule rounds up; a zero or subnormal maximum comes out below -127 under every
+// rule, so it needs no branch of its own.
+struct MxScaleRule {
+    uint32_t add;
+    int sub;
+    __device__ __forceinline__ MxScaleRule(int elem, int rule)
+    {
+        const uint32_t frac = elem == 2 ? 0x400000u : 0x600000u; // 6 = 1.5 * 2^2, else 1.75 * 2^n
+        const int emax = elem == 2 ? 2 : (elem == 1 ? 15 : 8);
+        add = rule == 0 ? 0x800000u - frac : (rule == 1 ? 0x7FFFFFu - frac : 0u);
+        sub = 127 + emax + (rule == 0 ? 1 : 0);
+    }
+    __device__ __forceinline__ int exp(uint32_t u) const
+    {
+        const int e = (int)((u + add) >> 23) - sub;
+        return u == 0x7F800000u ? 127 : max(e, -127);
+    }
+};
+
+// EPL scaled elements of an MX block as codes (ELEM 0 E4M3, 1 E5M2: EPL bytes;
+// 2 e2m1: EPL / 2 bytes) at dst.
+template <int ELEM, bool NAN_RULE, int EPL>
+__device__ __forceinline__ void mx_store_codes(const float (&v)[EPL], int e, uint8_t* dst)
+{
+    float t[EPL];
+#pragma unroll
+    for (int j = 0; j < EPL; j++)
+        t[j] = ldexpf(v[j], -e);
+    if constexpr (ELEM == 2) {
+        uint32_t w = e2m1_encode4<NAN_RULE>(t[0], t[1], t[2], t[3]);
+        if constexpr (EPL == 8) {
+            w |= e2m1_encode4<NAN_RULE>(t[4], t[5], t[6], t[7]) << 16;
+            *(uint32_t*)dst = w;
+        } else {
+            *(uint16_t*)dst = (uint16_t)w;
+        }
+    } else {
+        uint32_t w[EPL / 4];
+#pragma unroll
+        for (int j = 0; j < EPL / 4; j++)
+            w[j] = ELEM == 1
+                       ? e5m2_encode4<NAN_RULE>(t[4 * j], t[4 * j + 1], t[4 * j + 2], t[4 * j + 3])
+                       : e4m3_encode4<NAN_RULE>(t[4 * j], t[4 * j + 1], t[4 * j + 2], t[4 * j + 3]);
+        if constexpr (EPL == 8)
+            *(uint2*)dst = make_uint2(w[0], w[1]);
+        else
+            *(uint32_t*)dst = w[0];
+    }
+}
+
+// EPL elements divided by their scale as E4M3 bytes at dst.
+template <bool NAN_RULE, int EPL, class D>
+__device__ __forceinline__ void fp8_store_codes(const D& d, const float (&v)[EPL], uint8_t* dst)
+{
+    float t[EPL];
+    d.div(v, t);
+    uint32_t w[EPL / 4];
+#pragma unroll
+    for (int j = 0; j < EPL / 4; j++)
+        w[j] = e4m3_encode4<NAN_RULE>(t[4 * j], t[4 * j + 1], t[4 * j + 2], t[4 * j + 3]);
+    if constexpr (EPL == 8)
+        *(uint2*)dst = make_uint2(w[0], w[1]);
+    else
+        *(uint32_t*)dst = w[0];
 }
 
 // ---- MX 1x32 (E4M3 or packed e2m1 codes) -------------------------------------
 // A 1x32 block is LPB = 32/EPL lanes of EPL elements (16-byte loads where the
 // layout allows); each lane handles U blocks, BPP = 256/LPB blocks apart, so U
 // independent loads are in flight per lane before the first reduction.
-// E5: E5M2 elements instead of E4M3 (FP4 false).
-template <int IN, int EPL, bool FP4, int U, bool E5 = false>
+// ELEM: 0 E4M3, 1 E5M2, 2 e2m1.
+template <int IN, int EPL, int ELEM, int U>
 __global__ __launch_bounds__(256) void quant_mx_kernel(const void* __restrict__ x, int rows,
                                                        int K, int ld_x, uint8_t* __restrict__ q,
                                                        int ld_q, uint8_t* __restrict__ s,
@@ -139,7 +220,8 @@ __global__ __launch_bounds__(256) void quant_mx_kernel(const void* __restrict__ 
     const long long total = (long long)rows * nb;
     const int sub = threadIdx.x % LPB;
     const long long base = (long long)blockIdx.x * (BPP * U) + threadIdx.x / LPB;
-    float v[U][EPL];
+    const MxScaleRule scale(ELEM, rule);
+    Raw<IN, EPL> raw[U];
     int rr[U], bb[U];
     bool ok[U];
 #pragma unroll
@@ -148,48 +230,90 @@ __global__ __launch_bounds__(256) void quant_mx_kernel(const void* __restrict__ 
         ok[u] = blk < total;
         rr[u] = ok[u] ? (int)(blk / nb) : 0;
         bb[u] = ok[u] ? (int)(blk - (long long)rr[u] * nb) : 0;
-        load_elems<IN, EPL>(x, (size_t)rr[u] * ld_x + bb[u] * 32 + sub * EPL, ok[u], v[u]);
+        raw[u].load(x, (size_t)rr[u] * ld_x + bb[u] * 32 + sub * EPL, ok[u]);
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
-        const float amax = __uint_as_float(block_amax<LPB, EPL>(v[u]));
+        float v[EPL];
+        raw[u].unpack(ok[u], v);
+        bool nan;
+        const int e = scale.exp(block_amax<LPB, EPL>(v, nan));
         if (!ok[u])
             continue;
-        const int e = FP4 ? mx4_scale_exp(amax, rule)
-                          : (E5 ? mx5_scale_exp(amax, rule) : mx_scale_exp(amax, rule));
-        uint8_t* qrow = q + (size_t)rr[u] * ld_q;
-        if constexpr (FP4) {
-            float t[EPL];
-#pragma unroll
-            for (int j = 0; j < EPL; j++)
-                t[j] = ldexpf(v[u][j], -e);
-            uint32_t w = e2m1_encode4(t[0], t[1], t[2], t[3]);
-            if constexpr (EPL == 8)
-                w |= e2m1_encode4(t[4], t[5], t[6], t[7]) << 16;
-            if constexpr (EPL == 8)
-                *(uint32_t*)(qrow + bb[u] * 16 + sub * 4) = w;
-            else
-                *(uint16_t*)(qrow + bb[u] * 16 + sub * 2) = (uint16_t)w;
-        } else {
-            float t[EPL];
-#pragma unroll
-            for (int j = 0; j < EPL; j++)
-                t[j] = ldexpf(v[u][j], -e);
-            auto enc4 = [](float p, float q_, float r, float w) {
-                return E5 ? e5m2_encode4(p, q_, r, w) : e4m3_encode4(p, q_, r, w);
-            };
-            if constexpr (EPL == 8) {
-                uint2 w;
-                w.x = enc4(t[0], t[1], t[2], t[3]);
-                w.y = enc4(t[4], t[5], t[6], t[7]);
-                *(uint2*)(qrow + bb[u] * 32 + sub * 8) = w;
-            } else {
-                *(uint32_t*)(qrow + bb[u] * 32 + sub * 4) = enc4(t[0], t[1], t[2], t[3]);
-            }
-        }
+        const int k = bb[u] * 32 + sub * EPL;
+        uint8_t* dst = q + (size_t)rr[u] * ld_q + (ELEM == 2 ? k / 2 : k);
+        if (nan)
+            mx_store_codes<ELEM, true>(v, e, dst);
+        else
+            mx_store_codes<ELEM, false>(v, e, dst);
         if (sub == 0)
             s[(size_t)rr[u] * ld_s + bb[u]] = (uint8_t)(e + 127);
     }
+}
+
+// ---- MX activations in the GEMM's layout -------------------------------------------
+// Quantise, pad the rows to a multiple of 256 (codes 0, scales 0x7F) and
+// shuffle the scales in one pass. One workgroup per 32 rows x 256 K, the
+// elements under one 256-byte block of the shuffled scales (the layout of
+// shuffle_scale_kernel): it reads up to 16 KB of bf16 in four 16-byte loads per
+// lane, whole 512-byte row pieces each, and collects the block's scales in
+// LDS. Bound by bytes (x read once, codes written once) and below about 1 MB
+// by the launch; as separate passes (quantiser, fill, copy, scale shuffle) it
+// took four launches and moved the codes three times. Measured on MI355X,
+// 8192x8192 bf16: 32.9 us (6.1 TB/s); a whole call with its GEMM, before ->
+// after: 256x256x512 MXFP8 45.5 -> 25.4 us (launches),
+// 16x28672x8192 47.0 -> 42.1, 64x8192x28672 64.3 -> 60.0, 1000x8192x8192 96.3 ->
+// 85.7, 2048x8192x8192 MXFP4 86.3 -> 74.6.
+// EPL = 4: fp32, or bf16 rows that do not allow 16-byte loads.
+// ELEM: 0 E4M3, 1 E5M2, 2 e2m1.
+template <int IN, int EPL, int ELEM>
+__global__ __launch_bounds__(256) void prepare_mx_a_kernel(const void* __restrict__ x, int M,
+                                                           int K, int ld_x,
+                                                           uint8_t* __restrict__ q,
+                                                           uint8_t* __restrict__ s, int sn,
+                                                           int rule)
+{
+    constexpr int LPB = 32 / EPL;  // lanes per 1x32 block
+    constexpr int LPR = 8 * LPB;   // lanes per row of 256 K
+    constexpr int RPP = 256 / LPR; // rows per pass
+    constexpr int NP = 32 / RPP;   // passes
+    __shared__ __attribute__((aligned(4))) uint8_t sblk[256];
+    const int tid = threadIdx.x, sub = tid % LPB, bc = (tid % LPR) / LPB;
+    const int n3 = sn / 8, d0 = blockIdx.x / n3, d3 = blockIdx.x - d0 * n3;
+    const int k = d3 * 256 + (tid % LPR) * EPL;
+    const int r_lo = tid / LPR; // row inside the block of pass 0
+    const bool in_k = k < K;    // K % 32 == 0: whole blocks
+    const size_t ld_q = ELEM == 2 ? (size_t)K / 2 : (size_t)K;
+    const MxScaleRule scale(ELEM, rule);
+    Raw<IN, EPL> raw[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        const int r = d0 * 32 + i * RPP + r_lo;
+        raw[i].load(x, (size_t)r * ld_x + k, in_k && r < M);
+    }
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        const int rl = i * RPP + r_lo, r = d0 * 32 + rl;
+        const bool real = in_k && r < M;
+        float v[EPL];
+        raw[i].unpack(real, v); // a pad row: zeros, code 0
+        bool nan;
+        const int e = scale.exp(block_amax<LPB, EPL>(v, nan));
+        if (in_k) {
+            uint8_t* dst = q + (size_t)r * ld_q + (ELEM == 2 ? k / 2 : k);
+            if (nan)
+                mx_store_codes<ELEM, true>(v, e, dst);
+            else
+                mx_store_codes<ELEM, false>(v, e, dst);
+        }
+        // byte (d5, d2, d4, d1) of the block: column 4 * d4 + d5, row 16 * d1 + d2
+        if (sub == 0)
+            sblk[(((bc & 3) * 16 + (rl & 15)) * 2 + (bc >> 2)) * 2 + (rl >> 4)] =
+                real ? (uint8_t)(e + 127) : (uint8_t)0x7F;
+    }
+    __syncthreads();
+    if (tid < 64)
+        ((uint32_t*)(s + (size_t)blockIdx.x * 256))[tid] = ((const uint32_t*)sblk)[tid];
 }
 
 // ---- DeepSeek 1x128 -----------------------------------------------------------
@@ -247,7 +371,7 @@ __global__ __launch_bounds__(256) void quant_1x128_kernel(const void* __restrict
     const long long total = (long long)rows * ng;
     const int sub = threadIdx.x % LPB;
     const long long base = (long long)blockIdx.x * (BPP * U) + threadIdx.x / LPB;
-    float v[U][EPL];
+    Raw<IN, EPL> raw[U];
     int rr[U], gg[U];
     bool ok[U];
 #pragma unroll
@@ -256,25 +380,23 @@ __global__ __launch_bounds__(256) void quant_1x128_kernel(const void* __restrict
         ok[u] = blk < total;
         rr[u] = ok[u] ? (int)(blk / ng) : 0;
         gg[u] = ok[u] ? (int)(blk - (long long)rr[u] * ng) : 0;
-        load_elems<IN, EPL>(x, (size_t)rr[u] * ld_x + gg[u] * 128 + sub * EPL, ok[u], v[u]);
+        raw[u].load(x, (size_t)rr[u] * ld_x + gg[u] * 128 + sub * EPL, ok[u]);
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
-        const float amax = __uint_as_float(block_amax<LPB, EPL>(v[u]));
+        float v[EPL];
+        raw[u].unpack(ok[u], v);
+        bool nan;
+        const float amax = __uint_as_float(block_amax<LPB, EPL>(v, nan));
         if (!ok[u])
             continue;
         const float sc = ds_scale(amax);
-        float t[EPL];
-        ScaleDiv(sc).div(v[u], t);
+        const ScaleDiv d(sc);
         uint8_t* dst = q + (size_t)rr[u] * ld_q + gg[u] * 128 + sub * EPL;
-        if constexpr (EPL == 8) {
-            uint2 w;
-            w.x = e4m3_encode4(t[0], t[1], t[2], t[3]);
-            w.y = e4m3_encode4(t[4], t[5], t[6], t[7]);
-            *(uint2*)dst = w;
-        } else {
-            *(uint32_t*)dst = e4m3_encode4(t[0], t[1], t[2], t[3]);
-        }
+        if (nan)
+            fp8_store_codes<true>(d, v, dst);
+        else
+            fp8_store_codes<false>(d, v, dst);
         if (sub == 0)
             sfa[(size_t)gg[u] * ld_s + rr[u]] = sc;
     }
@@ -299,13 +421,17 @@ __global__ __launch_bounds__(kTileThreads) void quant_128x128_kernel(
     const int g = blockIdx.x, rb = blockIdx.y;
     const int tid = threadIdx.x;
     const int col = (tid % LPR) * EPL, r_lo = tid / LPR;
+    Raw<IN, EPL> raw[NP];
     float v[NP][EPL];
     uint32_t amax = 0u;
 #pragma unroll
     for (int i = 0; i < NP; i++) {
         const int r = rb * 128 + r_lo + i * RPP;
-        load_elems<IN, EPL>(x, (size_t)r * ld_x + g * 128 + col, r < rows, v[i]);
+        raw[i].load(x, (size_t)r * ld_x + g * 128 + col, r < rows);
     }
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        raw[i].unpack(rb * 128 + r_lo + i * RPP < rows, v[i]);
     // the tile's maximum over the plain keys; only a tile holding a NaN
     // (the maximum says so, the same in every wave) takes the NaN-ignoring one
     auto tile_max = [&](bool nan_free) {
@@ -325,7 +451,8 @@ __global__ __launch_bounds__(kTileThreads) void quant_128x128_kernel(
         return m;
     };
     amax = tile_max(false);
-    if (amax > 0x7F800000u) {
+    const bool nan = amax > 0x7F800000u;
+    if (nan) {
         __syncthreads(); // every wave has read wmax before it is written again
         amax = tile_max(true);
     }
@@ -336,17 +463,11 @@ __global__ __launch_bounds__(kTileThreads) void quant_128x128_kernel(
         const int r = rb * 128 + r_lo + i * RPP;
         if (r >= rows)
             continue;
-        float t[EPL];
-        d.div(v[i], t);
         uint8_t* dst = q + (size_t)r * ld_q + g * 128 + col;
-        if constexpr (EPL == 8) {
-            uint2 w;
-            w.x = e4m3_encode4(t[0], t[1], t[2], t[3]);
-            w.y = e4m3_encode4(t[4], t[5], t[6], t[7]);
-            *(uint2*)dst = w;
-        } else {
-            *(uint32_t*)dst = e4m3_encode4(t[0], t[1], t[2], t[3]);
-        }
+        if (nan)
+            fp8_store_codes<true>(d, v[i], dst);
+        else
+            fp8_store_codes<false>(d, v[i], dst);
     }
     if (tid == 0)
         sfb[(size_t)rb * ld_s + g] = sc;
@@ -395,15 +516,16 @@ __global__ __launch_bounds__(256) void amax_kernel(const void* __restrict__ x, s
     const size_t nv = n / EPL;
     const size_t stride = (size_t)gridDim.x * 256;
     for (size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x; i0 < nv; i0 += stride * kTensorU) {
-        float v[kTensorU][EPL];
-#pragma unroll
-        for (int u = 0; u < kTensorU; u++) {
-            const size_t i = i0 + u * stride;
-            load_elems<IN, EPL>(x, i * EPL, i < nv, v[u]);
-        }
+        Raw<IN, EPL> raw[kTensorU];
 #pragma unroll
         for (int u = 0; u < kTensorU; u++)
-            a = max(a, amax_n<EPL>(v[u]));
+            raw[u].load(x, (i0 + u * stride) * EPL, i0 + u * stride < nv);
+#pragma unroll
+        for (int u = 0; u < kTensorU; u++) {
+            float v[EPL];
+            raw[u].unpack(i0 + u * stride < nv, v);
+            a = max(a, amax_n<EPL>(v));
+        }
     }
     if (blockIdx.x == 0 && threadIdx.x < n % EPL)
         a = max(a, abs_key(load_one<IN>(x, nv * EPL + threadIdx.x)));
@@ -437,27 +559,17 @@ __global__ __launch_bounds__(256) void quant_tensor_kernel(const void* __restric
     const size_t nv = n / EPL;
     const size_t stride = (size_t)gridDim.x * 256;
     for (size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x; i0 < nv; i0 += stride * kTensorU) {
-        float v[kTensorU][EPL];
+        Raw<IN, EPL> raw[kTensorU];
+#pragma unroll
+        for (int u = 0; u < kTensorU; u++)
+            raw[u].load(x, (i0 + u * stride) * EPL, i0 + u * stride < nv);
 #pragma unroll
         for (int u = 0; u < kTensorU; u++) {
             const size_t i = i0 + u * stride;
-            load_elems<IN, EPL>(x, i * EPL, i < nv, v[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < kTensorU; u++) {
-            const size_t i = i0 + u * stride;
-            if (i < nv) {
-                float t[EPL];
-                d.div(v[u], t);
-                if constexpr (EPL == 8) {
-                    uint2 w;
-                    w.x = e4m3_encode4(t[0], t[1], t[2], t[3]);
-                    w.y = e4m3_encode4(t[4], t[5], t[6], t[7]);
-                    *(uint2*)(q + i * 8) = w;
-                } else {
-                    *(uint32_t*)(q + i * 4) = e4m3_encode4(t[0], t[1], t[2], t[3]);
-                }
-            }
+            float v[EPL];
+            raw[u].unpack(i < nv, v);
+            if (i < nv)
+                fp8_store_codes<true>(d, v, q + i * EPL);
         }
     }
     if (blockIdx.x == 0 && threadIdx.x < n % EPL) {
@@ -545,7 +657,7 @@ static bool bf16_wide(int in_dtype, const void* x, int ld_x, const void* q, int 
            ld_q % store_align == 0 && ((uintptr_t)q % store_align) == 0;
 }
 
-template <bool FP4, bool E5 = false>
+template <int ELEM>
 static void launch_quant_mx(int in_dtype, bool wide, long long blocks, hipStream_t st,
                             const void* x, int rows, int K, int ld_x, uint8_t* q, int ld_q,
                             uint8_t* s, int ld_s, int rule)
@@ -554,13 +666,13 @@ static void launch_quant_mx(int in_dtype, bool wide, long long blocks, hipStream
     const int u = (in_dtype != GA_IN_F32 && wide) ? kQUWide : kQU;
     const unsigned grid = grid1d(blocks, (256 / (32 / epl)) * u);
     if (in_dtype == GA_IN_F32)
-        hipLaunchKernelGGL((quant_mx_kernel<GA_IN_F32, 4, FP4, kQU, E5>), dim3(grid), dim3(256), 0,
+        hipLaunchKernelGGL((quant_mx_kernel<GA_IN_F32, 4, ELEM, kQU>), dim3(grid), dim3(256), 0,
                            st, x, rows, K, ld_x, q, ld_q, s, ld_s, rule);
     else if (wide)
-        hipLaunchKernelGGL((quant_mx_kernel<GA_IN_BF16, 8, FP4, kQUWide, E5>), dim3(grid),
+        hipLaunchKernelGGL((quant_mx_kernel<GA_IN_BF16, 8, ELEM, kQUWide>), dim3(grid),
                            dim3(256), 0, st, x, rows, K, ld_x, q, ld_q, s, ld_s, rule);
     else
-        hipLaunchKernelGGL((quant_mx_kernel<GA_IN_BF16, 4, FP4, kQU, E5>), dim3(grid), dim3(256),
+        hipLaunchKernelGGL((quant_mx_kernel<GA_IN_BF16, 4, ELEM, kQU>), dim3(grid), dim3(256),
                            0, st, x, rows, K, ld_x, q, ld_q, s, ld_s, rule);
 }
 
@@ -587,6 +699,21 @@ static void launch_quant_tensor(const void* x, size_t n, uint8_t* q, float* scal
     }
 }
 
+template <int ELEM>
+static void launch_prepare_mx_a(int in_dtype, bool wide, dim3 grid, hipStream_t st, const void* x,
+                                int M, int K, int ld_x, uint8_t* q, uint8_t* s, int sn, int rule)
+{
+    if (in_dtype == GA_IN_F32)
+        hipLaunchKernelGGL((prepare_mx_a_kernel<GA_IN_F32, 4, ELEM>), grid, dim3(256), 0, st, x, M,
+                           K, ld_x, q, s, sn, rule);
+    else if (wide)
+        hipLaunchKernelGGL((prepare_mx_a_kernel<GA_IN_BF16, 8, ELEM>), grid, dim3(256), 0, st, x,
+                           M, K, ld_x, q, s, sn, rule);
+    else
+        hipLaunchKernelGGL((prepare_mx_a_kernel<GA_IN_BF16, 4, ELEM>), grid, dim3(256), 0, st, x,
+                           M, K, ld_x, q, s, sn, rule);
+}
+
 static ga_status check_in(int in_dtype)
 {
     if (in_dtype != GA_IN_F32 && in_dtype != GA_IN_BF16)
@@ -609,10 +736,10 @@ ga_status ga_quant_mx8(const void* x, int in_dtype, int rows, int K, int ld_x, v
     long long blocks = (long long)rows * (K / 32);
     const bool wide = bf16_wide(in_dtype, x, ld_x, q, ld_q, 8);
     if (fmt == 1)
-        launch_quant_mx<false, true>(in_dtype, wide, blocks, (hipStream_t)stream, x, rows, K,
+        launch_quant_mx<1>(in_dtype, wide, blocks, (hipStream_t)stream, x, rows, K,
                                      ld_x, (uint8_t*)q, ld_q, (uint8_t*)scales, ld_s, scale_rule);
     else
-        launch_quant_mx<false>(in_dtype, wide, blocks, (hipStream_t)stream, x, rows, K, ld_x,
+        launch_quant_mx<0>(in_dtype, wide, blocks, (hipStream_t)stream, x, rows, K, ld_x,
                                (uint8_t*)q, ld_q, (uint8_t*)scales, ld_s, scale_rule);
     GA_HIP_CHECK(hipGetLastError());
     return GA_OK;
@@ -635,9 +762,35 @@ ga_status ga_quant_mxfp4(const void* x, int in_dtype, int rows, int K, int ld_x,
     if (K % 32 || ld_x % 4 || ld_q % 2)
         return fail(GA_ERR_SHAPE, "quant_mxfp4: K %% 32, ld_x %% 4 and ld_q %% 2 must be 0");
     long long blocks = (long long)rows * (K / 32);
-    launch_quant_mx<true>(in_dtype, bf16_wide(in_dtype, x, ld_x, q, ld_q, 4), blocks,
+    launch_quant_mx<2>(in_dtype, bf16_wide(in_dtype, x, ld_x, q, ld_q, 4), blocks,
                           (hipStream_t)stream, x, rows, K, ld_x, (uint8_t*)q, ld_q,
                           (uint8_t*)scales, ld_s, scale_rule);
+    GA_HIP_CHECK(hipGetLastError());
+    return GA_OK;
+}
+
+ga_status ga_prepare_mx_a(const void* x, int in_dtype, int M, int K, int ld_x, int elem,
+                          void* codes, void* scales, int scale_rule, void* stream)
+{
+    if (check_in(in_dtype) != GA_OK)
+        return GA_ERR_ARG;
+    if (!x || !codes || !scales || M <= 0 || K <= 0 || ld_x < K || scale_rule < 0 ||
+        scale_rule > 2 || elem < 0 || elem > 2)
+        return fail(GA_ERR_ARG, "prepare_mx_a: bad argument (elem 0 E4M3, 1 E5M2, 2 e2m1)");
+    if (K % 32 || ld_x % 4)
+        return fail(GA_ERR_SHAPE, "prepare_mx_a: K %% 32 and ld_x %% 4 must be 0");
+    const int sn = (K / 32 + 7) / 8 * 8;
+    // one workgroup per 32 rows (padded to 256) x 256 K
+    const dim3 grid((unsigned)(((long long)M + 255) / 256 * 8 * (sn / 8)));
+    const bool wide = bf16_wide(in_dtype, x, ld_x, codes, elem == 2 ? K / 2 : K, elem == 2 ? 4 : 8);
+    hipStream_t st = (hipStream_t)stream;
+    uint8_t *q = (uint8_t*)codes, *s = (uint8_t*)scales;
+    if (elem == 2)
+        launch_prepare_mx_a<2>(in_dtype, wide, grid, st, x, M, K, ld_x, q, s, sn, scale_rule);
+    else if (elem == 1)
+        launch_prepare_mx_a<1>(in_dtype, wide, grid, st, x, M, K, ld_x, q, s, sn, scale_rule);
+    else
+        launch_prepare_mx_a<0>(in_dtype, wide, grid, st, x, M, K, ld_x, q, s, sn, scale_rule);
     GA_HIP_CHECK(hipGetLastError());
     return GA_OK;
 }

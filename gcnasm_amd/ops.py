@@ -125,15 +125,20 @@ class MxOperand:
         self.codes, self.scales, self.rows, self.K = codes, scales, rows, K
 
 
+def _prepare_a(x, sh, elem, scale_rule, stream):
+    M, K = _rows(x)
+    codes = torch.empty((sh.a_rows_pad(), sh.Kp()), dtype=torch.uint8, device=x.device)
+    ss = torch.empty((sh.scale_a_rows() * sh.scale_cols(),), dtype=torch.uint8, device=x.device)
+    check(lib().ga_prepare_mx_a(x.data_ptr(), _in_dtype(x), M, K, x.stride(0), elem,
+                                codes.data_ptr(), ss.data_ptr(), scale_rule,
+                                _stream_handle(stream)))
+    return MxOperand(codes, ss, M, K)
+
+
 def prepare_mx_a(x, scale_rule=_lib.GA_MX_SCALE_FLOOR_448, stream=None):
     """Activation [M, K] -> MxOperand (A rows zero-padded to 256)."""
     M, K = x.shape
-    sh = Shape(M, 1, K)
-    q, s = quant_mxfp8(x, scale_rule, stream)
-    codes = torch.zeros((sh.a_rows_pad(), K), dtype=torch.uint8, device=x.device)
-    codes[:M].copy_(q)
-    ss = shuffle_scale(s, sh.scale_a_rows(), sh.scale_cols(), stream)
-    return MxOperand(codes, ss, M, K)
+    return _prepare_a(x, Shape(M, 1, K), 0, scale_rule, stream)
 
 
 def prepare_mx_b(w, scale_rule=_lib.GA_MX_SCALE_FLOOR_448, bpreshuffle=True, stream=None):
@@ -149,12 +154,7 @@ def prepare_mx_b(w, scale_rule=_lib.GA_MX_SCALE_FLOOR_448, bpreshuffle=True, str
 def prepare_mx4_a(x, scale_rule=_lib.GA_MX_SCALE_FLOOR_448, stream=None):
     """Activation [M, K] -> MXFP4 MxOperand: packed e2m1 [round_up(M, 256), K/2]."""
     M, K = x.shape
-    sh = Shape(M, 1, K, elem_bits=4)
-    q, s = quant_mxfp4(x, scale_rule, stream)
-    codes = torch.zeros((sh.a_rows_pad(), K // 2), dtype=torch.uint8, device=x.device)
-    codes[:M].copy_(q)
-    ss = shuffle_scale(s, sh.scale_a_rows(), sh.scale_cols(), stream)
-    return MxOperand(codes, ss, M, K)
+    return _prepare_a(x, Shape(M, 1, K, elem_bits=4), 2, scale_rule, stream)
 
 
 def prepare_mx4_b(w, scale_rule=_lib.GA_MX_SCALE_FLOOR_448, bpreshuffle=True, stream=None):

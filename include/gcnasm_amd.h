@@ -295,6 +295,15 @@ ga_status ga_quant_mx8(const void* x, int in_dtype, int rows, int K, int ld_x, v
 ga_status ga_quant_mxfp4(const void* x, int in_dtype, int rows, int K, int ld_x,
                          void* q, int ld_q, void* scales, int ld_s, int scale_rule,
                          void* stream);
+/* An MX activation operand in the GEMMs' layout in one pass: x [M, K] (row
+ * stride ld_x elements) -> codes [round_up(M, 256), K] E4M3 (elem 0) or E5M2
+ * (elem 1), or [round_up(M, 256), K/2] packed e2m1 (elem 2), rows past M
+ * zero, and the scales padded with 0x7F to [round_up(M, 256),
+ * round_up(K/32, 8)] and shuffled. The same bytes as the quantiser, zero rows
+ * and ga_shuffle_scale_device. K % 32 == 0, ld_x % 4 == 0; codes 8-byte and
+ * scales 4-byte aligned. */
+ga_status ga_prepare_mx_a(const void* x, int in_dtype, int M, int K, int ld_x, int elem,
+                          void* codes, void* scales, int scale_rule, void* stream);
 /* DeepSeek activation quantiser: per 1x128 block along K, s = amax/448 (fp32),
  * q = e4m3(x / s). Scales are written transposed, sfa[k/128 * ld_s + row]
  * (opus SFA layout [K/128, M]). K % 128 == 0. */

@@ -336,3 +336,45 @@ def test_quant_per_tensor_scratch_sizes(dev, n, in_bf16):
             np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32),
                                           np.asarray(scale, np.float32).reshape(1).view(np.uint32))
             np.testing.assert_array_equal(q.cpu().numpy(), want.reshape(-1))
+
+
+@pytest.mark.parametrize("rule", [0, 1, 2])
+@pytest.mark.parametrize("in_bf16", [False, True])
+@pytest.mark.parametrize("M,K", [(1, 32), (17, 288), (32, 256), (33, 1056), (256, 512), (300, 384)])
+def test_prepare_activations_one_pass(dev, M, K, in_bf16, rule):
+    """prepare_mx_a / prepare_mx4_a and the E5M2 form write the bytes of the
+    oracle's quantiser, zero rows and the oracle's scale shuffle, from rows
+    with a stride and from a base that does not allow 16-byte loads; NaN,
+    infinities and an all-zero block among the values."""
+    from gcnasm_amd import _lib
+    buf = oracle.gen_mx_input(M, K + 64, 9 + rule, 1.0, 6)
+    buf[0, 4:8] = [np.nan, np.inf, -np.inf, -np.nan]
+    buf[M - 1, K - 28:K] = 0.0
+    if in_bf16:
+        bits = oracle.to_bf16_bits(buf)
+        buf = oracle.bf16_bits_to_f32(bits)
+        t = torch.from_numpy(bits.view(np.int16)).to(dev).view(torch.bfloat16)
+    else:
+        t = torch.from_numpy(buf).to(dev)
+    sh = f4gemm.Shape(M, 1, K)
+    rows, cols = sh.scale_a_rows(), sh.scale_cols()
+    for off in (0, 4):
+        x, xt = np.ascontiguousarray(buf[:, off:off + K]), t[:, off:off + K]
+        for elem in (0, 1, 2):
+            q, s = (oracle.quant_mxfp8(x, rule) if elem == 0 else
+                    oracle.quant_mx8(x, 1, rule) if elem == 1 else oracle.quant_mxfp4(x, rule))
+            want = np.zeros((rows, q.shape[1]), np.uint8)
+            want[:M] = q
+            if elem == 1:
+                codes = torch.full(want.shape, 0xAA, dtype=torch.uint8, device=dev)
+                scales = torch.full((rows * cols,), 0xAA, dtype=torch.uint8, device=dev)
+                _lib.check(_lib.lib().ga_prepare_mx_a(
+                    xt.data_ptr(), 1 if in_bf16 else 0, M, K, xt.stride(0), 1, codes.data_ptr(),
+                    scales.data_ptr(), rule, None))
+            else:
+                a = (ops.prepare_mx_a if elem == 0 else ops.prepare_mx4_a)(xt, rule)
+                codes, scales = a.codes, a.scales
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(codes.cpu().numpy(), want)
+            np.testing.assert_array_equal(scales.cpu().numpy(),
+                                          oracle.shuffle_scale(s, M, K // 32, rows, cols))
