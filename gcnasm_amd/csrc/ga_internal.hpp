@@ -84,8 +84,10 @@ size_t bs_sk_counter_bytes(const ga_opus_gemm_kargs& ka);
 size_t bs_sk_workspace_bytes(const ga_opus_gemm_kargs& ka, int nwg);
 void launch_bs_pp_sk(const ga_opus_gemm_kargs& ka, int mode, int out_dtype, int nwg, void* ws,
                      hipStream_t stream);
-// The same GEMMs for up to 64 rows, streaming B (gemm_bs_decode.hip); same
-// mode numbering.
+// The same GEMMs for few rows, K cut over the waves of a workgroup
+// (gemm_bs_decode.hip); same mode numbering. bs_decode_estimate_us: its
+// estimated time.
+float bs_decode_estimate_us(const ga_opus_gemm_kargs& ka, int num_cu);
 ga_status launch_bs_decode(const ga_opus_gemm_kargs& ka, int mode, int out_dtype,
                            hipStream_t stream);
 // 128-K groups per K slice of that kernel (slices are summed in order).

@@ -13,16 +13,14 @@
 // through the buffer range check; a partial last N group of 128 is fine).
 // C is fp32 (the reference's output type) or bf16.
 //
-// 33-64 rows with enough columns, or more rows whose 128x128 tiles fit on
-// the CUs in one round (this file): 4 waves, 64x256 or 128x128 tile, K step
-// 128, three LDS stages, A and B
-// staged with buffer_load ... lds (8 whole 128-byte rows per instruction)
-// into swizzled LDS rows (chunk c of row r at slot c ^ ((r >> 1) & 7)),
-// v_mfma_scale_f32_16x16x128_f8f6f4 with unit E8M0 scales (127) and the
-// operands swapped so a lane owns 4 consecutive N of one C row. More rows go
-// to the 256x256 eight-wave kernel of gemm_bs_pp.hip, fewer rows (or too
-// few 256-column tiles) to the
-// B-streaming kernel of gemm_bs_decode.hip.
+// More rows than the K-split kernel of gemm_bs_decode.hip is the faster one
+// for, while the 128x128 tiles fit on the CUs in one round (this file): 4 waves,
+// 128x128 tile, K step 128, three LDS stages, A and B staged with buffer_load
+// ... lds (8 whole 128-byte rows per instruction) into swizzled LDS rows (chunk
+// c of row r at slot c ^ ((r >> 1) & 7)), v_mfma_scale_f32_16x16x128_f8f6f4 with
+// unit E8M0 scales (127) and the operands swapped so a lane owns 4 consecutive
+// N of one C row. More tiles go to the 256x256 eight-wave kernel of
+// gemm_bs_pp.hip.
 #include "ga_device.hpp"
 #include "ga_internal.hpp"
 #include "ga_pp.hpp"
@@ -281,26 +279,34 @@ static ga_status launch_bs(const ga_opus_gemm_kargs& ka, hipStream_t stream)
 }
 
 // Which kernel dispatch_bs runs for these kargs on a device with num_cu CUs.
-enum BsPath { BS_PATH_TILE128, BS_PATH_PP, BS_PATH_TILE64, BS_PATH_DECODE };
+enum BsPath { BS_PATH_TILE128, BS_PATH_PP, BS_PATH_DECODE };
 static BsPath bs_path(const ga_opus_gemm_kargs& ka, int num_cu)
 {
-    // More than 64 rows: the 256x256 eight-wave kernel (gemm_bs_pp.hip), or
-    // this file's 128x128 tile when its tiles fit on the CUs in one round
-    // (measured on MI355X, fp32 C: 512x7168x2048 35.4 -> 18.8 us,
-    // 512x2112x7168 86.1 -> 43.7 us, 1024x4096x4096 54.9 -> 29.7 us; with a
-    // second round, e.g. 768x7168x2048, the eight-wave kernel is faster).
-    if (ka.m > 64) {
-        const long long t128 =
-            (long long)((ka.m + 127) / 128) * ((ka.n + 127) / 128) * ka.batch;
-        return t128 <= num_cu ? BS_PATH_TILE128 : BS_PATH_PP;
+    // Up to 64 rows: the K-split kernel (gemm_bs_decode.hip). More rows: it
+    // against the 256x256 eight-wave kernel (gemm_bs_pp.hip), or against this
+    // file's 128x128 tile when its tiles fit on the CUs in one round (measured
+    // on MI355X, fp32 C: 512x7168x2048 35.4 -> 18.8 us; with a second round,
+    // e.g. 768x7168x2048, the eight-wave kernel is faster), by their estimated
+    // times. The tiles' times hardly depend on how many of the CUs a round
+    // covers: 4.5 + 0.72 us per 128-K group for the 128x128 tile (measured
+    // 11.0 us at 8 groups, 17.0 at 16, 28.2 at 32, 50.7 at 64), 10.7 + 1.2 per
+    // group and round for the 256x256 kernel (25.2 at 12, 29.6 at 16, 87 at
+    // 64; 51.3 for two rounds at 12). The K-split kernel was measured up to 768
+    // rows and is not considered above 1024.
+    if (ka.m <= 64)
+        return BS_PATH_DECODE;
+    const long long t128 = (long long)((ka.m + 127) / 128) * ((ka.n + 127) / 128) * ka.batch;
+    const bool one_round = t128 <= num_cu;
+    if (ka.m <= 1024) {
+        const long long t256 = (long long)((ka.m + 255) / 256) * ((ka.n + 255) / 256) * ka.batch;
+        const float groups = (float)(ka.k / 128);
+        const float tile_us = one_round ? 4.5f + 0.72f * groups
+                                        : (float)((t256 + num_cu - 1) / num_cu) *
+                                              (10.7f + 1.2f * groups);
+        if (bs_decode_estimate_us(ka, num_cu) < tile_us)
+            return BS_PATH_DECODE;
     }
-    // Up to 64 rows: the B-streaming kernel (gemm_bs_decode.hip), unless
-    // 33-64 rows leave this file's 64x256 tile enough workgroups (a quarter
-    // of the CUs): then its A reuse across 256 columns wins.
-    const long long tiles = (long long)((ka.n + 255) / 256) * ka.batch;
-    if (ka.m > 32 && tiles * 4 >= num_cu)
-        return BS_PATH_TILE64;
-    return BS_PATH_DECODE;
+    return one_round ? BS_PATH_TILE128 : BS_PATH_PP;
 }
 
 template <int MODE, int OUT>
@@ -317,8 +323,6 @@ static ga_status dispatch_bs(const ga_opus_gemm_kargs& ka, hipStream_t stream)
         launch_bs_pp(ka, MODE, OUT, stream);
         GA_HIP_CHECK(hipGetLastError());
         return GA_OK;
-    case BS_PATH_TILE64:
-        return launch_bs<BsCfg<64, 256, 1, 4, MODE, OUT>>(ka, stream);
     default:
         return launch_bs_decode(ka, MODE, OUT, stream);
     }
@@ -386,7 +390,10 @@ static ga_status bs_stream_k_plan(const ga_opus_gemm_kargs& ka, int* nwg)
     ga_status st = device_cu_count(&num_cu);
     if (st != GA_OK)
         return st;
-    *nwg = bs_path(ka, num_cu) == BS_PATH_PP ? bs_sk_workgroups(ka, num_cu) : 0;
+    // (in place of the 256x256 kernel, and of the K-split kernel where its
+    // 128x128 tiles would not fit on the CUs in one round either)
+    const long long t128 = (long long)((ka.m + 127) / 128) * ((ka.n + 127) / 128) * ka.batch;
+    *nwg = ka.m > 64 && t128 > num_cu ? bs_sk_workgroups(ka, num_cu) : 0;
     return GA_OK;
 }
 

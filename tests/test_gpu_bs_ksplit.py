@@ -1,0 +1,88 @@
+"""The K-split kernel of the fp32-scaled FP8 GEMMs (few rows): every wave tile
+and slice count its plan picks, at the edges of rows, columns and K, with
+padded strides and batches, against the CPU oracle in the K slices the library
+reports."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from gcnasm_amd import _lib, opus_gemm
+from helpers import assert_parity, bf16_compare, f32_compare
+
+pytestmark = pytest.mark.gpu
+
+# rows: one block of 16 or 32, two to four of 32, blocks of 64 with a short
+# last one; columns below, at and past a 16-column group and a 128-column
+# block, few and many groups; K of one group, fewer groups than slices, a
+# number that no slice count divides, and long.
+SHAPES = [(1, 16, 128), (1, 37, 256), (15, 4112, 384), (16, 8200, 1152), (17, 130, 640),
+          (32, 2100, 1152), (33, 1000, 2048), (63, 4097, 384), (64, 24576, 256), (65, 300, 128),
+          (127, 2112, 896), (128, 1024, 3456), (129, 515, 1152), (200, 6000, 640),
+          (300, 2113, 1792), (513, 1032, 1024), (700, 4096, 512), (1024, 200, 1280),
+          (8, 64, 8192), (24, 80, 7168), (64, 96, 7168)]
+
+
+def problem(batch, M, N, K, group_n, seed):
+    rng = np.random.default_rng(seed)
+    G = K // 128
+
+    def codes(rows):
+        x = rng.standard_normal((batch, rows, K)).astype(np.float32)
+        return np.stack([oracle.quant_fp8_per_tensor(v)[0] for v in x])
+
+    sfa = rng.uniform(0.5, 2.0, (batch, G, M)).astype(np.float32)
+    shape = (batch, -(-N // 128), G) if group_n == 128 else (batch, G, N)
+    return codes(M), codes(N), sfa, rng.uniform(0.5, 2.0, shape).astype(np.float32)
+
+
+def padded(x, ld, dev):
+    """x [batch, rows, K] on the device with rows of ld bytes, the pad 0x7F (NaN codes)."""
+    out = np.full(x.shape[:-1] + (ld,), 0x7F, x.dtype)
+    out[..., :x.shape[-1]] = x
+    return torch.from_numpy(out).to(dev)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("group_n", [128, 1, 0])
+def test_k_split_kernel(dev, shape, group_n):
+    M, N, K = shape
+    batch, pad_a, pad_b, pad_c = (2, 16, 48, 3) if M <= 129 and N <= 1100 else (1, 0, 32, 4)
+    qa, qb, sfa, sfb = problem(batch, M, N, K, group_n or 128, M + N + K)
+    gps = opus_gemm.k_slices(M, N, K, batch)
+    A, B = padded(qa, K + pad_a, dev), padded(qb, K + pad_b, dev)
+    SA, SB = torch.from_numpy(sfa).to(dev), torch.from_numpy(sfb).to(dev)
+    rows = np.unique(np.r_[np.arange(min(M, 48)), np.arange(max(0, M - 20), M)])
+    want, absdot = [], []
+    for b in range(batch):
+        a = np.ascontiguousarray(qa[b][rows])
+        if group_n:
+            s = np.ascontiguousarray(sfa[b][:, rows])
+            want.append(oracle.gemm_blockscale_mfma(a, qb[b], s, sfb[b], group_n, gps))
+            absdot.append(oracle.blockscale_absdot(a, qb[b], s, sfb[b], group_n))
+        else:
+            sa, sb = sfa[0].reshape(-1)[:1], sfb[0].reshape(-1)[:1]
+            want.append(oracle.gemm_per_tensor_mfma(a, qb[b], sa, sb, gps))
+            absdot.append(oracle.fp8_absdot(a, qb[b]) * float(sa[0]) * float(sb[0]))
+    want, absdot = np.stack(want), np.stack(absdot)
+    for dtype in (torch.float32, torch.bfloat16):
+        C = torch.full((batch, M, N + pad_c), float("nan"), dtype=dtype, device=dev)
+        ka = opus_gemm.make_kargs(A, B, C, SA, SB, M, N, K, batch, group_n)
+        ka.stride_a, ka.stride_b, ka.stride_c = K + pad_a, K + pad_b, N + pad_c
+        ka.stride_a_batch, ka.stride_b_batch = M * ka.stride_a, N * ka.stride_b
+        ka.stride_c_batch = M * ka.stride_c
+        out = _lib.GA_DTYPE_F32 if dtype == torch.float32 else _lib.GA_DTYPE_BF16
+        print("k-split", shape, group_n, dtype, "groups per slice", gps, flush=True)
+        if group_n:
+            opus_gemm.gemm_a8w8_blockscale(ka, out, group_n)
+        else:
+            opus_gemm.fp8_gemm(ka, out)
+        torch.cuda.synchronize()
+        assert torch.isnan(C[:, :, N:]).all() and not torch.isnan(C[:, :, :N]).any()
+        got = C[:, rows, :N].contiguous()
+        if dtype == torch.float32:
+            ok, st = f32_compare(got.cpu().numpy(), want, absdot=absdot)
+        else:
+            ok, st = bf16_compare(got.view(torch.int16).cpu().numpy().view(np.uint16),
+                                  oracle.to_bf16_bits(want), absdot)
+        assert_parity(st, "k-split %s g%d %s" % (shape, group_n, dtype))
