@@ -69,6 +69,15 @@ void launch_mx_decode_split(const ga_f4gemm_kargs& args, int gdz, int phys, int 
 // 256x256 eight-wave kernel with operand formats fmt, grid of its own tiles.
 void launch_mx_pp_fmt(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh,
                       int gdz, bool bps, int fmt, hipStream_t stream);
+// Few rows, small tiles, K cut over the waves of a workgroup
+// (gemm_mx_ksplit.hip): gdz 1, 2, 4 or 8 K slices, no workspace (wsh: a caller's
+// slot, only checked). mx_ksplit_estimate_us: its estimated time at one slice.
+float mx_ksplit_estimate_us(const ga_f4gemm_kargs& args, bool fp4, int num_cu);
+void launch_mx_ksplit(const ga_f4gemm_kargs& args, int gdz, bool bps, bool fp4, int fmt,
+                      const ga_splitk_ws_handle* wsh, int num_cu, hipStream_t stream);
+// 128x256 eight-wave kernel, any MX element format, grid of its own tiles.
+void launch_mx_pp_half(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh,
+                       int gdz, bool bps, bool fp4, int fmt, hipStream_t stream);
 
 // Compute units of the current device (queried once per device).
 ga_status device_cu_count(int* num_cu);

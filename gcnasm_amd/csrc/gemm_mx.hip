@@ -957,14 +957,52 @@ size_t ga_kernel_workspace_bytes(int idx, const ga_launch_desc* ld, int M, int N
 
 namespace ga {
 
+// Which kernel a launch runs: the entry's own, or one picked by the shape. The
+// choice is the same for every entry of an element width (and for either B
+// layout and every 8-bit format), so the output does not depend on the tile a
+// caller names; the K-split kernel's sums are cut in K, the others' not.
+enum MxRoute { MX_ROUTE_OWN, MX_ROUTE_KSPLIT, MX_ROUTE_HALF };
+
+static MxRoute mx_route(const ga_f4gemm_kargs& a, bool fp4, int gdz, int num_cu)
+{
+    const long long M = a.M, N = a.N, K = a.K;
+    if (M <= 64) {
+        // The few-row kernels (gemm_mx_decode.hip) keep the weights that come
+        // from HBM and the splits that are not 2, 4 or 8 even slices; the
+        // K-split kernel takes the smaller ones, from 17 rows on up to 96 MB
+        // (measured on MI355X, MXFP8, 64 rows, theirs against its: 8192x8192
+        // 23.2 / 14.8 us, 28672x8192 41.6 / 52.6, 8192x28672 at eight slices
+        // 51.6 / 63; 16 rows, 8192x8192 12.9 / 13.0, 5120x5120 10.4 / 7.5).
+        const long long mb = N * K / (fp4 ? 2 : 1) >> 20;
+        if (gdz == 1)
+            return mb <= (M <= 16 ? 48 : 96) ? MX_ROUTE_KSPLIT : MX_ROUTE_OWN;
+        return M > 16 && (gdz == 2 || gdz == 4 || gdz == 8) && mb <= 96 ? MX_ROUTE_KSPLIT
+                                                                       : MX_ROUTE_OWN;
+    }
+    // More rows: while the 128x256 tiles fit on the CUs in one round, they (256
+    // tiles of 256x256 would be at most half a round) or the K-split kernel, by
+    // estimated time. A tile's time is a start, and per K step a little more the
+    // more CUs compete for L2 and power (MXFP8, 64 steps: 44 us with 32 tiles,
+    // 45 with 128, 55 with 192, 60 with 256; MXFP4, 32 steps: 31 with 32, 38
+    // with 256). With more tiles the entry's own kernel, mostly 256x256, is the
+    // faster one (1536x8192x8192: 88 us against 111).
+    const long long tiles = (M + 127) / 128 * ((N + 255) / 256);
+    if (gdz != 1 || tiles > num_cu)
+        return MX_ROUTE_OWN;
+    const float frac = (float)tiles / (float)num_cu;
+    const float steps = (float)(K / (fp4 ? 256 : 128));
+    const float half_us = 6.0f + steps * (fp4 ? 0.80f + 0.22f * frac : 0.62f + 0.25f * frac);
+    return mx_ksplit_estimate_us(a, fp4, num_cu) < half_us ? MX_ROUTE_KSPLIT : MX_ROUTE_HALF;
+}
+
 // ga_kernel_launch with the split-K workspace given either as a buffer
 // (workspace, workspace_bytes; NULL: the library-owned one) or as a device
 // slot read by the kernels at entry (wsh; graph-capture safe), and the
 // operand element formats fmt = fmt(A) | fmt(B) << 1 (0 E4M3, 1 E5M2; MXFP8
-// kernels only). With fmt != 0 the rows above the decode path run the
-// 256x256 kernel whatever the entry's tile: every MXFP8 kernel computes the
-// same fp32 chain of 128-K steps per K slice, so the tile is not visible in
-// the output.
+// kernels only). With fmt != 0 the rows above the decode path that no route
+// takes run the 256x256 kernel whatever the entry's tile: every tile kernel
+// computes the same fp32 chain of 128-K steps per K slice, so the tile is not
+// visible in the output.
 static ga_status kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, int gdy, int gdz,
                                void* workspace, size_t workspace_bytes,
                                const ga_splitk_ws_handle* wsh, void* stream, int fmt = 0)
@@ -1036,25 +1074,33 @@ static ga_status kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, in
     if (gdz > 1 && workspace && workspace_bytes < (size_t)gdz * M * N * sizeof(float))
         return fail(GA_ERR_WORKSPACE, "workspace %zu bytes, need %zu", workspace_bytes,
                     (size_t)gdz * M * N * sizeof(float));
-    const bool decode = (int)args->M <= k.small_m_stream && mx_decode_applies(*args, gdz);
     int num_cu = 0;
-    if (decode) {
+    {
         ga_status st = device_cu_count(&num_cu);
         if (st != GA_OK)
             return st;
     }
+    const bool fp4 = k.elem_bits == 4, bps = k.cfg.bpreshuffle != 0;
+    const MxRoute route = mx_route(*args, fp4, gdz, num_cu);
+    const bool decode = (int)args->M <= k.small_m_stream && mx_decode_applies(*args, gdz);
     int phys = gdz; // workgroups along K of the 17-64-row decode kernels
     const int split_groups = decode ? mx_decode_split_groups(*args, gdz, num_cu, &phys) : 0;
+    const bool no_ws = gdz == 1 || (decode && (split_groups == 0 || phys == 1));
+    if (route == MX_ROUTE_KSPLIT && no_ws) {
+        launch_mx_ksplit(*args, gdz, bps, fp4, fmt, nullptr, num_cu, s);
+        GA_HIP_CHECK(hipGetLastError());
+        return GA_OK;
+    }
     if (decode && split_groups == 0) {
         // few rows: stream B, K slices summed inside the kernel (no workspace)
-        launch_mx_decode(*args, gdz, k.cfg.bpreshuffle != 0, k.elem_bits == 4, fmt, num_cu, s);
+        launch_mx_decode(*args, gdz, bps, fp4, fmt, num_cu, s);
         GA_HIP_CHECK(hipGetLastError());
         return GA_OK;
     }
     if (decode && phys == 1) {
         // 17-64 rows, every K slice in one workgroup along K (no workspace)
-        launch_mx_decode_split(*args, gdz, 1, split_groups, k.cfg.bpreshuffle != 0,
-                               k.elem_bits == 4, fmt, nullptr, nullptr, num_cu, s);
+        launch_mx_decode_split(*args, gdz, 1, split_groups, bps, fp4, fmt, nullptr, nullptr,
+                               num_cu, s);
         GA_HIP_CHECK(hipGetLastError());
         return GA_OK;
     }
@@ -1082,18 +1128,28 @@ static ga_status kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, in
             if (cs != hipStreamCaptureStatusNone)
                 return fail(GA_ERR_WORKSPACE, "split-K launch under stream capture needs a "
                                               "caller workspace");
-            void* p = nullptr;
-            ga_status st = default_workspace(need, &p);
-            if (st != GA_OK)
-                return st;
-            ws = (float*)p;
+            if (route != MX_ROUTE_KSPLIT) {
+                void* p = nullptr;
+                ga_status st = default_workspace(need, &p);
+                if (st != GA_OK)
+                    return st;
+                ws = (float*)p;
+            }
         }
     }
-    if (split_groups > 0)
-        launch_mx_decode_split(*args, gdz, phys, split_groups, k.cfg.bpreshuffle != 0, k.elem_bits == 4,
-                               fmt, ws, wsh, num_cu, s);
+    if (route == MX_ROUTE_KSPLIT) {
+        // the slices are summed in the workgroup, no partials and no reduce; the
+        // workspace rules of a split call above hold as for the other kernels
+        launch_mx_ksplit(*args, gdz, bps, fp4, fmt, wsh, num_cu, s);
+        GA_HIP_CHECK(hipGetLastError());
+        return GA_OK;
+    }
+    if (route == MX_ROUTE_HALF)
+        launch_mx_pp_half(*args, ws, nullptr, gdz, bps, fp4, fmt, s);
+    else if (split_groups > 0)
+        launch_mx_decode_split(*args, gdz, phys, split_groups, bps, fp4, fmt, ws, wsh, num_cu, s);
     else if (fmt != 0)
-        launch_mx_pp_fmt(*args, ws, gdz > 1 ? wsh : nullptr, gdz, k.cfg.bpreshuffle != 0, fmt, s);
+        launch_mx_pp_fmt(*args, ws, gdz > 1 ? wsh : nullptr, gdz, bps, fmt, s);
     else
         k.launch(*args, ws, gdz > 1 ? wsh : nullptr, gdx, gdy, gdz, s);
     GA_HIP_CHECK(hipGetLastError());

@@ -181,6 +181,29 @@ struct PpArgs {
     int log2_k_split;
 };
 
+__device__ __forceinline__ PpArgs uni_args(const ga_f4gemm_kargs& args)
+{
+    PpArgs a;
+    a.ptr_A = uni_ptr(args.ptr_A);
+    a.ptr_B = uni_ptr(args.ptr_B);
+    a.ptr_ScaleA = uni_ptr(args.ptr_ScaleA);
+    a.ptr_ScaleB = uni_ptr(args.ptr_ScaleB);
+    a.ptr_C = uni_ptr(args.ptr_C);
+    a.ptr_D = uni_ptr(args.ptr_D);
+    a.alpha = args.alpha; // epilogue VALU operands: may stay in VGPRs
+    a.beta = args.beta;
+    a.M = uni(args.M);
+    a.N = uni(args.N);
+    a.K = uni(args.K);
+    a.stride_A0 = uni(args.stride_A0);
+    a.stride_B0 = uni(args.stride_B0);
+    a.stride_ScaleA0 = uni(args.stride_ScaleA0);
+    a.stride_ScaleB0 = uni(args.stride_ScaleB0);
+    a.stride_C0 = uni(args.stride_C0);
+    a.log2_k_split = (int)uni((uint32_t)args.log2_k_split);
+    return a;
+}
+
 // One 256x256 output tile (K slice blockIdx.z): prologue, K loop, epilogue.
 // On return every LDS read of the tile is complete (the last barrier is
 // after the last read); copies of steps past the slice may still be landing,
@@ -555,29 +578,306 @@ void mx_pp_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
     __shared__ __attribute__((aligned(1024))) char smem[kLds];
     if (wsh && !(ws = resolve_ws(wsh, gridDim.z, args.M, args.N)))
         return; // workspace slot shorter than the split-K layout: write nothing
-    PpArgs a;
-    a.ptr_A = uni_ptr(args.ptr_A);
-    a.ptr_B = uni_ptr(args.ptr_B);
-    a.ptr_ScaleA = uni_ptr(args.ptr_ScaleA);
-    a.ptr_ScaleB = uni_ptr(args.ptr_ScaleB);
-    a.ptr_C = uni_ptr(args.ptr_C);
-    a.ptr_D = uni_ptr(args.ptr_D);
-    a.alpha = args.alpha; // epilogue VALU operands: may stay in VGPRs
-    a.beta = args.beta;
-    a.M = uni(args.M);
-    a.N = uni(args.N);
-    a.K = uni(args.K);
-    a.stride_A0 = uni(args.stride_A0);
-    a.stride_B0 = uni(args.stride_B0);
-    a.stride_ScaleA0 = uni(args.stride_ScaleA0);
-    a.stride_ScaleB0 = uni(args.stride_ScaleB0);
-    a.stride_C0 = uni(args.stride_C0);
-    a.log2_k_split = (int)uni((uint32_t)args.log2_k_split);
+    const PpArgs a = uni_args(args);
     const int ntiles = tiles_x * tiles_y;
     for (int lin = blockIdx.x; lin < ntiles; lin += gridDim.x) {
         int tile_m, tile_n;
         map_tile_lin(lin, tiles_x, tiles_y, kPpGroupM, tile_m, tile_n);
         pp_tile<BPS, FP4, F>(a, ws, smem, tile_m, tile_n);
+    }
+    wait_vmcnt<0>(); // copies of steps past the last slice land before exit
+}
+
+// ---- 128x256 tile ------------------------------------------------------------------
+// The same pipeline for half the rows: two groups of four waves one barrier
+// apart, group g on rows 64g .. 64g + 63, SIMD s on columns 32s .. 32s + 31 of
+// both 128-column halves. A K step is one memory half (all its copies and
+// fragment reads) and one MFMA half of 16 MFMAs per group; three 48 KB slots,
+// a step's copies issued two steps ahead into the slot both groups have left.
+// For problems whose 256x256 tiles leave much of the last round idle: a step
+// takes about half as long and moves 48 KB instead of 64, so full rounds stay
+// with the larger tile.
+constexpr int kHSlot = 3 * kHalf; // A, B columns 0-127, B columns 128-255
+constexpr int kHScaleSlot = 12 * 256; // 4 A + 8 B shuffled 32-row scale blocks
+constexpr int kHScaleBase = 3 * kHSlot;
+constexpr int kHLds = kHScaleBase + 3 * kHScaleSlot;
+static_assert(kHLds <= 160 * 1024 && 128 * kStagePitch <= kHLds, "LDS budget");
+constexpr int kHGroupM = 8;
+
+// Copies (6 per wave) of K step t into slot `slot`.
+__device__ __forceinline__ void issue_h(const PpLoad& L, char* smem, int t, int slot, int wave)
+{
+    char* dst = smem + slot * kHSlot + wave * 1024;
+    const uint32_t oa = (uint32_t)t * 128, ob = (uint32_t)t * L.b_kstep;
+    lds_load16(L.ra, (lds_void*)dst, L.va + uni(oa), 0);
+    lds_load16(L.ra, (lds_void*)(dst + 8192), L.va + uni(oa + L.a_hstep), 0);
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+        lds_load16(L.rb, (lds_void*)(dst + kHalf + c * 8192), L.vb + uni(ob + c * L.b_hstep), 0);
+}
+
+// Half `half` (0: A rows, 1: B rows) of the scales of 256-K block `pair` into
+// ring slot `ring`: wave w copies block w of the 8 of B, block w % 4 of A.
+__device__ __forceinline__ void issue_hs(const PpLoad& L, char* smem, int pair, int half, int ring,
+                                         int wave)
+{
+    char* dst = smem + kHScaleBase + ring * kHScaleSlot + (half ? 4 + wave : wave & 3) * 256;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(half ? L.rsb : L.rsa, (lds_void*)dst, 4,
+                                             (half ? L.vsb : L.vsa) + uni((uint32_t)pair * 256), 0,
+                                             0, 0);
+}
+
+template <bool BPS, bool FP4, int F>
+__device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restrict__ ws,
+                                             char* smem, int tile_m, int tile_n)
+{
+    constexpr int kEPB = FP4 ? 2 : 1;
+    constexpr int kStepK = 128 * kEPB;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = wave >> 2, simd = wave & 3;
+    const int M = (int)args.M, N = (int)args.N, K = (int)args.K;
+    const int m0 = tile_m * 128, n0 = tile_n * 256;
+
+    const int z = blockIdx.z, gdz = gridDim.z;
+    int kpt = K;
+    if (gdz > 1)
+        kpt = ((K >> args.log2_k_split) + 255) / 256 * 256;
+    const int kb = z * kpt;
+    const int ke = min(K, kb + kpt);
+    const int nsteps = (ke - kb) / kStepK;
+    const int kbb = kb / kEPB;
+
+    v4f acc[2][4][2];
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+                acc[q][i][t] = (v4f){0.f, 0.f, 0.f, 0.f};
+
+    if (nsteps > 0) {
+        const uint32_t lda = args.stride_A0 / kEPB, ldb = args.stride_B0 / kEPB; // bytes
+        const int Kb = K / kEPB;                                                  // bytes
+        PpLoad L;
+        int crow, ckc;
+        copy_lane(wave, lane, crow, ckc);
+        {
+            const char* pa = (const char*)args.ptr_A + (size_t)m0 * lda;
+            long long abytes = (long long)(M - m0) * lda;
+            L.ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
+            L.va = (uint32_t)crow * lda + ckc * 16 + (uint32_t)kbb;
+            L.a_hstep = 64 * lda;
+            if (BPS) {
+                // copy c (64 columns): groups 4c + wave/2, bytes (wave&1)*1024 + lane*16
+                const char* pb = (const char*)args.ptr_B + (size_t)(n0 / 16) * Kb * 16;
+                long long bbytes = (long long)(N - n0) * Kb;
+                L.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+                L.b_kstep = 2048;
+                L.b_hstep = 4 * (uint32_t)Kb * 16;
+                L.vb = (uint32_t)(wave >> 1) * (uint32_t)Kb * 16 + (wave & 1) * 1024 +
+                       lane * 16 + (uint32_t)kbb * 16;
+            } else {
+                const char* pb = (const char*)args.ptr_B + (size_t)n0 * ldb;
+                long long bbytes = (long long)(N - n0) * ldb;
+                L.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+                L.b_kstep = 128;
+                L.b_hstep = 64 * ldb;
+                L.vb = (uint32_t)crow * ldb + ckc * 16 + (uint32_t)kbb;
+            }
+            const uint32_t sna = args.stride_ScaleA0, snb = args.stride_ScaleB0;
+            L.rsa = make_rsrc(args.ptr_ScaleA, (uint32_t)((M + 31) / 32 * 32) * sna);
+            L.rsb = make_rsrc(args.ptr_ScaleB, (uint32_t)((N + 31) / 32 * 32) * snb);
+            L.vsa = ((uint32_t)(m0 / 32 + (wave & 3)) * (sna / 8) + (uint32_t)(kb / 256)) * 256 +
+                    lane * 4;
+            L.vsb = ((uint32_t)(n0 / 32 + wave) * (snb / 8) + (uint32_t)(kb / 256)) * 256 +
+                    lane * 4;
+        }
+
+        ReadBase rb;
+        {
+            uint32_t o, o64;
+            operand_lane(lane, o, o64);
+            rb.a0 = smem + grp * 64 * 128 + o;
+            rb.a1 = smem + grp * 64 * 128 + o64;
+            if (BPS) {
+                rb.b0 = smem + kHalf + simd * 32 * 128 + lane * 16;
+                rb.b1 = rb.b0 + 1024;
+            } else {
+                rb.b0 = smem + kHalf + simd * 32 * 128 + o;
+                rb.b1 = smem + kHalf + simd * 32 * 128 + o64;
+            }
+            rb.sa = smem + kHScaleBase + grp * 2 * 256 + lane * 4;
+            rb.sb = smem + kHScaleBase + (4 + simd) * 256 + lane * 4;
+        }
+
+        v8i fa[4], fb0[2], fb1[2];
+        uint32_t sa[2], sb0, sb1;
+        // copies per step: 6 operand, 1 scale (MXFP8: half of a pair of steps)
+        // or 2 (MXFP4: a step is 256 K)
+        constexpr int kC = FP4 ? 8 : 7;
+        if constexpr (FP4) {
+            issue_h(L, smem, 0, 0, wave);
+            issue_hs(L, smem, 0, 0, 0, wave);
+            issue_hs(L, smem, 0, 1, 0, wave);
+            issue_h(L, smem, 1, 1, wave);
+            issue_hs(L, smem, 1, 0, 1, wave);
+            issue_hs(L, smem, 1, 1, 1, wave);
+        } else {
+            issue_hs(L, smem, 0, 0, 0, wave);
+            issue_hs(L, smem, 0, 1, 0, wave);
+            issue_h(L, smem, 0, 0, wave);
+            issue_hs(L, smem, 1, 0, 1, wave);
+            issue_h(L, smem, 1, 1, wave);
+            issue_hs(L, smem, 1, 1, 1, wave);
+        }
+        part_sync<kC>();
+        if (grp == 1)
+            slot_sync(); // second group runs one barrier behind
+
+        // Step s in slot S = s % 3: copies of step s + 2 into the slot of step
+        // s - 1, whose last reads (the second group's) ended one barrier ago.
+        // Waiting for all but the newest kC copies after the memory half
+        // retires step s + 1's, which either group reads two barriers on at
+        // the earliest. MXFP8 scales: half P of pair (s >> 1) + 2 (as in the
+        // 256x256 tile), read whole in even steps.
+        int r0 = 0; // scale ring slot of step s (MXFP8: of pair s >> 1)
+        auto step = [&](int s, auto SC, auto PC) {
+            constexpr int S = decltype(SC)::value, P = decltype(PC)::value;
+            const int r2 = r0 == 0 ? 2 : r0 - 1; // (r0 + 2) % 3
+            issue_h(L, smem, s + 2, (S + 2) % 3, wave);
+            if constexpr (FP4) {
+                issue_hs(L, smem, s + 2, 0, r2, wave);
+                issue_hs(L, smem, s + 2, 1, r2, wave);
+            } else {
+                issue_hs(L, smem, (s >> 1) + 2, P, r2, wave);
+            }
+            if constexpr (FP4 || P == 0) {
+                const char* pa = rb.sa + r0 * kHScaleSlot;
+                const char* pb = rb.sb + r0 * kHScaleSlot;
+                sa[0] = *(const uint32_t*)pa;
+                sa[1] = *(const uint32_t*)(pa + 256);
+                sb0 = *(const uint32_t*)pb;
+                sb1 = *(const uint32_t*)(pb + 4 * 256);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                fa[i] = lds_frag(rb.a0 + S * kHSlot + i * 2048, rb.a1 + S * kHSlot + i * 2048);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+                fb0[t] = lds_frag(rb.b0 + S * kHSlot + t * 2048, rb.b1 + S * kHSlot + t * 2048);
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+                fb1[t] = lds_frag(rb.b0 + S * kHSlot + kHalf + t * 2048,
+                                  rb.b1 + S * kHSlot + kHalf + t * 2048);
+            part_sync<kC>();
+            mma_two<FP4, F, FP4 ? 0 : 2 * P>(acc[0], acc[1], fa, fb0, fb1, sa, sb0, sb1);
+            part_sync<kC>();
+            if constexpr (FP4 || P == 1)
+                r0 = r0 == 2 ? 0 : r0 + 1;
+        };
+        // slot and parity are compile-time: six steps per iteration
+        int s = 0;
+        for (; s + 6 <= nsteps; s += 6)
+            static_for<6>([&](auto J) {
+                constexpr int j = decltype(J)::value;
+                step(s + j, std::integral_constant<int, j % 3>{},
+                     std::integral_constant<int, j % 2>{});
+            });
+        static_for<5>([&](auto J) {
+            constexpr int j = decltype(J)::value;
+            if (s + j < nsteps)
+                step(s + j, std::integral_constant<int, j % 3>{},
+                     std::integral_constant<int, j % 2>{});
+        });
+        if (grp == 0)
+            slot_sync(); // matches the second group's extra barrier
+    }
+
+    const int ldd = (int)args.stride_C0;
+    const float alpha = args.alpha, beta = args.beta;
+    const bool use_c = beta != 0.0f && args.ptr_C != nullptr;
+    const bool staged = gdz == 1 && !use_c && m0 + 128 <= M && n0 + 256 <= N && (ldd & 7) == 0 &&
+                        ((uintptr_t)args.ptr_D & 15) == 0;
+    if (staged) {
+        wait_vmcnt<0>();
+        wait_lds_barrier();
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    const v4f v = acc[q][i][t];
+                    const uint32_t lo = (uint32_t)f32_to_bf16(alpha * v[0]) |
+                                        ((uint32_t)f32_to_bf16(alpha * v[1]) << 16);
+                    const uint32_t hi = (uint32_t)f32_to_bf16(alpha * v[2]) |
+                                        ((uint32_t)f32_to_bf16(alpha * v[3]) << 16);
+                    stage_put(smem, grp * 64 + i * 16 + (lane & 15),
+                              q * 128 + simd * 32 + t * 16 + (lane >> 4) * 4, lo, hi);
+                }
+        barrier_lds();
+        uint16_t* dst = (uint16_t*)args.ptr_D + (size_t)m0 * ldd + n0;
+        const int col = (lane & 31) * 8;
+#pragma unroll
+        for (int it = 0; it < 8; it++) {
+            const int row = wave * 16 + it * 2 + (lane >> 5);
+            *(v4i*)(dst + (size_t)row * ldd + col) =
+                *(const v4i*)(smem + row * kStagePitch + col * 2);
+        }
+        barrier_lds(); // staged rows read before the LDS takes the next tile's copies
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int m = m0 + grp * 64 + i * 16 + (lane & 15);
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int n = n0 + q * 128 + simd * 32 + t * 16 + (lane >> 4) * 4;
+                if (m >= M || n >= N)
+                    continue;
+                const v4f v = acc[q][i][t];
+                if (gdz > 1) {
+                    *(v4f*)(ws + ((size_t)z * M + m) * N + n) = v;
+                } else {
+                    uint16_t o[4];
+                    const uint16_t* cin =
+                        use_c ? (const uint16_t*)args.ptr_C + (size_t)m * ldd + n : nullptr;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        float x = alpha * v[j];
+                        if (use_c)
+                            x = x + beta * bf16_to_f32(cin[j]);
+                        o[j] = f32_to_bf16(x);
+                    }
+                    uint2 pk;
+                    pk.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
+                    pk.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
+                    *(uint2*)((uint16_t*)args.ptr_D + (size_t)m * ldd + n) = pk;
+                }
+            }
+        }
+}
+
+template <bool BPS, bool FP4, int F = 0>
+__global__ __attribute__((amdgpu_flat_work_group_size(kNT, kNT), amdgpu_waves_per_eu(2, 2)))
+void mx_pp_half_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
+                       const ga_splitk_ws_handle* __restrict__ wsh, int tiles_x, int tiles_y)
+{
+    __shared__ __attribute__((aligned(1024))) char smem[kHLds];
+    if (wsh && !(ws = resolve_ws(wsh, gridDim.z, args.M, args.N)))
+        return; // workspace slot shorter than the split-K layout: write nothing
+    const PpArgs a = uni_args(args);
+    const int ntiles = tiles_x * tiles_y;
+    for (int lin = blockIdx.x; lin < ntiles; lin += gridDim.x) {
+        int tile_m, tile_n;
+        map_tile_lin(lin, tiles_x, tiles_y, kHGroupM, tile_m, tile_n);
+        pp_half_tile<BPS, FP4, F>(a, ws, smem, tile_m, tile_n);
     }
     wait_vmcnt<0>(); // copies of steps past the last slice land before exit
 }
@@ -652,6 +952,39 @@ void launch_mx_pp_fmt(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws
                 : launch_pp_f<false, 3>(args, ws, wsh, gdz, stream); break;
     default: bps ? launch_pp_f<true, 0>(args, ws, wsh, gdz, stream)
                  : launch_pp_f<false, 0>(args, ws, wsh, gdz, stream); break;
+    }
+}
+
+namespace {
+
+template <bool BPS, bool FP4, int F>
+void launch_half(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh, int gdz,
+                 hipStream_t stream)
+{
+    const int gdx = ((int)args.N + 255) / 256, gdy = ((int)args.M + 127) / 128;
+    hipLaunchKernelGGL((mx_pp_half_kernel<BPS, FP4, F>), dim3(pp_grid(gdx * gdy), 1, gdz),
+                       dim3(kNT), 0, stream, args, ws, wsh, gdx, gdy);
+}
+
+} // namespace
+
+void launch_mx_pp_half(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh,
+                       int gdz, bool bps, bool fp4, int fmt, hipStream_t stream)
+{
+    if (fp4) {
+        bps ? launch_half<true, true, 0>(args, ws, wsh, gdz, stream)
+            : launch_half<false, true, 0>(args, ws, wsh, gdz, stream);
+        return;
+    }
+    switch (fmt) {
+    case 1: bps ? launch_half<true, false, 1>(args, ws, wsh, gdz, stream)
+                : launch_half<false, false, 1>(args, ws, wsh, gdz, stream); break;
+    case 2: bps ? launch_half<true, false, 2>(args, ws, wsh, gdz, stream)
+                : launch_half<false, false, 2>(args, ws, wsh, gdz, stream); break;
+    case 3: bps ? launch_half<true, false, 3>(args, ws, wsh, gdz, stream)
+                : launch_half<false, false, 3>(args, ws, wsh, gdz, stream); break;
+    default: bps ? launch_half<true, false, 0>(args, ws, wsh, gdz, stream)
+                 : launch_half<false, false, 0>(args, ws, wsh, gdz, stream); break;
     }
 }
 

@@ -389,10 +389,11 @@ ga_status ga_kernel_launch_noalloc(int idx, const ga_f4gemm_kargs* args, int gdx
  * fmt_a / fmt_b of mfma_scale_f32_16x16x128_f8f6f4) at the GEMM level; the
  * reference's asm_f4gemm kernels have fixed formats. idx must be an MXFP8
  * registry entry (GA_ERR_ARG for MXFP4 kernels and other codes). Rows above
- * the decode path (M > 64) run the 256x256 eight-wave kernel whichever tile
- * idx names (the grid arguments are checked against idx as usual); every
- * MXFP8 kernel computes the same fp32 chain per K slice, so the output does
- * not depend on the tile. fmt_a = fmt_b = 0 is ga_kernel_launch. */
+ * the decode path (M > 64) run a kernel picked by the shape whichever tile
+ * idx names (the grid arguments are checked against idx as usual); the pick is
+ * the same for every entry and the tile kernels compute the same fp32 chain
+ * per K slice, so the output does not depend on the tile. fmt_a = fmt_b = 0 is
+ * ga_kernel_launch. */
 ga_status ga_kernel_launch_fmt(int idx, const ga_f4gemm_kargs* args, int gdx, int gdy, int gdz,
                                int fmt_a, int fmt_b, void* workspace, size_t workspace_bytes,
                                void* stream);

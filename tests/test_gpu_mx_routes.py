@@ -1,0 +1,128 @@
+"""The MX kernels that a launch's shape picks (the K-split kernel, the 128x256
+tile, the entry's own kernel), each at the edges of its tiles and of the rule
+that picks it, against the CPU oracle: formats, B layouts, splits, alpha and
+beta, a strided D."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from gcnasm_amd import f4gemm
+from helpers import assert_parity, bf16_compare
+
+pytestmark = pytest.mark.gpu
+
+NAMES = {(8, 1): "ga_mxfp8_bf16_BpreShuffle_256x256", (8, 0): "ga_mxfp8_bf16_noBpreShuffle_256x256",
+         (4, 1): "ga_mxfp4_bf16_BpreShuffle_256x256", (4, 0): "ga_mxfp4_bf16_noBpreShuffle_256x256"}
+
+
+def run(dev, M, N, K, elem, bps, fa=0, fb=0, l2=0, alpha=1.0, beta=0.0, pad_d=0, seed=1):
+    xa = oracle.gen_mx_input(M, K, seed, 1.0, 4)
+    xb = oracle.gen_mx_input(N, K, seed + 1, 1.0, 4)
+    if elem == 4:
+        (qa, sa), (qb, sb) = oracle.quant_mxfp4(xa), oracle.quant_mxfp4(xb)
+    else:
+        (qa, sa), (qb, sb) = oracle.quant_mx8(xa, fa), oracle.quant_mx8(xb, fb)
+    sh = f4gemm.Shape(M, N, K, elem_bits=elem)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)  # noqa: E731
+    A = t(qa)
+    B = t(f4gemm.shuffle_weight_16x16(qb, N, sh.Kp()) if bps else qb)
+    SA = t(f4gemm.shuffle_scale(sa, M, K // 32, sh.scale_a_rows(), sh.scale_cols()))
+    SB = t(f4gemm.shuffle_scale(sb, N, K // 32, sh.scale_b_rows(), sh.scale_cols()))
+    ldd = N + pad_d
+    D = torch.full((M, ldd), float("nan"), dtype=torch.bfloat16, device=dev)
+    C = torch.randn((M, ldd), generator=torch.Generator(device=dev).manual_seed(seed),
+                    device=dev).to(torch.bfloat16) if beta else None
+    name = NAMES[(elem, bps)] + ("_splitK" if l2 else "")
+    cfg = [c for c in f4gemm.manifest() + f4gemm.manifest_fp4() if c.knl_name == name][0]
+    ld = f4gemm.make_launch(cfg, M, N, K, l2)
+    args = f4gemm.fill_args(D, C, A, B, SA, SB, M, N, K, ldd, sh.scale_cols(),
+                            sh.scale_cols(), alpha, beta, ld.log2_k_split)
+    kern = f4gemm.Kernel().load(None, cfg)
+    ws = torch.empty(max(1, kern.workspace_bytes(ld, M, N) // 4), dtype=torch.float32, device=dev)
+    print("mx route", M, N, K, elem, bps, fa, fb, l2, flush=True)
+    kern.launch(args, ld.gdx, ld.gdy, ld.gdz, workspace=ws, fmt_a=fa, fmt_b=fb)
+    torch.cuda.synchronize()
+    assert torch.isnan(D[:, N:]).all() and not torch.isnan(D[:, :N]).any()
+    rows = np.unique(np.r_[np.arange(min(M, 24)), np.arange(max(0, M - 40), M),
+                           np.arange(0, M, 97)])
+    qr, sr = np.ascontiguousarray(qa[rows]), np.ascontiguousarray(sa[rows])
+    if elem == 4:
+        want = oracle.gemm_mx_fp32acc(qr, sr, qb, sb, 4, l2)
+        dot = oracle.mx4_absdot(qr, sr, qb, sb)
+    else:
+        want = oracle.gemm_mx8_mfma(qr, sr, qb, sb, fa, fb, l2)
+        dot = oracle.mx_absdot(qr, sr, qb, sb, fa, fb)
+    want = (np.float32(alpha) * want).astype(np.float32)
+    dot = abs(alpha) * dot
+    if beta:
+        c = C[:, :N].float().cpu().numpy()[rows]
+        want, dot = want + np.float32(beta) * c, dot + abs(beta) * np.abs(c)
+    got = D[:, :N].contiguous().view(torch.int16).cpu().numpy().view(np.uint16)[rows]
+    ok, st = bf16_compare(got, oracle.to_bf16_bits(want), dot)
+    assert_parity(st, "mx %dx%dx%d e%d bps%d f%d%d l%d" % (M, N, K, elem, bps, fa, fb, l2))
+
+
+# K-split: rows at the 32- and 64-row blocks, an odd number of 16-column groups,
+# one group, more shares than CUs; K of one 256-K unit, an odd number of steps
+# (MXFP8), fewer units than slices and long.
+KSPLIT = [(1, 16, 256), (16, 48, 1280), (17, 1040, 512), (31, 528, 768), (33, 2064, 1024),
+          (64, 144, 8192), (65, 16, 512), (96, 4112, 768), (129, 1040, 2304), (200, 3088, 1024),
+          (300, 784, 1536), (500, 2064, 512), (1000, 272, 1024)]
+
+
+@pytest.mark.parametrize("shape", KSPLIT)
+@pytest.mark.parametrize("elem,bps", [(8, 1), (8, 0), (4, 1), (4, 0)])
+def test_k_split(dev, shape, elem, bps):
+    run(dev, *shape, elem, bps, pad_d=4, seed=sum(shape))
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 272, 128), (70, 144, 384), (150, 528, 1152)])
+@pytest.mark.parametrize("bps", [1, 0])
+def test_k_split_odd_steps(dev, M, N, K, bps):
+    """MXFP8 K that is not a multiple of 256: the last slice ends in half a
+    scale block; alpha, beta and C."""
+    run(dev, M, N, K, 8, bps, alpha=0.5, beta=2.0, pad_d=8, seed=K)
+
+
+@pytest.mark.parametrize("fa,fb", [(1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("M,N,K,bps", [(48, 1040, 1024, 1), (130, 528, 768, 1),
+                                       (130, 528, 768, 0), (900, 8192, 512, 1)])
+def test_formats(dev, M, N, K, bps, fa, fb):
+    run(dev, M, N, K, 8, bps, fa, fb, seed=M)
+
+
+@pytest.mark.parametrize("l2", [1, 2, 3])
+@pytest.mark.parametrize("M,N,K", [(17, 1040, 2048), (64, 2064, 4096), (48, 528, 2304)])
+def test_k_split_keeps_a_callers_slices(dev, M, N, K, l2):
+    """17-64 rows with a split: the caller's slices as the kernel's (a short
+    last one among them), MXFP8 and MXFP4."""
+    run(dev, M, N, K, 8, 1, l2=l2, seed=l2)
+    run(dev, M, N, K, 4, 1, l2=l2, seed=l2)
+
+
+# The 128x256 tile: whole and ragged tiles, one K step to seven (its slots and
+# scale ring wrap at 3 and 6), alpha / beta (the unstaged stores), and one
+# round of tiles on the CUs exactly full.
+HALF = [(1000, 8192, 128), (1024, 8192, 256), (900, 8208, 384), (1000, 8192, 640),
+        (2048, 4096, 768), (1990, 4080, 896)]
+
+
+@pytest.mark.parametrize("shape", HALF)
+@pytest.mark.parametrize("bps", [1, 0])
+def test_half_tile(dev, shape, bps):
+    M, N, K = shape
+    run(dev, M, N, K, 8, bps, seed=K)
+    if K % 256 == 0:
+        run(dev, M, N, 2 * K, 4, bps, seed=K)
+
+
+def test_half_tile_alpha_beta(dev):
+    run(dev, 1000, 8192, 512, 8, 1, alpha=-1.5, beta=0.25, pad_d=12, seed=3)
+
+
+@pytest.mark.parametrize("elem", [8, 4])
+def test_more_tiles_than_cus(dev, elem):
+    """Past one round of 128x256 tiles: the entry's own kernel, ragged."""
+    run(dev, 2100, 4368, 512, elem, 1, seed=elem)
+    run(dev, 2100, 4368, 256, elem, 0, seed=elem + 1)
