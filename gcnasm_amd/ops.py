@@ -125,10 +125,14 @@ class MxOperand:
         self.codes, self.scales, self.rows, self.K = codes, scales, rows, K
 
 
-def _prepare_a(x, sh, elem, scale_rule, stream):
-    M, K = _rows(x)
-    codes = torch.empty((sh.a_rows_pad(), sh.Kp()), dtype=torch.uint8, device=x.device)
-    ss = torch.empty((sh.scale_a_rows() * sh.scale_cols(),), dtype=torch.uint8, device=x.device)
+def _prepare_a(x, elem_bits, elem, scale_rule, stream):
+    M, K = x.shape
+    if M <= 0 or K <= 0:
+        Shape(M, 1, K, elem_bits)  # raises
+    _rows(x)
+    pad = (M + 255) // 256 * 256
+    codes = torch.empty((pad, K * elem_bits // 8), dtype=torch.uint8, device=x.device)
+    ss = torch.empty((pad * ((K // 32 + 7) // 8 * 8),), dtype=torch.uint8, device=x.device)
     check(lib().ga_prepare_mx_a(x.data_ptr(), _in_dtype(x), M, K, x.stride(0), elem,
                                 codes.data_ptr(), ss.data_ptr(), scale_rule,
                                 _stream_handle(stream)))
@@ -137,8 +141,7 @@ def _prepare_a(x, sh, elem, scale_rule, stream):
 
 def prepare_mx_a(x, scale_rule=_lib.GA_MX_SCALE_FLOOR_448, stream=None):
     """Activation [M, K] -> MxOperand (A rows zero-padded to 256)."""
-    M, K = x.shape
-    return _prepare_a(x, Shape(M, 1, K), 0, scale_rule, stream)
+    return _prepare_a(x, 8, 0, scale_rule, stream)
 
 
 def prepare_mx_b(w, scale_rule=_lib.GA_MX_SCALE_FLOOR_448, bpreshuffle=True, stream=None):
@@ -153,8 +156,7 @@ def prepare_mx_b(w, scale_rule=_lib.GA_MX_SCALE_FLOOR_448, bpreshuffle=True, str
 
 def prepare_mx4_a(x, scale_rule=_lib.GA_MX_SCALE_FLOOR_448, stream=None):
     """Activation [M, K] -> MXFP4 MxOperand: packed e2m1 [round_up(M, 256), K/2]."""
-    M, K = x.shape
-    return _prepare_a(x, Shape(M, 1, K, elem_bits=4), 2, scale_rule, stream)
+    return _prepare_a(x, 4, 2, scale_rule, stream)
 
 
 def prepare_mx4_b(w, scale_rule=_lib.GA_MX_SCALE_FLOOR_448, bpreshuffle=True, stream=None):
@@ -172,9 +174,8 @@ def mxfp4_gemm(a, b, bpreshuffle=True, log2_k_split=0, out=None, num_cu=0, works
     """D [M, N] bf16 = A * B^T for MXFP4 operands (prepare_mx4_a/b) through the
     MXFP4 manifest. Returns (D, registry index, launch desc)."""
     M, N, K = a.rows, b.rows, a.K
-    sh = Shape(M, N, K, elem_bits=4)
     if out is None:
-        out = torch.empty((sh.d_rows_pad(), N), dtype=torch.bfloat16, device=a.codes.device)
+        out = torch.empty(((M + 31) // 32 * 32, N), dtype=torch.bfloat16, device=a.codes.device)
     chosen = ctypes.c_int(-1)
     ld = _lib.LaunchDesc()
     ws_ptr, ws_bytes = None, 0
@@ -192,9 +193,8 @@ def mxfp8_gemm(a, b, bpreshuffle=True, log2_k_split=0, out=None, num_cu=0, works
     """D [M, N] bf16 = A * B^T through the heuristic-chosen compiled kernel.
     Returns (D, kernel index, launch desc)."""
     M, N, K = a.rows, b.rows, a.K
-    sh = Shape(M, N, K)
     if out is None:
-        out = torch.empty((sh.d_rows_pad(), N), dtype=torch.bfloat16, device=a.codes.device)
+        out = torch.empty(((M + 31) // 32 * 32, N), dtype=torch.bfloat16, device=a.codes.device)
     chosen = ctypes.c_int(-1)
     ld = _lib.LaunchDesc()
     ws_ptr, ws_bytes = None, 0
