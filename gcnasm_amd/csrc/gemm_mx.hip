@@ -961,7 +961,7 @@ namespace ga {
 // choice is the same for every entry of an element width (and for either B
 // layout and every 8-bit format), so the output does not depend on the tile a
 // caller names; the K-split kernel's sums are cut in K, the others' not.
-enum MxRoute { MX_ROUTE_OWN, MX_ROUTE_KSPLIT, MX_ROUTE_HALF };
+enum MxRoute { MX_ROUTE_OWN, MX_ROUTE_KSPLIT, MX_ROUTE_QUARTER, MX_ROUTE_HALF };
 
 static MxRoute mx_route(const ga_f4gemm_kargs& a, bool fp4, int gdz, int num_cu)
 {
@@ -979,20 +979,30 @@ static MxRoute mx_route(const ga_f4gemm_kargs& a, bool fp4, int gdz, int num_cu)
         return M > 16 && (gdz == 2 || gdz == 4 || gdz == 8) && mb <= 96 ? MX_ROUTE_KSPLIT
                                                                        : MX_ROUTE_OWN;
     }
-    // More rows: while the 128x256 tiles fit on the CUs in one round, they (256
-    // tiles of 256x256 would be at most half a round) or the K-split kernel, by
+    // More rows: while the 128x256 tiles fit on the CUs in one round (the 256x256
+    // tiles would be at most half a round), the largest parallelism that still
+    // is one round, 128x128 or 128x256 tiles, or the K-split kernel, by
     // estimated time. A tile's time is a start, and per K step a little more the
-    // more CUs compete for L2 and power (MXFP8, 64 steps: 44 us with 32 tiles,
-    // 45 with 128, 55 with 192, 60 with 256; MXFP4, 32 steps: 31 with 32, 38
-    // with 256). With more tiles the entry's own kernel, mostly 256x256, is the
-    // faster one (1536x8192x8192: 88 us against 111).
-    const long long tiles = (M + 127) / 128 * ((N + 255) / 256);
-    if (gdz != 1 || tiles > num_cu)
+    // more CUs compete for L2 and power (64 MXFP8 / 32 MXFP4 steps, 128x128:
+    // 36 / 24 us with 64 tiles, 39 / 26 with 256; 128x256: 45 / 31 with 32, 60 /
+    // 38 with 256; 512x8192x8192 as 256 tiles of 128x128 38.9 us, as 128 of
+    // 128x256 53.0, K-split 55.5). With more tiles of 128x256 the entry's own
+    // kernel, mostly 256x256, is the faster one (1536x8192x8192: 88 us against
+    // 111), and two rounds of 128x128 lose to one of 128x256 (1000x8192x8192
+    // 77.6 against 59.8).
+    const long long rows = (M + 127) / 128;
+    const long long halves = rows * ((N + 255) / 256), quarters = rows * ((N + 127) / 128);
+    if (gdz != 1 || halves > num_cu)
         return MX_ROUTE_OWN;
-    const float frac = (float)tiles / (float)num_cu;
+    const bool one = quarters <= num_cu;
+    const float frac = (float)(one ? quarters : halves) / (float)num_cu;
     const float steps = (float)(K / (fp4 ? 256 : 128));
-    const float half_us = 6.0f + steps * (fp4 ? 0.80f + 0.22f * frac : 0.62f + 0.25f * frac);
-    return mx_ksplit_estimate_us(a, fp4, num_cu) < half_us ? MX_ROUTE_KSPLIT : MX_ROUTE_HALF;
+    const float tile_us =
+        one ? (fp4 ? 7.5f : 6.3f) + steps * (fp4 ? 0.52f + 0.06f * frac : 0.47f + 0.04f * frac)
+            : 6.0f + steps * (fp4 ? 0.80f + 0.22f * frac : 0.62f + 0.25f * frac);
+    if (mx_ksplit_estimate_us(a, fp4, num_cu) < tile_us)
+        return MX_ROUTE_KSPLIT;
+    return one ? MX_ROUTE_QUARTER : MX_ROUTE_HALF;
 }
 
 // ga_kernel_launch with the split-K workspace given either as a buffer
@@ -1144,8 +1154,9 @@ static ga_status kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, in
         GA_HIP_CHECK(hipGetLastError());
         return GA_OK;
     }
-    if (route == MX_ROUTE_HALF)
-        launch_mx_pp_half(*args, ws, nullptr, gdz, bps, fp4, fmt, s);
+    if (route == MX_ROUTE_HALF || route == MX_ROUTE_QUARTER)
+        launch_mx_pp_half(*args, ws, nullptr, gdz, bps, fp4, fmt, route == MX_ROUTE_HALF ? 2 : 1,
+                          s);
     else if (split_groups > 0)
         launch_mx_decode_split(*args, gdz, phys, split_groups, bps, fp4, fmt, ws, wsh, num_cu, s);
     else if (fmt != 0)

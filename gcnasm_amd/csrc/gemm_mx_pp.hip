@@ -214,7 +214,7 @@ __device__ __forceinline__ PpArgs uni_args(const ga_f4gemm_kargs& args)
 // as an MXFP8 step, so copies, LDS layout and fragment reads are shared; a
 // step reads one whole shuffled scale dword per 32-row block.
 // Two quadrants with shared A fragments: acc0 += A x B0, acc1 += A x B1
-// (16 MFMAs at raised issue priority).
+// (16 MFMAs at raised issue priority). TWO false: the first alone.
 // MXFP8 with whole scale dwords: SB = 2 * (128-K half) selects the step's
 // bytes in the operand (0 when the step's two bytes were read into 0-15).
 // Issue order: A tiles 0-3 in the first quadrant and 3-0 in the second, B
@@ -222,7 +222,7 @@ __device__ __forceinline__ PpArgs uni_args(const ga_f4gemm_kargs& args)
 // (the MFMA pipe's power falls with the operand bits that change: MXFP8
 // 8192^3 375.3 -> 370.6 us, 4096^3 55.0 -> 54.3 us on one box, best of
 // 5 x 100 calls; each accumulator's K order, and so the output, unchanged).
-template <bool FP4, int F, int SB = 0>
+template <bool FP4, int F, int SB = 0, bool TWO = true>
 __device__ __forceinline__ void mma_two(v4f (&acc0)[4][2], v4f (&acc1)[4][2], const v8i (&a)[4],
                                         const v8i (&b0)[2], const v8i (&b1)[2],
                                         const uint32_t (&sa)[2], uint32_t sb0, uint32_t sb1)
@@ -247,7 +247,8 @@ __device__ __forceinline__ void mma_two(v4f (&acc0)[4][2], v4f (&acc1)[4][2], co
         });
     };
     quadrant(acc0, b0, sb0, std::integral_constant<int, 0>{});
-    quadrant(acc1, b1, sb1, std::integral_constant<int, 1>{});
+    if constexpr (TWO)
+        quadrant(acc1, b1, sb1, std::integral_constant<int, 1>{});
     __builtin_amdgcn_s_setprio(0);
 }
 
@@ -588,56 +589,67 @@ void mx_pp_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
     wait_vmcnt<0>(); // copies of steps past the last slice land before exit
 }
 
-// ---- 128x256 tile ------------------------------------------------------------------
-// The same pipeline for half the rows: two groups of four waves one barrier
-// apart, group g on rows 64g .. 64g + 63, SIMD s on columns 32s .. 32s + 31 of
-// both 128-column halves. A K step is one memory half (all its copies and
-// fragment reads) and one MFMA half of 16 MFMAs per group; three 48 KB slots,
-// a step's copies issued two steps ahead into the slot both groups have left.
-// For problems whose 256x256 tiles leave much of the last round idle: a step
-// takes about half as long and moves 48 KB instead of 64, so full rounds stay
-// with the larger tile.
-constexpr int kHSlot = 3 * kHalf; // A, B columns 0-127, B columns 128-255
-constexpr int kHScaleSlot = 12 * 256; // 4 A + 8 B shuffled 32-row scale blocks
-constexpr int kHScaleBase = 3 * kHSlot;
-constexpr int kHLds = kHScaleBase + 3 * kHScaleSlot;
-static_assert(kHLds <= 160 * 1024 && 128 * kStagePitch <= kHLds, "LDS budget");
+// ---- 128x256 and 128x128 tiles -------------------------------------------------------
+// The same pipeline for half the rows and NB = 2 or 1 halves of 128 columns: two
+// groups of four waves one barrier apart, group g on rows 64g .. 64g + 63, SIMD
+// s on columns 32s .. 32s + 31 of each half. A K step is one memory half (all
+// its copies and fragment reads) and one MFMA half of 8 NB MFMAs per group;
+// three 48 KB or four 32 KB slots, a step's copies issued two or three steps
+// ahead into the slot both groups have left. For problems whose 256x256 tiles
+// leave much of the last round idle: a step takes about half (a third) as long
+// and moves 48 (32) KB instead of 64, so full rounds stay with the larger tile.
+template <int NB, bool FP4>
+struct HalfCfg {
+    static constexpr int kSlot = (1 + NB) * kHalf; // A, then the B halves
+    static constexpr int NS = NB == 2 ? 3 : 4;
+    static constexpr int kScaleSlot = (4 + 4 * NB) * 256; // shuffled 32-row scale blocks
+    static constexpr int kScaleBase = NS * kSlot;
+    static constexpr int kRing = FP4 ? NS : 3; // scale slots: steps, or pairs of steps
+    static constexpr int kLds = kScaleBase + kRing * kScaleSlot;
+    static constexpr int kCopies = 2 + 2 * NB + (FP4 ? 2 : 1); // per wave and step
+    static_assert(kLds <= 160 * 1024 && 128 * kStagePitch <= kLds, "LDS budget");
+};
 constexpr int kHGroupM = 8;
 
-// Copies (6 per wave) of K step t into slot `slot`.
+// Operand copies of K step t into slot `slot`.
+template <int NB>
 __device__ __forceinline__ void issue_h(const PpLoad& L, char* smem, int t, int slot, int wave)
 {
-    char* dst = smem + slot * kHSlot + wave * 1024;
+    char* dst = smem + slot * (1 + NB) * kHalf + wave * 1024;
     const uint32_t oa = (uint32_t)t * 128, ob = (uint32_t)t * L.b_kstep;
     lds_load16(L.ra, (lds_void*)dst, L.va + uni(oa), 0);
     lds_load16(L.ra, (lds_void*)(dst + 8192), L.va + uni(oa + L.a_hstep), 0);
 #pragma unroll
-    for (int c = 0; c < 4; c++)
+    for (int c = 0; c < 2 * NB; c++)
         lds_load16(L.rb, (lds_void*)(dst + kHalf + c * 8192), L.vb + uni(ob + c * L.b_hstep), 0);
 }
 
 // Half `half` (0: A rows, 1: B rows) of the scales of 256-K block `pair` into
-// ring slot `ring`: wave w copies block w of the 8 of B, block w % 4 of A.
+// ring slot `ring`: wave w copies block w (mod 4 where there are 4).
+template <int NB, bool FP4>
 __device__ __forceinline__ void issue_hs(const PpLoad& L, char* smem, int pair, int half, int ring,
                                          int wave)
 {
-    char* dst = smem + kHScaleBase + ring * kHScaleSlot + (half ? 4 + wave : wave & 3) * 256;
+    using H = HalfCfg<NB, FP4>;
+    char* dst = smem + H::kScaleBase + ring * H::kScaleSlot +
+                (half ? 4 + (NB == 2 ? wave : wave & 3) : wave & 3) * 256;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(half ? L.rsb : L.rsa, (lds_void*)dst, 4,
                                              (half ? L.vsb : L.vsa) + uni((uint32_t)pair * 256), 0,
                                              0, 0);
 }
 
-template <bool BPS, bool FP4, int F>
+template <int NB, bool BPS, bool FP4, int F>
 __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restrict__ ws,
                                              char* smem, int tile_m, int tile_n)
 {
+    using H = HalfCfg<NB, FP4>;
     constexpr int kEPB = FP4 ? 2 : 1;
     constexpr int kStepK = 128 * kEPB;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2, simd = wave & 3;
     const int M = (int)args.M, N = (int)args.N, K = (int)args.K;
-    const int m0 = tile_m * 128, n0 = tile_n * 256;
+    const int m0 = tile_m * 128, n0 = tile_n * 128 * NB;
 
     const int z = blockIdx.z, gdz = gridDim.z;
     int kpt = K;
@@ -648,9 +660,9 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
     const int nsteps = (ke - kb) / kStepK;
     const int kbb = kb / kEPB;
 
-    v4f acc[2][4][2];
+    v4f acc[2][4][2]; // [1] is unused with one half
 #pragma unroll
-    for (int q = 0; q < 2; q++)
+    for (int q = 0; q < NB; q++)
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -691,8 +703,8 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
             L.rsb = make_rsrc(args.ptr_ScaleB, (uint32_t)((N + 31) / 32 * 32) * snb);
             L.vsa = ((uint32_t)(m0 / 32 + (wave & 3)) * (sna / 8) + (uint32_t)(kb / 256)) * 256 +
                     lane * 4;
-            L.vsb = ((uint32_t)(n0 / 32 + wave) * (snb / 8) + (uint32_t)(kb / 256)) * 256 +
-                    lane * 4;
+            L.vsb = ((uint32_t)(n0 / 32 + (NB == 2 ? wave : wave & 3)) * (snb / 8) +
+                     (uint32_t)(kb / 256)) * 256 + lane * 4;
         }
 
         ReadBase rb;
@@ -708,89 +720,96 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
                 rb.b0 = smem + kHalf + simd * 32 * 128 + o;
                 rb.b1 = smem + kHalf + simd * 32 * 128 + o64;
             }
-            rb.sa = smem + kHScaleBase + grp * 2 * 256 + lane * 4;
-            rb.sb = smem + kHScaleBase + (4 + simd) * 256 + lane * 4;
+            rb.sa = smem + H::kScaleBase + grp * 2 * 256 + lane * 4;
+            rb.sb = smem + H::kScaleBase + (4 + simd) * 256 + lane * 4;
         }
 
         v8i fa[4], fb0[2], fb1[2];
         uint32_t sa[2], sb0, sb1;
-        // copies per step: 6 operand, 1 scale (MXFP8: half of a pair of steps)
-        // or 2 (MXFP4: a step is 256 K)
-        constexpr int kC = FP4 ? 8 : 7;
+        constexpr int NS = H::NS, kC = H::kCopies;
+        // what follows the copies of the first step that the first memory half
+        // reads: NS - 2 whole steps
         if constexpr (FP4) {
-            issue_h(L, smem, 0, 0, wave);
-            issue_hs(L, smem, 0, 0, 0, wave);
-            issue_hs(L, smem, 0, 1, 0, wave);
-            issue_h(L, smem, 1, 1, wave);
-            issue_hs(L, smem, 1, 0, 1, wave);
-            issue_hs(L, smem, 1, 1, 1, wave);
+            static_for<NS - 1>([&](auto J) {
+                constexpr int j = decltype(J)::value;
+                issue_h<NB>(L, smem, j, j, wave);
+                issue_hs<NB, FP4>(L, smem, j, 0, j, wave);
+                issue_hs<NB, FP4>(L, smem, j, 1, j, wave);
+            });
         } else {
-            issue_hs(L, smem, 0, 0, 0, wave);
-            issue_hs(L, smem, 0, 1, 0, wave);
-            issue_h(L, smem, 0, 0, wave);
-            issue_hs(L, smem, 1, 0, 1, wave);
-            issue_h(L, smem, 1, 1, wave);
-            issue_hs(L, smem, 1, 1, 1, wave);
+            // pairs 0 and, half by half with steps 0 and 1, pair 1
+            issue_hs<NB, FP4>(L, smem, 0, 0, 0, wave);
+            issue_hs<NB, FP4>(L, smem, 0, 1, 0, wave);
+            static_for<NS - 1>([&](auto J) {
+                constexpr int j = decltype(J)::value;
+                issue_h<NB>(L, smem, j, j, wave);
+                issue_hs<NB, FP4>(L, smem, 1, j & 1, 1, wave);
+            });
         }
-        part_sync<kC>();
+        part_sync<kC*(NS - 2)>();
         if (grp == 1)
             slot_sync(); // second group runs one barrier behind
 
-        // Step s in slot S = s % 3: copies of step s + 2 into the slot of step
-        // s - 1, whose last reads (the second group's) ended one barrier ago.
-        // Waiting for all but the newest kC copies after the memory half
-        // retires step s + 1's, which either group reads two barriers on at
-        // the earliest. MXFP8 scales: half P of pair (s >> 1) + 2 (as in the
-        // 256x256 tile), read whole in even steps.
+        // Step s in slot S = s % NS: copies of step s + NS - 1 into the slot of
+        // step s - 1, whose last reads (the second group's) ended one barrier
+        // ago. Waiting for all but the newest NS - 2 steps' copies after the
+        // memory half retires step s + 1's, which either group reads two
+        // barriers on at the earliest. MXFP8 scales: half P of pair
+        // (s >> 1) + 2 (as in the 256x256 tile), read whole in even steps; with
+        // four slots they land one barrier before their first read.
         int r0 = 0; // scale ring slot of step s (MXFP8: of pair s >> 1)
         auto step = [&](int s, auto SC, auto PC) {
             constexpr int S = decltype(SC)::value, P = decltype(PC)::value;
-            const int r2 = r0 == 0 ? 2 : r0 - 1; // (r0 + 2) % 3
-            issue_h(L, smem, s + 2, (S + 2) % 3, wave);
+            const int r2 = r0 == 0 ? H::kRing - 1 : r0 - 1; // of the step (pair) before
+            issue_h<NB>(L, smem, s + NS - 1, (S + NS - 1) % NS, wave);
             if constexpr (FP4) {
-                issue_hs(L, smem, s + 2, 0, r2, wave);
-                issue_hs(L, smem, s + 2, 1, r2, wave);
+                issue_hs<NB, FP4>(L, smem, s + NS - 1, 0, r2, wave);
+                issue_hs<NB, FP4>(L, smem, s + NS - 1, 1, r2, wave);
             } else {
-                issue_hs(L, smem, (s >> 1) + 2, P, r2, wave);
+                issue_hs<NB, FP4>(L, smem, (s >> 1) + 2, P, r2, wave);
             }
             if constexpr (FP4 || P == 0) {
-                const char* pa = rb.sa + r0 * kHScaleSlot;
-                const char* pb = rb.sb + r0 * kHScaleSlot;
+                const char* pa = rb.sa + r0 * H::kScaleSlot;
+                const char* pb = rb.sb + r0 * H::kScaleSlot;
                 sa[0] = *(const uint32_t*)pa;
                 sa[1] = *(const uint32_t*)(pa + 256);
                 sb0 = *(const uint32_t*)pb;
-                sb1 = *(const uint32_t*)(pb + 4 * 256);
+                if constexpr (NB == 2)
+                    sb1 = *(const uint32_t*)(pb + 4 * 256);
             }
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                fa[i] = lds_frag(rb.a0 + S * kHSlot + i * 2048, rb.a1 + S * kHSlot + i * 2048);
+                fa[i] = lds_frag(rb.a0 + S * H::kSlot + i * 2048, rb.a1 + S * H::kSlot + i * 2048);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int t = 0; t < 2; t++)
-                fb0[t] = lds_frag(rb.b0 + S * kHSlot + t * 2048, rb.b1 + S * kHSlot + t * 2048);
+                fb0[t] = lds_frag(rb.b0 + S * H::kSlot + t * 2048, rb.b1 + S * H::kSlot + t * 2048);
+            if constexpr (NB == 2) {
 #pragma unroll
-            for (int t = 0; t < 2; t++)
-                fb1[t] = lds_frag(rb.b0 + S * kHSlot + kHalf + t * 2048,
-                                  rb.b1 + S * kHSlot + kHalf + t * 2048);
-            part_sync<kC>();
-            mma_two<FP4, F, FP4 ? 0 : 2 * P>(acc[0], acc[1], fa, fb0, fb1, sa, sb0, sb1);
-            part_sync<kC>();
+                for (int t = 0; t < 2; t++)
+                    fb1[t] = lds_frag(rb.b0 + S * H::kSlot + kHalf + t * 2048,
+                                      rb.b1 + S * H::kSlot + kHalf + t * 2048);
+            }
+            part_sync<kC*(NS - 2)>();
+            mma_two<FP4, F, FP4 ? 0 : 2 * P, NB == 2>(acc[0], acc[1], fa, fb0, fb1, sa, sb0, sb1);
+            part_sync<kC*(NS - 2)>();
             if constexpr (FP4 || P == 1)
-                r0 = r0 == 2 ? 0 : r0 + 1;
+                r0 = r0 == H::kRing - 1 ? 0 : r0 + 1;
         };
-        // slot and parity are compile-time: six steps per iteration
+        // slot and parity are compile-time: six (four) steps per iteration
+        constexpr int U = NS == 3 ? 6 : 4;
         int s = 0;
-        for (; s + 6 <= nsteps; s += 6)
-            static_for<6>([&](auto J) {
+        for (; s + U <= nsteps; s += U)
+            static_for<U>([&](auto J) {
                 constexpr int j = decltype(J)::value;
-                step(s + j, std::integral_constant<int, j % 3>{},
+                step(s + j, std::integral_constant<int, j % NS>{},
                      std::integral_constant<int, j % 2>{});
             });
-        static_for<5>([&](auto J) {
+        static_for<U - 1>([&](auto J) {
             constexpr int j = decltype(J)::value;
             if (s + j < nsteps)
-                step(s + j, std::integral_constant<int, j % 3>{},
+                step(s + j, std::integral_constant<int, j % NS>{},
                      std::integral_constant<int, j % 2>{});
         });
         if (grp == 0)
@@ -800,13 +819,13 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
     const int ldd = (int)args.stride_C0;
     const float alpha = args.alpha, beta = args.beta;
     const bool use_c = beta != 0.0f && args.ptr_C != nullptr;
-    const bool staged = gdz == 1 && !use_c && m0 + 128 <= M && n0 + 256 <= N && (ldd & 7) == 0 &&
-                        ((uintptr_t)args.ptr_D & 15) == 0;
+    const bool staged = gdz == 1 && !use_c && m0 + 128 <= M && n0 + 128 * NB <= N &&
+                        (ldd & 7) == 0 && ((uintptr_t)args.ptr_D & 15) == 0;
     if (staged) {
         wait_vmcnt<0>();
         wait_lds_barrier();
 #pragma unroll
-        for (int q = 0; q < 2; q++)
+        for (int q = 0; q < NB; q++)
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -821,10 +840,11 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
                 }
         barrier_lds();
         uint16_t* dst = (uint16_t*)args.ptr_D + (size_t)m0 * ldd + n0;
-        const int col = (lane & 31) * 8;
+        constexpr int kLanes = 16 * NB; // 16-byte stores to a row
+        const int col = (lane % kLanes) * 8;
 #pragma unroll
-        for (int it = 0; it < 8; it++) {
-            const int row = wave * 16 + it * 2 + (lane >> 5);
+        for (int it = 0; it < 16 * kLanes / 64; it++) {
+            const int row = wave * 16 + it * (64 / kLanes) + lane / kLanes;
             *(v4i*)(dst + (size_t)row * ldd + col) =
                 *(const v4i*)(smem + row * kStagePitch + col * 2);
         }
@@ -832,7 +852,7 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
         return;
     }
 #pragma unroll
-    for (int q = 0; q < 2; q++)
+    for (int q = 0; q < NB; q++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int m = m0 + grp * 64 + i * 16 + (lane & 15);
@@ -864,12 +884,12 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
         }
 }
 
-template <bool BPS, bool FP4, int F = 0>
+template <int NB, bool BPS, bool FP4, int F = 0>
 __global__ __attribute__((amdgpu_flat_work_group_size(kNT, kNT), amdgpu_waves_per_eu(2, 2)))
 void mx_pp_half_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
                        const ga_splitk_ws_handle* __restrict__ wsh, int tiles_x, int tiles_y)
 {
-    __shared__ __attribute__((aligned(1024))) char smem[kHLds];
+    __shared__ __attribute__((aligned(1024))) char smem[HalfCfg<NB, FP4>::kLds];
     if (wsh && !(ws = resolve_ws(wsh, gridDim.z, args.M, args.N)))
         return; // workspace slot shorter than the split-K layout: write nothing
     const PpArgs a = uni_args(args);
@@ -877,7 +897,7 @@ void mx_pp_half_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
     for (int lin = blockIdx.x; lin < ntiles; lin += gridDim.x) {
         int tile_m, tile_n;
         map_tile_lin(lin, tiles_x, tiles_y, kHGroupM, tile_m, tile_n);
-        pp_half_tile<BPS, FP4, F>(a, ws, smem, tile_m, tile_n);
+        pp_half_tile<NB, BPS, FP4, F>(a, ws, smem, tile_m, tile_n);
     }
     wait_vmcnt<0>(); // copies of steps past the last slice land before exit
 }
@@ -957,34 +977,41 @@ void launch_mx_pp_fmt(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws
 
 namespace {
 
-template <bool BPS, bool FP4, int F>
-void launch_half(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh, int gdz,
-                 hipStream_t stream)
+template <int NB, bool BPS, bool FP4, int F>
+void launch_half_n(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh, int gdz,
+                   hipStream_t stream)
 {
-    const int gdx = ((int)args.N + 255) / 256, gdy = ((int)args.M + 127) / 128;
-    hipLaunchKernelGGL((mx_pp_half_kernel<BPS, FP4, F>), dim3(pp_grid(gdx * gdy), 1, gdz),
+    const int gdx = ((int)args.N + 128 * NB - 1) / (128 * NB), gdy = ((int)args.M + 127) / 128;
+    hipLaunchKernelGGL((mx_pp_half_kernel<NB, BPS, FP4, F>), dim3(pp_grid(gdx * gdy), 1, gdz),
                        dim3(kNT), 0, stream, args, ws, wsh, gdx, gdy);
+}
+
+template <bool FP4, int F>
+void launch_half(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh, int gdz,
+                 bool bps, int halves, hipStream_t stream)
+{
+    if (halves == 2)
+        bps ? launch_half_n<2, true, FP4, F>(args, ws, wsh, gdz, stream)
+            : launch_half_n<2, false, FP4, F>(args, ws, wsh, gdz, stream);
+    else
+        bps ? launch_half_n<1, true, FP4, F>(args, ws, wsh, gdz, stream)
+            : launch_half_n<1, false, FP4, F>(args, ws, wsh, gdz, stream);
 }
 
 } // namespace
 
 void launch_mx_pp_half(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh,
-                       int gdz, bool bps, bool fp4, int fmt, hipStream_t stream)
+                       int gdz, bool bps, bool fp4, int fmt, int halves, hipStream_t stream)
 {
     if (fp4) {
-        bps ? launch_half<true, true, 0>(args, ws, wsh, gdz, stream)
-            : launch_half<false, true, 0>(args, ws, wsh, gdz, stream);
+        launch_half<true, 0>(args, ws, wsh, gdz, bps, halves, stream);
         return;
     }
     switch (fmt) {
-    case 1: bps ? launch_half<true, false, 1>(args, ws, wsh, gdz, stream)
-                : launch_half<false, false, 1>(args, ws, wsh, gdz, stream); break;
-    case 2: bps ? launch_half<true, false, 2>(args, ws, wsh, gdz, stream)
-                : launch_half<false, false, 2>(args, ws, wsh, gdz, stream); break;
-    case 3: bps ? launch_half<true, false, 3>(args, ws, wsh, gdz, stream)
-                : launch_half<false, false, 3>(args, ws, wsh, gdz, stream); break;
-    default: bps ? launch_half<true, false, 0>(args, ws, wsh, gdz, stream)
-                 : launch_half<false, false, 0>(args, ws, wsh, gdz, stream); break;
+    case 1: launch_half<false, 1>(args, ws, wsh, gdz, bps, halves, stream); break;
+    case 2: launch_half<false, 2>(args, ws, wsh, gdz, bps, halves, stream); break;
+    case 3: launch_half<false, 3>(args, ws, wsh, gdz, bps, halves, stream); break;
+    default: launch_half<false, 0>(args, ws, wsh, gdz, bps, halves, stream); break;
     }
 }
 

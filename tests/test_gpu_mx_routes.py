@@ -1,7 +1,7 @@
 """The MX kernels that a launch's shape picks (the K-split kernel, the 128x256
-tile, the entry's own kernel), each at the edges of its tiles and of the rule
-that picks it, against the CPU oracle: formats, B layouts, splits, alpha and
-beta, a strided D."""
+and 128x128 tiles, the entry's own kernel), each at the edges of its tiles and
+of the rule that picks it, against the CPU oracle: formats, B layouts, splits,
+alpha and beta, a strided D."""
 import numpy as np
 import pytest
 import torch
@@ -115,6 +115,26 @@ def test_half_tile(dev, shape, bps):
     run(dev, M, N, K, 8, bps, seed=K)
     if K % 256 == 0:
         run(dev, M, N, 2 * K, 4, bps, seed=K)
+
+
+# The 128x128 tile where its tiles fill one round: the same edges, its slots and
+# scale ring wrapping at 4 and 6 steps, and the unstaged stores.
+QUARTER = [(1000, 4096, 384), (2048, 2048, 128), (1990, 2064, 512), (512, 8192, 640),
+           (500, 8192, 768), (1024, 4096, 896), (2048, 2048, 1152)]
+
+
+@pytest.mark.parametrize("shape", QUARTER)
+@pytest.mark.parametrize("bps", [1, 0])
+def test_quarter_tile(dev, shape, bps):
+    M, N, K = shape
+    run(dev, M, N, K, 8, bps, seed=K)
+    run(dev, M, N, 2 * K, 4, bps, seed=K)
+
+
+def test_quarter_tile_formats_alpha_beta(dev):
+    run(dev, 1000, 4096, 2048, 8, 1, 1, 0, alpha=-1.5, beta=0.25, pad_d=12, seed=5)
+    run(dev, 1000, 4096, 2048, 8, 0, 0, 1, pad_d=4, seed=6)
+    run(dev, 1000, 4096, 2048, 8, 1, 1, 1, seed=7)
 
 
 def test_half_tile_alpha_beta(dev):
