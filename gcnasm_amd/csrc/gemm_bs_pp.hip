@@ -211,7 +211,7 @@ void bs_pp_kernel(ga_opus_gemm_kargs ka)
         apply_scales<MODE>(svn, acc[3], p);
     } else {
         auto group = [&](int s, auto SLOT) {
-            constexpr int slot = decltype(SLOT)::value;
+            const int slot = SLOT;
             const int r0 = s & 3, r2 = (s + 2) & 3, rprev = (s - 1) & 3;
             // phase 1 (folds in quadrant 11 of the previous group)
             BS_MEM_SLOT(1, 1, rprev, issue_a(L, smem, 1, s + 1, wave), read_a<0>(rb, slot, fa),
@@ -238,13 +238,20 @@ void bs_pp_kernel(ga_opus_gemm_kargs ka)
             mma_quadrant<MODE, true>(acc[3], p, fa, fb1, acc[2], sv);
             slot_sync();
         };
-        int s = 0;
-        for (; s + 1 < nsteps; s += 2) {
-            group(s, std::integral_constant<int, 0>{});
-            group(s + 1, std::integral_constant<int, 1>{});
+        if constexpr (MODE == PS_GROUP1) {
+            // one group per iteration: two need more registers than there are
+            // (832 spilled: 1536x8192x8192, bf16 C, 1457 us against 126 now)
+            for (int s = 0; s < nsteps; s++)
+                group(s, s & 1);
+        } else {
+            int s = 0;
+            for (; s + 1 < nsteps; s += 2) {
+                group(s, std::integral_constant<int, 0>{});
+                group(s + 1, std::integral_constant<int, 1>{});
+            }
+            if (s < nsteps)
+                group(s, std::integral_constant<int, 0>{});
         }
-        if (s < nsteps)
-            group(s, std::integral_constant<int, 0>{});
         if (grp == 0)
             slot_sync(); // matches the second group's extra barrier
         const ScaleVals last = read_scales<MODE, 1, 1>(rb, (nsteps - 1) & 3);
