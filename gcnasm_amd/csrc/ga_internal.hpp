@@ -85,7 +85,10 @@ ga_status device_cu_count(int* num_cu);
 // 256x256 eight-wave fp32-scaled FP8 GEMM (gemm_bs_pp.hip); mode 0 = block
 // scale GROUP_N 128, 1 = GROUP_N 1, 2 = per-tensor.
 void launch_bs_pp(const ga_opus_gemm_kargs& ka, int mode, int out_dtype, hipStream_t stream);
-// The same kernel's stream-K form (batch 1): workgroups it would use on
+// 128x256 (halves 2) and 128x128 (1) tiles of the same GEMMs.
+void launch_bs_half(const ga_opus_gemm_kargs& ka, int mode, int out_dtype, int halves,
+                    hipStream_t stream);
+// The 256x256 kernel's stream-K form (batch 1): workgroups it would use on
 // num_cu CUs (0: the whole-tile form is the better one), its workspace
 // (per-tile counters, zero between calls, then 2 * nwg fp32 partial tiles),
 // the counters' share of it, and the launch.

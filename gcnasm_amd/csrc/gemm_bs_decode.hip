@@ -27,7 +27,7 @@
 //  * columns past N and rows past M read as zero (range-checked buffers),
 //    scale indices are clamped, stores are masked.
 // Measured on MI355X (bf16 C, GROUP_N 128), operands loaded into registers or
-// 128x128 / 64x256 tiles -> this kernel: 1x7168x2048 7.7 -> 5.3 us, 16x2112x7168
+// four-wave 128x128 / 64x256 tiles -> this kernel: 1x7168x2048 7.7 -> 5.3 us, 16x2112x7168
 // 12.2 -> 5.9, 32x7168x2048 13.1 -> 5.8, 64x2112x7168 22.3 -> 8.4, 64x24576x1536
 // 15.6 -> 10.8, 128x8192x8192 50.7 -> 17.5, 300x2112x7168 45.1 -> 15.7,
 // 512x4096x4096 28.4 -> 17.5.

@@ -5,7 +5,11 @@
 //   padded + shuffled (f4gemm_ref.hpp:98-130); B optionally preshuffled in
 //   16x16-byte subtiles (f4gemm_ref.hpp:78-96).
 //
-// Kernel design (gfx950, wave64, 256 threads = 4 waves):
+// A launch runs the manifest entry's own kernel or one picked by its shape
+// (mx_route: gemm_mx_ksplit.hip, the 128x256 and 128x128 tiles of
+// gemm_mx_pp.hip, gemm_mx_decode.hip for few rows).
+//
+// Kernel design of this file's tiles (gfx950, wave64, 256 threads = 4 waves):
 //  * block tile BM x BN, K step 128; waves in a WAVES_M x WAVES_N grid, each
 //    owning (BM/WAVES_M) x (BN/WAVES_N) of C as 16x16 MFMA tiles.
 //  * A and B are staged in LDS with buffer_load ... lds (16 B per lane,

@@ -1,4 +1,5 @@
-// gemm_mx_pp.hip -- 256x256 MXFP8 GEMM tile for large M and N (f4gemm ABI).
+// gemm_mx_pp.hip -- eight-wave MXFP8 / MXFP4 GEMM tiles (f4gemm ABI): 256x256
+// for large M and N, and (further down) 128x256 and 128x128.
 //
 // Same contract as the 4-wave kernels of gemm_mx.hip (operands, shuffled
 // scales, optional preshuffled B, split-K into an fp32 workspace); this file

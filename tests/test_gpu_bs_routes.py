@@ -1,6 +1,7 @@
-"""The K-split kernel of the fp32-scaled FP8 GEMMs (few rows): every wave tile
-and slice count its plan picks, at the edges of rows, columns and K, with
-padded strides and batches, against the CPU oracle in the K slices the library
+"""The kernels of the fp32-scaled FP8 GEMMs that a call's shape picks: the K-split
+kernel (few rows; every wave tile and slice count of its plan) and the tiles of
+128x128, 128x256 and 256x256, at the edges of rows, columns and K, with padded
+strides and batches, against the CPU oracle in the K slices the library
 reports."""
 import numpy as np
 import pytest
@@ -43,13 +44,11 @@ def padded(x, ld, dev):
     return torch.from_numpy(out).to(dev)
 
 
-@pytest.mark.parametrize("shape", SHAPES)
-@pytest.mark.parametrize("group_n", [128, 1, 0])
-def test_k_split_kernel(dev, shape, group_n):
+def run(dev, shape, group_n, batch, pad_a, pad_b, pad_c, whole_k=False):
     M, N, K = shape
-    batch, pad_a, pad_b, pad_c = (2, 16, 48, 3) if M <= 129 and N <= 1100 else (1, 0, 32, 4)
     qa, qb, sfa, sfb = problem(batch, M, N, K, group_n or 128, M + N + K)
     gps = opus_gemm.k_slices(M, N, K, batch)
+    assert not whole_k or gps == K // 128
     A, B = padded(qa, K + pad_a, dev), padded(qb, K + pad_b, dev)
     SA, SB = torch.from_numpy(sfa).to(dev), torch.from_numpy(sfb).to(dev)
     rows = np.unique(np.r_[np.arange(min(M, 48)), np.arange(max(0, M - 20), M)])
@@ -72,7 +71,7 @@ def test_k_split_kernel(dev, shape, group_n):
         ka.stride_a_batch, ka.stride_b_batch = M * ka.stride_a, N * ka.stride_b
         ka.stride_c_batch = M * ka.stride_c
         out = _lib.GA_DTYPE_F32 if dtype == torch.float32 else _lib.GA_DTYPE_BF16
-        print("k-split", shape, group_n, dtype, "groups per slice", gps, flush=True)
+        print("fp32 scales", shape, group_n, dtype, "groups per slice", gps, flush=True)
         if group_n:
             opus_gemm.gemm_a8w8_blockscale(ka, out, group_n)
         else:
@@ -85,4 +84,36 @@ def test_k_split_kernel(dev, shape, group_n):
         else:
             ok, st = bf16_compare(got.view(torch.int16).cpu().numpy().view(np.uint16),
                                   oracle.to_bf16_bits(want), absdot)
-        assert_parity(st, "k-split %s g%d %s" % (shape, group_n, dtype))
+        assert_parity(st, "fp32 scales %s g%d %s" % (shape, group_n, dtype))
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("group_n", [128, 1, 0])
+def test_k_split_kernel(dev, shape, group_n):
+    M, N, K = shape
+    run(dev, shape, group_n, *((2, 16, 48, 3) if M <= 129 and N <= 1100 else (1, 0, 32, 4)))
+
+
+# More rows than the K-split kernel takes. 128x128 tiles: whole and ragged, one
+# group to nine (LDS slots wrap at 4, scale slots at 8). 128x256: one to seven
+# (3 and 4), the last round full. 256x256: odd and even numbers of groups.
+QUARTER = [(1100, 2000, 128), (1100, 1024, 256), (1152, 2049, 384), (1026, 128, 512),
+           (2048, 2048, 640), (1280, 770, 1152), (4100, 520, 1024)]
+HALF = [(1100, 6900, 128), (1152, 4096, 256), (2048, 4096, 384), (2000, 3600, 512),
+        (1280, 4098, 640), (1152, 6400, 896)]
+FULL = [(1100, 7700, 128), (2304, 4096, 256), (2100, 4360, 384), (2304, 4100, 640)]
+
+
+@pytest.mark.parametrize("shape", QUARTER + HALF + FULL)
+@pytest.mark.parametrize("group_n", [128, 1, 0])
+def test_tiles(dev, shape, group_n):
+    M, N, K = shape
+    run(dev, shape, group_n, 1, 0, 32 if M % 128 else 0, -N % 4 + 4 if N % 8 else 8, True)
+
+
+@pytest.mark.parametrize("shape", [(1030, 384, 384), (1030, 2100, 384)])
+@pytest.mark.parametrize("group_n", [128, 1, 0])
+def test_tiles_batched_unaligned(dev, shape, group_n):
+    """128x128 and 128x256 tiles, three batches, padded A and B rows, C rows
+    that no 16-byte store fits."""
+    run(dev, shape, group_n, 3, 16, 48, 3, True)
