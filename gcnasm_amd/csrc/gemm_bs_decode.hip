@@ -98,12 +98,13 @@ void bs_decode_kernel(ga_opus_gemm_kargs ka, int nwg, int mblocks, int ks, int g
     if (nsteps > 0) {
         const uint32_t lda = (uint32_t)ka.stride_a, ldb = (uint32_t)ka.stride_b;
         const char* pa = (const char*)ka.ptr_a + (size_t)b * ka.stride_a_batch + (size_t)m0 * lda;
-        const long long abytes = (long long)M * lda;
+        // up to the last row's K: copies past K never leave the operands
+        const long long abytes = (long long)(M - 1) * lda + ka.k;
         const auto ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
         const char* pb = (const char*)ka.ptr_b + (size_t)b * ka.stride_b_batch +
                          (size_t)cg0 * 16 * ldb;
         const long long brows = min(ng_here * 16, N - cg0 * 16);
-        const auto rb = make_rsrc(pb, (uint32_t)min(brows * ldb, 0xFFFFFFF0ll));
+        const auto rb = make_rsrc(pb, (uint32_t)min((brows - 1) * ldb + ka.k, 0xFFFFFFF0ll));
         // copy h (0, 1) of a 16-row block: lane l fetches row 8h + l / 8 from
         // whole 128-byte lines into slot l % 8
         const uint32_t crow = (uint32_t)lane >> 3, cslot = lane & 7;

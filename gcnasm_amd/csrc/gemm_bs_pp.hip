@@ -50,8 +50,9 @@ __device__ __forceinline__ void bs_load_setup(const ga_opus_gemm_kargs& ka, int 
                      (size_t)m0 * ka.stride_a;
     const char* pb = (const char*)ka.ptr_b + (size_t)b * ka.stride_b_batch +
                      (size_t)n0 * ka.stride_b;
-    const long long abytes = (long long)(M - m0) * ka.stride_a;
-    const long long bbytes = (long long)(N - n0) * ka.stride_b;
+    // up to the last row's K bytes: copies past K never leave the operands
+    const long long abytes = (long long)(M - 1 - m0) * ka.stride_a + K;
+    const long long bbytes = (long long)(N - 1 - n0) * ka.stride_b + K;
     L.ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
     L.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
     L.va = (uint32_t)crow * ka.stride_a + ckc * 16;

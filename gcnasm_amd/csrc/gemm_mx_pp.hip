@@ -678,7 +678,8 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
         copy_lane(wave, lane, crow, ckc);
         {
             const char* pa = (const char*)args.ptr_A + (size_t)m0 * lda;
-            long long abytes = (long long)(M - m0) * lda;
+            // up to the last row's K: copies past K never leave the operands
+            long long abytes = (long long)(M - 1 - m0) * lda + Kb;
             L.ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
             L.va = (uint32_t)crow * lda + ckc * 16 + (uint32_t)kbb;
             L.a_hstep = 64 * lda;
@@ -693,7 +694,7 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
                        lane * 16 + (uint32_t)kbb * 16;
             } else {
                 const char* pb = (const char*)args.ptr_B + (size_t)n0 * ldb;
-                long long bbytes = (long long)(N - n0) * ldb;
+                long long bbytes = (long long)(N - 1 - n0) * ldb + Kb;
                 L.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
                 L.b_kstep = 128;
                 L.b_hstep = 64 * ldb;
