@@ -188,7 +188,9 @@ __device__ __forceinline__ void mx_store_codes(const float (&v)[EPL], int e, uin
     }
 }
 
-// EPL elements divided by their scale as E4M3 bytes at dst.
+// EPL elements divided by their scale as E4M3 bytes at dst. NAN_RULE false: no
+// quotient is a NaN, i.e. no element is one and the scale is neither infinite
+// (inf/inf) nor zero (0/0); ScaleDiv::fast holds for no such scale.
 template <bool NAN_RULE, int EPL, class D>
 __device__ __forceinline__ void fp8_store_codes(const D& d, const float (&v)[EPL], uint8_t* dst)
 {
@@ -387,13 +389,14 @@ __global__ __launch_bounds__(256) void quant_1x128_kernel(const void* __restrict
         float v[EPL];
         raw[u].unpack(ok[u], v);
         bool nan;
-        const float amax = __uint_as_float(block_amax<LPB, EPL>(v, nan));
+        const float sc = ds_scale(__uint_as_float(block_amax<LPB, EPL>(v, nan)));
+        const ScaleDiv d(sc);
+        // as uniform as nan: one such scale in the wave is enough
+        const bool nan_rule = nan || __builtin_amdgcn_ballot_w64(!d.fast) != 0;
         if (!ok[u])
             continue;
-        const float sc = ds_scale(amax);
-        const ScaleDiv d(sc);
         uint8_t* dst = q + (size_t)rr[u] * ld_q + gg[u] * 128 + sub * EPL;
-        if (nan)
+        if (nan_rule)
             fp8_store_codes<true>(d, v, dst);
         else
             fp8_store_codes<false>(d, v, dst);
@@ -451,7 +454,7 @@ __global__ __launch_bounds__(kTileThreads) void quant_128x128_kernel(
         return m;
     };
     amax = tile_max(false);
-    const bool nan = amax > 0x7F800000u;
+    const bool nan = amax > 0x7F800000u; // in every wave: amax is the tile's
     if (nan) {
         __syncthreads(); // every wave has read wmax before it is written again
         amax = tile_max(true);
@@ -464,7 +467,7 @@ __global__ __launch_bounds__(kTileThreads) void quant_128x128_kernel(
         if (r >= rows)
             continue;
         uint8_t* dst = q + (size_t)r * ld_q + g * 128 + col;
-        if (nan)
+        if (nan || !d.fast)
             fp8_store_codes<true>(d, v[i], dst);
         else
             fp8_store_codes<false>(d, v[i], dst);

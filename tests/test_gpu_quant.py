@@ -175,6 +175,49 @@ def test_quant_nan_blocks(dev, in_bf16):
     np.testing.assert_array_equal(q2.cpu().numpy(), o2)
 
 
+@pytest.mark.parametrize("narrow", [False, True])
+@pytest.mark.parametrize("in_bf16", [False, True])
+def test_quant_nan_quotients(dev, in_bf16, narrow):
+    """Quotients that are NaN where no input is: an infinity over the infinite
+    scale it makes, and a zero over a scale that rounds to 0 (an fp32 maximum
+    of at most 224 * 2^-149). Infinities of both signs as the first, last and
+    every element of a 1x128 group, beside a NaN, and in groups whose wave
+    holds no NaN; groups of the smallest subnormals. Codes and scales of the
+    three divided formats against the oracle. narrow: rows that take the
+    8-byte bf16 loads."""
+    rows, K, pad = 384, 1152, 4 if narrow else 0
+    x = oracle.randn(rows * (K + pad), 17).reshape(rows, K + pad) * np.float32(3.0)
+    inf, tiny = np.float32(np.inf), np.float32(2.0 ** -149)
+    x[0, 0] = inf                       # first of its group
+    x[1, 255] = -inf                    # last of its group
+    x[2, 256:384] = inf                 # a whole group
+    x[3, 384:512:2] = -inf
+    x[3, 385:512:2] = inf
+    x[4, 5], x[4, 6] = np.nan, -inf     # beside a NaN
+    x[290, 1100] = inf                  # the only one of its 128x128 tile
+    if not in_bf16:                     # 128x128 tiles (1, 2) and (1, 3) hold nothing larger
+        x[128:256, 256:512] = 0.0
+        x[130, 260], x[131, 270] = tiny, -tiny
+        x[140, 400], x[141, 401] = 223 * tiny, -200 * tiny
+        x[150, 300], x[151, 310] = 224 * tiny, 224 * tiny
+    x = np.ascontiguousarray(x)
+    if in_bf16:
+        xb = oracle.to_bf16_bits(x)
+        xt = torch.from_numpy(xb.view(np.int16)).to(dev).view(torch.bfloat16)[:, :K]
+        x = oracle.bf16_bits_to_f32(xb)
+    else:
+        xt = torch.from_numpy(x).to(dev)[:, :K]
+    x = np.ascontiguousarray(x[:, :K])
+    got = [ops.quant_fp8_1x128(xt), ops.quant_fp8_128x128(xt), ops.quant_fp8_per_tensor(xt)]
+    torch.cuda.synchronize()
+    want = [oracle.quant_fp8_1x128(x), oracle.quant_fp8_128x128(x), oracle.quant_fp8_per_tensor(x)]
+    assert (want[0][0][2, 256:384] == 0x7F).all() and np.isinf(want[0][1]).sum() == 6
+    assert in_bf16 or (want[0][1] == 0).any() and (want[1][1] == 0).any()
+    for (q, s), (qo, so) in zip(got, want):
+        np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), so.view(np.uint32))
+        np.testing.assert_array_equal(q.cpu().numpy(), qo)
+
+
 @pytest.mark.parametrize("amax", [1000.5, 3.7e-5, 1.7 * 2.0 ** -50, 2.0 ** -60, 3.0e38])
 def test_quant_division_every_bf16_value(dev, amax):
     """The 1x128, 128x128 and per-tensor quantisers divide by s = amax/448,
