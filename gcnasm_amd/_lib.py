@@ -29,6 +29,13 @@ GA_MX_SCALE_FLOOR_448 = 0
 GA_MX_SCALE_CEIL_448 = 1
 GA_MX_SCALE_OCP = 2
 GA_NAME_MAX = 96
+# ga_mx_plan.kernel
+GA_MX_RUNS_ENTRY = 0
+GA_MX_RUNS_K_SPLIT = 1
+GA_MX_RUNS_TILE128 = 2
+GA_MX_RUNS_FEW_ROWS = 3
+GA_MX_RUNS_FEW_ROWS_SPLIT = 4
+GA_MX_RUNS_FEW_ROWS_SHARED_A = 5
 
 
 class GaError(RuntimeError):
@@ -112,6 +119,13 @@ class TileConfig(ctypes.Structure):
         ("knl_name", ctypes.c_char * GA_NAME_MAX),
         ("co_name", ctypes.c_char * GA_NAME_MAX),
     ]
+
+
+class MxPlan(ctypes.Structure):
+    """ga_mx_plan: the kernel a launch runs (kernel: GA_MX_RUNS_*)."""
+
+    _fields_ = [("kernel", ctypes.c_int), ("rows", ctypes.c_int), ("cols", ctypes.c_int),
+                ("k_slices", ctypes.c_int), ("k_workgroups", ctypes.c_int)]
 
 
 class LaunchDesc(ctypes.Structure):
@@ -203,6 +217,7 @@ SIGNATURES = {
     "ga_kernel_launch": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, _i, _vp, _sz, _vp]),
     "ga_kernel_launch_ws_handle": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, _i, _vp, _vp]),
     "ga_kernel_launch_noalloc": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, _i, _vp]),
+    "ga_kernel_plan": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, ctypes.POINTER(MxPlan)]),
     "ga_kernel_launch_fmt": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, _i, _i, _i, _vp, _sz,
                                   _vp]),
     "ga_mxfp8_gemm": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _sz,

@@ -73,6 +73,9 @@ void launch_mx_pp_fmt(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws
 // (gemm_mx_ksplit.hip): gdz 1, 2, 4 or 8 K slices, no workspace (wsh: a caller's
 // slot, only checked). mx_ksplit_estimate_us: its estimated time at one slice.
 float mx_ksplit_estimate_us(const ga_f4gemm_kargs& args, bool fp4, int num_cu);
+// How it cuts a launch: rows and columns per wave, K slices.
+void mx_ksplit_cut(const ga_f4gemm_kargs& args, bool fp4, int gdz, int num_cu, int* rows,
+                   int* cols, int* slices);
 void launch_mx_ksplit(const ga_f4gemm_kargs& args, int gdz, bool bps, bool fp4, int fmt,
                       const ga_splitk_ws_handle* wsh, int num_cu, hipStream_t stream);
 // 128x256 (halves 2) and 128x128 (1) eight-wave kernels, any MX element format,

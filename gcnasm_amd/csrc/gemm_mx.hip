@@ -1009,6 +1009,25 @@ static MxRoute mx_route(const ga_f4gemm_kargs& a, bool fp4, int gdz, int num_cu)
     return one ? MX_ROUTE_QUARTER : MX_ROUTE_HALF;
 }
 
+// What a launch of `entry` runs: the route, and for a few-row launch that no
+// route takes its variant.
+struct MxPlan {
+    MxRoute route;
+    bool decode;
+    int split_groups; // > 0: split variant, 16-column groups per wave
+    int phys;         // its workgroups along K
+};
+
+static MxPlan mx_plan(const MxKernel& entry, const ga_f4gemm_kargs& args, int gdz, int num_cu)
+{
+    MxPlan p;
+    p.route = mx_route(args, entry.elem_bits == 4, gdz, num_cu);
+    p.decode = (int)args.M <= entry.small_m_stream && mx_decode_applies(args, gdz);
+    p.phys = gdz;
+    p.split_groups = p.decode ? mx_decode_split_groups(args, gdz, num_cu, &p.phys) : 0;
+    return p;
+}
+
 // ga_kernel_launch with the split-K workspace given either as a buffer
 // (workspace, workspace_bytes; NULL: the library-owned one) or as a device
 // slot read by the kernels at entry (wsh; graph-capture safe), and the
@@ -1095,10 +1114,7 @@ static ga_status kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, in
             return st;
     }
     const bool fp4 = k.elem_bits == 4, bps = k.cfg.bpreshuffle != 0;
-    const MxRoute route = mx_route(*args, fp4, gdz, num_cu);
-    const bool decode = (int)args->M <= k.small_m_stream && mx_decode_applies(*args, gdz);
-    int phys = gdz; // workgroups along K of the 17-64-row decode kernels
-    const int split_groups = decode ? mx_decode_split_groups(*args, gdz, num_cu, &phys) : 0;
+    const auto [route, decode, split_groups, phys] = mx_plan(k, *args, gdz, num_cu);
     const bool no_ws = gdz == 1 || (decode && (split_groups == 0 || phys == 1));
     if (route == MX_ROUTE_KSPLIT && no_ws) {
         launch_mx_ksplit(*args, gdz, bps, fp4, fmt, nullptr, num_cu, s);
@@ -1196,6 +1212,42 @@ static ga_status kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, in
 } // namespace ga
 
 extern "C" {
+
+ga_status ga_kernel_plan(int idx, const ga_f4gemm_kargs* args, int gdz, int num_cu,
+                         ga_mx_plan* plan)
+{
+    if (!args || !plan || idx < 0 || idx >= mx_registry_total())
+        return fail(GA_ERR_ARG, "kernel_plan: bad kernel index %d or null argument", idx);
+    if ((int)args->M <= 0 || (int)args->N <= 0 || (int)args->K <= 0 || gdz < 1)
+        return fail(GA_ERR_ARG, "kernel_plan: empty shape");
+    if (num_cu <= 0) {
+        ga_status st = device_cu_count(&num_cu);
+        if (st != GA_OK)
+            return st;
+    }
+    const MxKernel& k = *mx_registry_get(idx);
+    const MxPlan p = mx_plan(k, *args, gdz, num_cu);
+    *plan = {GA_MX_RUNS_ENTRY, k.cfg.tile_M, k.cfg.tile_N, gdz, gdz};
+    if (p.route == MX_ROUTE_KSPLIT) {
+        plan->kernel = GA_MX_RUNS_K_SPLIT;
+        mx_ksplit_cut(*args, k.elem_bits == 4, gdz, num_cu, &plan->rows, &plan->cols,
+                      &plan->k_slices);
+        plan->k_workgroups = 1;
+    } else if (p.route == MX_ROUTE_HALF || p.route == MX_ROUTE_QUARTER) {
+        plan->kernel = GA_MX_RUNS_TILE128;
+        plan->rows = 128;
+        plan->cols = p.route == MX_ROUTE_HALF ? 256 : 128;
+    } else if (p.decode) {
+        const bool shared = p.split_groups > 0 && p.phys == 1 && args->M > 32;
+        plan->kernel = p.split_groups == 0 ? GA_MX_RUNS_FEW_ROWS
+                       : shared            ? GA_MX_RUNS_FEW_ROWS_SHARED_A
+                                           : GA_MX_RUNS_FEW_ROWS_SPLIT;
+        plan->rows = args->M <= 16 ? 16 : args->M <= 32 ? 32 : 64;
+        plan->cols = 16 * p.split_groups;
+        plan->k_workgroups = p.split_groups > 0 ? p.phys : 1;
+    }
+    return GA_OK;
+}
 
 ga_status ga_kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, int gdy, int gdz,
                            void* workspace, size_t workspace_bytes, void* stream)

@@ -142,7 +142,8 @@ void mx_decode_kernel(ga_f4gemm_kargs args, int nwg, int ks, float* __restrict__
     // them; more rows: one wave per slice, summed through LDS. Split variant:
     // the ks K slices run on gridDim.y workgroups along K, each taking
     // kseq = ceil(ks / gridDim.y) <= 2 consecutive slices (all of them when
-    // gridDim.y is 1, for up to 32 rows).
+    // gridDim.y is 1, for up to 32 rows); every one of them has a slice
+    // (mx_decode_split_groups).
     constexpr bool kSeq = XS == 0 && TM == 1;
     constexpr bool kFoldTot = kSeq || (XS > 0 && TM <= 2); // chains summed in registers
     constexpr int SA = (TM + 1) / 2; // A scale dwords (32-row blocks)
@@ -1044,6 +1045,11 @@ int mx_decode_split_groups(const ga_f4gemm_kargs& args, int gdz, int num_cu, int
     int p = 1;
     if (groups < 5LL * num_cu)
         p = std::min(gdz, std::max((gdz + 1) / 2, (int)((8LL * num_cu + groups - 1) / groups)));
+    // each takes ceil(gdz / p) slices, so fewer than p may cover them all: a
+    // workgroup past the last slice would have no steps, and no place in the
+    // workspace for its partials (4 slices over 3: two do)
+    const int kseq = (gdz + p - 1) / p;
+    p = (gdz + kseq - 1) / kseq;
     // waves (tasks x workgroups along K) in whole rounds of one per CU, as
     // few rounds as eight groups per wave allow, the groups spread evenly
     // over them (N = 28672, one along K: 7 groups, 256 waves; N = 8192, four:

@@ -402,6 +402,15 @@ float mx_ksplit_estimate_us(const ga_f4gemm_kargs& args, bool fp4, int num_cu)
     return ks_plan(args, fp4, 1, num_cu).est;
 }
 
+void mx_ksplit_cut(const ga_f4gemm_kargs& args, bool fp4, int gdz, int num_cu, int* rows,
+                   int* cols, int* slices)
+{
+    const KsPlan p = ks_plan(args, fp4, gdz, num_cu);
+    *rows = 16 * p.tm;
+    *cols = 16 * p.ng;
+    *slices = p.ks;
+}
+
 void launch_mx_ksplit(const ga_f4gemm_kargs& args, int gdz, bool bps, bool fp4, int fmt,
                       const ga_splitk_ws_handle* wsh, int num_cu, hipStream_t stream)
 {

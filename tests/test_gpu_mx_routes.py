@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import oracle
-from gcnasm_amd import f4gemm
+from gcnasm_amd import _lib, f4gemm
 from helpers import assert_parity, bf16_compare
 
 pytestmark = pytest.mark.gpu
@@ -39,11 +39,15 @@ def run(dev, M, N, K, elem, bps, fa=0, fb=0, l2=0, alpha=1.0, beta=0.0, pad_d=0,
     args = f4gemm.fill_args(D, C, A, B, SA, SB, M, N, K, ldd, sh.scale_cols(),
                             sh.scale_cols(), alpha, beta, ld.log2_k_split)
     kern = f4gemm.Kernel().load(None, cfg)
-    ws = torch.empty(max(1, kern.workspace_bytes(ld, M, N) // 4), dtype=torch.float32, device=dev)
+    need = kern.workspace_bytes(ld, M, N) // 4
+    # past the bytes the call may use: two slices that no kernel writes
+    ws = torch.full((need + 2 * M * N,), float("nan"), dtype=torch.float32, device=dev)
+    plan = kern.plan(args, ld.gdz)
     print("mx route", M, N, K, elem, bps, fa, fb, l2, flush=True)
     kern.launch(args, ld.gdx, ld.gdy, ld.gdz, workspace=ws, fmt_a=fa, fmt_b=fb)
     torch.cuda.synchronize()
     assert torch.isnan(D[:, N:]).all() and not torch.isnan(D[:, :N]).any()
+    assert torch.isnan(ws[need:]).all()
     rows = np.unique(np.r_[np.arange(min(M, 24)), np.arange(max(0, M - 40), M),
                            np.arange(0, M, 97)])
     qr, sr = np.ascontiguousarray(qa[rows]), np.ascontiguousarray(sa[rows])
@@ -61,6 +65,7 @@ def run(dev, M, N, K, elem, bps, fa=0, fb=0, l2=0, alpha=1.0, beta=0.0, pad_d=0,
     got = D[:, :N].contiguous().view(torch.int16).cpu().numpy().view(np.uint16)[rows]
     ok, st = bf16_compare(got, oracle.to_bf16_bits(want), dot)
     assert_parity(st, "mx %dx%dx%d e%d bps%d f%d%d l%d" % (M, N, K, elem, bps, fa, fb, l2))
+    return plan
 
 
 # K-split: rows at the 32- and 64-row blocks, an odd number of 16-column groups,
@@ -99,6 +104,16 @@ def test_k_split_keeps_a_callers_slices(dev, M, N, K, l2):
     last one among them), MXFP8 and MXFP4."""
     run(dev, M, N, K, 8, 1, l2=l2, seed=l2)
     run(dev, M, N, K, 4, 1, l2=l2, seed=l2)
+
+
+# 17-64 rows, the slices over fewer workgroups along K than slices: 7 over 4,
+# 5 over 3, 6 over 3 and 4 over 2, the last with one slice or two.
+@pytest.mark.parametrize("M,N,K,l2,gdz,groups_k", [(20, 6000, 5120, 3, 7, 4), (64, 8192, 1280, 3, 5, 3),
+                                                   (33, 7168, 1536, 3, 6, 3),
+                                                   (17, 12288, 8448, 2, 4, 2)])
+def test_slices_over_fewer_workgroups(dev, M, N, K, l2, gdz, groups_k):
+    p = run(dev, M, N, K, 8, 1, l2=l2, pad_d=4, seed=gdz)
+    assert (p.kernel, p.k_slices, p.k_workgroups) == (_lib.GA_MX_RUNS_FEW_ROWS_SPLIT, gdz, groups_k)
 
 
 # The 128x256 tile: whole and ragged tiles, one K step to seven (its slots and
