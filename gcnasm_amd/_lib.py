@@ -36,6 +36,7 @@ GA_MX_RUNS_TILE128 = 2
 GA_MX_RUNS_FEW_ROWS = 3
 GA_MX_RUNS_FEW_ROWS_SPLIT = 4
 GA_MX_RUNS_FEW_ROWS_SHARED_A = 5
+GA_MX_RUNS_SHAPE_TILE = 6
 
 
 class GaError(RuntimeError):
@@ -217,7 +218,8 @@ SIGNATURES = {
     "ga_kernel_launch": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, _i, _vp, _sz, _vp]),
     "ga_kernel_launch_ws_handle": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, _i, _vp, _vp]),
     "ga_kernel_launch_noalloc": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, _i, _vp]),
-    "ga_kernel_plan": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, ctypes.POINTER(MxPlan)]),
+    "ga_kernel_plan": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, _i, _i,
+                           ctypes.POINTER(MxPlan)]),
     "ga_kernel_launch_fmt": (_i, [_i, ctypes.POINTER(F4gemmKargs), _i, _i, _i, _i, _i, _vp, _sz,
                                   _vp]),
     "ga_mxfp8_gemm": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _sz,

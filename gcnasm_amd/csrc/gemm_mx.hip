@@ -794,6 +794,13 @@ static int select_by_shape(const ga_f4gemm_kargs& args, int L, int num_cu)
     return idx;
 }
 
+// The preshuffled tile of a width for the shape (launch_by_shape's pick).
+static int tile_for_shape(bool fp4, const ga_f4gemm_kargs& args, int L, int num_cu)
+{
+    return fp4 ? select_by_shape<true, true>(args, L, num_cu)
+               : select_by_shape<true, false>(args, L, num_cu);
+}
+
 template <bool BPS, bool FP4>
 static void launch_by_shape(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh,
                             int gdx, int gdy, int gdz, hipStream_t stream)
@@ -962,27 +969,75 @@ size_t ga_kernel_workspace_bytes(int idx, const ga_launch_desc* ld, int M, int N
 namespace ga {
 
 // Which kernel a launch runs: the entry's own, or one picked by the shape. The
-// choice is the same for every entry of an element width (and for either B
-// layout and every 8-bit format), so the output does not depend on the tile a
-// caller names; the K-split kernel's sums are cut in K, the others' not.
-enum MxRoute { MX_ROUTE_OWN, MX_ROUTE_KSPLIT, MX_ROUTE_QUARTER, MX_ROUTE_HALF };
+// choice is the same for every entry of an element width and B layout, so the
+// output does not depend on the tile a caller names; the K-split kernel's sums
+// are cut in K, the others' not. MX_ROUTE_SHAPE: the manifest's tile for the
+// shape (launch_by_shape), whichever entry is named.
+enum MxRoute { MX_ROUTE_OWN, MX_ROUTE_KSPLIT, MX_ROUTE_QUARTER, MX_ROUTE_HALF, MX_ROUTE_SHAPE };
 
-static MxRoute mx_route(const ga_f4gemm_kargs& a, bool fp4, int gdz, int num_cu)
+// Up to 64 rows: the few-row kernels of gemm_mx_decode.hip, or the K-split
+// kernel. All times are MI355X, few-row / K-split.
+static bool mx_few_rows_ksplit(long long M, long long N, long long K, bool fp4, bool bps, int gdz,
+                               int num_cu)
+{
+    const long long mb = N * K / (fp4 ? 2 : 1) >> 20, row = K / (fp4 ? 2 : 1); // bytes
+    if (gdz == 1) {
+        // The few-row kernels keep weights that come from HBM. 17-64 rows: from
+        // 96 MB on (64 rows, 8192x8192 23.2 / 14.8 us, 28672x8192 41.6 / 52.6).
+        // Up to 16: from 32 MB on (16 rows, 8192x4096 6.8 / 5.6, 8192x5120
+        // 8.1 / 9.2; MXFP4 13824x4096 5.9 / 5.8, 16384x4096 5.9 / 6.9), unless
+        // there are few columns (4096x10240 12.4 / 10.0, 5120x8192 10.3 / 9.5),
+        // many for five to eight rows (49152x2048 MXFP4, 8 rows 14.4 / 12.3, 12 rows
+        // 11.9 / 12.4) or B is row-major (16384x3072 12.7 / 10.6).
+        if (M > 16)
+            return mb <= 96;
+        if (mb <= (fp4 ? 31 : 32))
+            return true;
+        return mb <= 48 && (!bps || N <= 5120 || (M > 4 && M <= 8 && N >= 24576));
+    }
+    // A caller's split: 17-64 rows in 2, 4 or 8 even slices.
+    if (M <= 16 || (gdz != 2 && gdz != 4 && gdz != 8) || mb > 96)
+        return false;
+    // Wide N: where the few-row kernels run all slices in one workgroup (five
+    // column groups per CU and more) they have no partials either, and the
+    // K-split kernel's slices leave it short waves. While that is one round of
+    // eight groups per wave it keeps two slices of up to 32 rows (28672x2048
+    // 13.9 / 11.9; 64 rows 12.5 / 15.2), four with over six groups per CU
+    // (28672x2048, 32 rows 14.2 / 13.8; 24576x2048 11.9 / 13.0) and eight with over
+    // seven (32768x2048 19.0 / 16.9; 28672x2048 14.6 / 16.0); beyond it two
+    // slices (49152x2048, 64 rows, 2 / 4 / 8 slices 24.8 / 21.5, 24.1 / 25.3, 25.1 / 26.8).
+    const long long groups = N / 16;
+    if (groups >= 5ll * num_cu) {
+        if (groups > 8ll * num_cu)
+            return gdz == 2;
+        return M <= 32 && (gdz == 2 || groups > (gdz == 4 ? 6ll : 7ll) * num_cu);
+    }
+    // Long rows of few columns: few workgroups, each with all of K to copy,
+    // where the few-row kernels spread the slices over the CUs. Up to 32 rows to
+    // 2048 columns (2048x28672, 32 rows, 2 / 8 slices 25.5 / 29.1, 14.6 / 22.6;
+    // 256x16384 13.7 / 15.1, 8.8 / 11.0; 2048x12288 13.2 / 12.2, 9.5 / 9.4, but eight
+    // slices of 1024x12288 8.1 / 9.3), with
+    // two slices or beyond 16 KB a row to 4095 (3072x28672, 8 slices 19.8 / 23.3;
+    // 3072x16384, 2 / 4 slices 17.1 / 18.3, 13.9 / 13.9; 4096x16384 18.6 / 18.7). More
+    // rows: eight slices, or four beyond 16 KB (1024x32768, 64 rows, 2 / 8 slices
+    // 39.3 / 31.2, 15.6 / 24.1, 40 rows, 4 slices 20.0 / 23.4; 256x16384, 40 rows,
+    // 4 / 8 slices 12.3 / 10.4, 9.4 / 11.0).
+    if (row >= 12288 && M <= 32 && N <= 1024 && gdz == 8)
+        return false;
+    if (row >= 16384) {
+        const bool longer = row > 16384;
+        if (M <= 32)
+            return !(N <= 2048 || (N < 4096 && (longer || gdz == 2)));
+        return !(N <= 2048 && (gdz == 8 || (gdz == 4 && longer)));
+    }
+    return true;
+}
+
+static MxRoute mx_route(const ga_f4gemm_kargs& a, bool fp4, bool bps, int fmt, int gdz, int num_cu)
 {
     const long long M = a.M, N = a.N, K = a.K;
-    if (M <= 64) {
-        // The few-row kernels (gemm_mx_decode.hip) keep the weights that come
-        // from HBM and the splits that are not 2, 4 or 8 even slices; the
-        // K-split kernel takes the smaller ones, from 17 rows on up to 96 MB
-        // (measured on MI355X, MXFP8, 64 rows, theirs against its: 8192x8192
-        // 23.2 / 14.8 us, 28672x8192 41.6 / 52.6, 8192x28672 at eight slices
-        // 51.6 / 63; 16 rows, 8192x8192 12.9 / 13.0, 5120x5120 10.4 / 7.5).
-        const long long mb = N * K / (fp4 ? 2 : 1) >> 20;
-        if (gdz == 1)
-            return mb <= (M <= 16 ? 48 : 96) ? MX_ROUTE_KSPLIT : MX_ROUTE_OWN;
-        return M > 16 && (gdz == 2 || gdz == 4 || gdz == 8) && mb <= 96 ? MX_ROUTE_KSPLIT
-                                                                       : MX_ROUTE_OWN;
-    }
+    if (M <= 64)
+        return mx_few_rows_ksplit(M, N, K, fp4, bps, gdz, num_cu) ? MX_ROUTE_KSPLIT : MX_ROUTE_OWN;
     // More rows: while the 128x256 tiles fit on the CUs in one round (the 256x256
     // tiles would be at most half a round), the largest parallelism that still
     // is one round, 128x128 or 128x256 tiles, or the K-split kernel, by
@@ -1001,12 +1056,26 @@ static MxRoute mx_route(const ga_f4gemm_kargs& a, bool fp4, int gdz, int num_cu)
     const bool one = quarters <= num_cu;
     const float frac = (float)(one ? quarters : halves) / (float)num_cu;
     const float steps = (float)(K / (fp4 ? 256 : 128));
-    const float tile_us =
+    float tile_us =
         one ? (fp4 ? 7.5f : 6.3f) + steps * (fp4 ? 0.52f + 0.06f * frac : 0.47f + 0.04f * frac)
             : 6.0f + steps * (fp4 ? 0.80f + 0.22f * frac : 0.62f + 0.25f * frac);
-    if (mx_ksplit_estimate_us(a, fp4, num_cu) < tile_us)
-        return MX_ROUTE_KSPLIT;
-    return one ? MX_ROUTE_QUARTER : MX_ROUTE_HALF;
+    MxRoute tile = one ? MX_ROUTE_QUARTER : MX_ROUTE_HALF;
+    float ksplit_us = mx_ksplit_estimate_us(a, fp4, num_cu);
+    if (M > 1024) {
+        // Past the rows its estimate was fitted on (1000), the K-split kernel takes
+        // up to 1.3 times as long (2048x512x8192: estimate 19.0, measured 24.5).
+        // And where at most half the CUs have a 128x128 tile, and N has 256
+        // columns, the four-wave tiles of twice as many workgroups are faster
+        // (4096x512x8192 30.8 us, 128x128 34.3, K-split 41.4; 3000x512x4096 17.3 /
+        // 20.4 / 21.5, MXFP4 4096x512x4096 11.9 / 14.6 / 12.9; 16384x128x8192 40.4 /
+        // 34.4 / 42.0).
+        ksplit_us *= 1.2f;
+        if (bps && fmt == 0 && 2 * quarters <= num_cu && N >= 256) {
+            tile = MX_ROUTE_SHAPE;
+            tile_us = 5.4f + 0.38f * steps;
+        }
+    }
+    return ksplit_us < tile_us ? MX_ROUTE_KSPLIT : tile;
 }
 
 // What a launch of `entry` runs: the route, and for a few-row launch that no
@@ -1018,10 +1087,11 @@ struct MxPlan {
     int phys;         // its workgroups along K
 };
 
-static MxPlan mx_plan(const MxKernel& entry, const ga_f4gemm_kargs& args, int gdz, int num_cu)
+static MxPlan mx_plan(const MxKernel& entry, const ga_f4gemm_kargs& args, int fmt, int gdz,
+                      int num_cu)
 {
     MxPlan p;
-    p.route = mx_route(args, entry.elem_bits == 4, gdz, num_cu);
+    p.route = mx_route(args, entry.elem_bits == 4, entry.cfg.bpreshuffle != 0, fmt, gdz, num_cu);
     p.decode = (int)args.M <= entry.small_m_stream && mx_decode_applies(args, gdz);
     p.phys = gdz;
     p.split_groups = p.decode ? mx_decode_split_groups(args, gdz, num_cu, &p.phys) : 0;
@@ -1114,7 +1184,7 @@ static ga_status kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, in
             return st;
     }
     const bool fp4 = k.elem_bits == 4, bps = k.cfg.bpreshuffle != 0;
-    const auto [route, decode, split_groups, phys] = mx_plan(k, *args, gdz, num_cu);
+    const auto [route, decode, split_groups, phys] = mx_plan(k, *args, fmt, gdz, num_cu);
     const bool no_ws = gdz == 1 || (decode && (split_groups == 0 || phys == 1));
     if (route == MX_ROUTE_KSPLIT && no_ws) {
         launch_mx_ksplit(*args, gdz, bps, fp4, fmt, nullptr, num_cu, s);
@@ -1179,6 +1249,9 @@ static ga_status kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, in
                           s);
     else if (split_groups > 0)
         launch_mx_decode_split(*args, gdz, phys, split_groups, bps, fp4, fmt, ws, wsh, num_cu, s);
+    else if (route == MX_ROUTE_SHAPE)
+        fp4 ? launch_by_shape<true, true>(*args, ws, nullptr, 0, 0, gdz, s)
+            : launch_by_shape<true, false>(*args, ws, nullptr, 0, 0, gdz, s);
     else if (fmt != 0)
         launch_mx_pp_fmt(*args, ws, gdz > 1 ? wsh : nullptr, gdz, bps, fmt, s);
     else
@@ -1213,20 +1286,23 @@ static ga_status kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, in
 
 extern "C" {
 
-ga_status ga_kernel_plan(int idx, const ga_f4gemm_kargs* args, int gdz, int num_cu,
-                         ga_mx_plan* plan)
+ga_status ga_kernel_plan(int idx, const ga_f4gemm_kargs* args, int gdz, int fmt_a, int fmt_b,
+                         int num_cu, ga_mx_plan* plan)
 {
     if (!args || !plan || idx < 0 || idx >= mx_registry_total())
         return fail(GA_ERR_ARG, "kernel_plan: bad kernel index %d or null argument", idx);
     if ((int)args->M <= 0 || (int)args->N <= 0 || (int)args->K <= 0 || gdz < 1)
         return fail(GA_ERR_ARG, "kernel_plan: empty shape");
+    if (fmt_a < 0 || fmt_a > 1 || fmt_b < 0 || fmt_b > 1)
+        return fail(GA_ERR_ARG, "kernel_plan: element formats must be 0 (E4M3) or 1 (E5M2)");
+    const int fmt = fmt_a | (fmt_b << 1);
     if (num_cu <= 0) {
         ga_status st = device_cu_count(&num_cu);
         if (st != GA_OK)
             return st;
     }
     const MxKernel& k = *mx_registry_get(idx);
-    const MxPlan p = mx_plan(k, *args, gdz, num_cu);
+    const MxPlan p = mx_plan(k, *args, fmt, gdz, num_cu);
     *plan = {GA_MX_RUNS_ENTRY, k.cfg.tile_M, k.cfg.tile_N, gdz, gdz};
     if (p.route == MX_ROUTE_KSPLIT) {
         plan->kernel = GA_MX_RUNS_K_SPLIT;
@@ -1237,6 +1313,11 @@ ga_status ga_kernel_plan(int idx, const ga_f4gemm_kargs* args, int gdz, int num_
         plan->kernel = GA_MX_RUNS_TILE128;
         plan->rows = 128;
         plan->cols = p.route == MX_ROUTE_HALF ? 256 : 128;
+    } else if (p.route == MX_ROUTE_SHAPE) {
+        const int tile = tile_for_shape(k.elem_bits == 4, *args, 0, num_cu);
+        plan->kernel = GA_MX_RUNS_SHAPE_TILE;
+        plan->rows = g_mx_kernels[tile].cfg.tile_M;
+        plan->cols = g_mx_kernels[tile].cfg.tile_N;
     } else if (p.decode) {
         const bool shared = p.split_groups > 0 && p.phys == 1 && args->M > 32;
         plan->kernel = p.split_groups == 0 ? GA_MX_RUNS_FEW_ROWS

@@ -235,11 +235,12 @@ class Kernel:
         d = ld.to_c()
         return lib().ga_kernel_workspace_bytes(self.idx, ctypes.byref(d), M, N)
 
-    def plan(self, args, gdz, num_cu=0):
+    def plan(self, args, gdz, num_cu=0, fmt_a=0, fmt_b=0):
         """The kernel launch(args, ..., gdz) runs on num_cu compute units (0: the
         current device's): a _lib.MxPlan."""
         p = _lib.MxPlan()
-        check(lib().ga_kernel_plan(self.idx, ctypes.byref(args), gdz, num_cu, ctypes.byref(p)))
+        check(lib().ga_kernel_plan(self.idx, ctypes.byref(args), gdz, int(fmt_a), int(fmt_b),
+                                   num_cu, ctypes.byref(p)))
         return p
 
     def launch(self, args, gdx, gdy, gdz, stream=None, workspace=None, ws_handle=None,

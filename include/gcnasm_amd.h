@@ -380,28 +380,30 @@ ga_status ga_kernel_launch_ws_handle(int idx, const ga_f4gemm_kargs* args, int g
 ga_status ga_kernel_launch_noalloc(int idx, const ga_f4gemm_kargs* args, int gdx, int gdy,
                                    int gdz, void* stream);
 
-/* The kernel that ga_kernel_launch(idx, args, ..., gdz) runs on a device with
- * num_cu compute units (0: the current device's), which the sizes, gdz and
- * log2_k_split of args decide; its pointers are not looked at, and with
- * num_cu given nothing here needs a GPU. kernel: one of GA_MX_RUNS_*. rows x
- * cols: its tile (ENTRY, TILE128), a wave's share of C (K_SPLIT; FEW_ROWS_*,
- * where 0 columns means that the launch has no fixed share). k_slices: fp32
+/* The kernel that ga_kernel_launch_fmt(idx, args, ..., gdz, fmt_a, fmt_b)
+ * (0, 0: ga_kernel_launch) runs on a device with num_cu compute units (0: the
+ * current device's), which the sizes, formats, gdz and log2_k_split of args
+ * decide; its pointers are not looked at, and with num_cu given nothing here
+ * needs a GPU. kernel: one of GA_MX_RUNS_*. rows x cols: its tile (ENTRY,
+ * TILE128, SHAPE_TILE), a wave's share of C (K_SPLIT; FEW_ROWS_*, where 0
+ * columns means that the launch has no fixed share). k_slices: fp32
  * chains per output, summed in order. k_workgroups: workgroups along K;
  * each takes ceil(k_slices / k_workgroups) slices, and with more than one the
  * partials pass through the workspace. */
 enum {
-    GA_MX_RUNS_ENTRY = 0,            /* the entry's own tile */
-    GA_MX_RUNS_K_SPLIT = 1,          /* K cut over the waves of a workgroup */
-    GA_MX_RUNS_TILE128 = 2,          /* 128x128 or 128x256 eight-wave tile */
-    GA_MX_RUNS_FEW_ROWS = 3,         /* B streamed, K slices in a workgroup */
-    GA_MX_RUNS_FEW_ROWS_SPLIT = 4,   /* B streamed, K slices over workgroups */
-    GA_MX_RUNS_FEW_ROWS_SHARED_A = 5 /* B streamed, A shared through LDS */
+    GA_MX_RUNS_ENTRY = 0,             /* the entry's own tile */
+    GA_MX_RUNS_K_SPLIT = 1,           /* K cut over the waves of a workgroup */
+    GA_MX_RUNS_TILE128 = 2,           /* 128x128 or 128x256 eight-wave tile */
+    GA_MX_RUNS_FEW_ROWS = 3,          /* B streamed, K slices in a workgroup */
+    GA_MX_RUNS_FEW_ROWS_SPLIT = 4,    /* B streamed, K slices over workgroups */
+    GA_MX_RUNS_FEW_ROWS_SHARED_A = 5, /* B streamed, A shared through LDS */
+    GA_MX_RUNS_SHAPE_TILE = 6         /* the manifest's tile for the shape */
 };
 typedef struct ga_mx_plan {
     int kernel, rows, cols, k_slices, k_workgroups;
 } ga_mx_plan;
-ga_status ga_kernel_plan(int idx, const ga_f4gemm_kargs* args, int gdz, int num_cu,
-                         ga_mx_plan* plan);
+ga_status ga_kernel_plan(int idx, const ga_f4gemm_kargs* args, int gdz, int fmt_a, int fmt_b,
+                         int num_cu, ga_mx_plan* plan);
 
 /* ga_kernel_launch with the 8-bit element format of each MXFP8 operand:
  * fmt_a (A) and fmt_b (B) are f8f6f4 format codes, 0 = E4M3 (fp8, what

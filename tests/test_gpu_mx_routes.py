@@ -42,7 +42,7 @@ def run(dev, M, N, K, elem, bps, fa=0, fb=0, l2=0, alpha=1.0, beta=0.0, pad_d=0,
     need = kern.workspace_bytes(ld, M, N) // 4
     # past the bytes the call may use: two slices that no kernel writes
     ws = torch.full((need + 2 * M * N,), float("nan"), dtype=torch.float32, device=dev)
-    plan = kern.plan(args, ld.gdz)
+    plan = kern.plan(args, ld.gdz, fmt_a=fa, fmt_b=fb)
     print("mx route", M, N, K, elem, bps, fa, fb, l2, flush=True)
     kern.launch(args, ld.gdx, ld.gdy, ld.gdz, workspace=ws, fmt_a=fa, fmt_b=fb)
     torch.cuda.synchronize()
@@ -154,6 +154,16 @@ def test_quarter_tile_formats_alpha_beta(dev):
 
 def test_half_tile_alpha_beta(dev):
     run(dev, 1000, 8192, 512, 8, 1, alpha=-1.5, beta=0.25, pad_d=12, seed=3)
+
+
+# More than 1024 rows whose 128x128 tiles leave half the CUs idle: the four-wave
+# tile of the shape, whichever entry is named, whole and ragged.
+@pytest.mark.parametrize("M,N,K", [(5290, 368, 1024), (4096, 512, 1152), (4090, 496, 1536)])
+def test_shape_tile(dev, M, N, K):
+    assert run(dev, M, N, K, 8, 1, pad_d=4, seed=K).kernel == _lib.GA_MX_RUNS_SHAPE_TILE
+    if K % 256 == 0:
+        p = run(dev, M, N, 2 * K, 4, 1, alpha=0.5, beta=2.0, seed=K)
+        assert p.kernel == _lib.GA_MX_RUNS_SHAPE_TILE
 
 
 @pytest.mark.parametrize("elem", [8, 4])
