@@ -111,6 +111,30 @@ def test_tiles(dev, shape, group_n):
     run(dev, shape, group_n, 1, 0, 32 if M % 128 else 0, -N % 4 + 4 if N % 8 else 8, True)
 
 
+# 33-64 rows with 64x256 tiles for three quarters of 256 CUs and more: one
+# group, an odd number, even; ragged columns; batches of few tiles each.
+@pytest.mark.parametrize("batch,shape", [(1, (33, 49157, 128)), (1, (64, 49152, 640)),
+                                         (1, (48, 65538, 256)), (24, (40, 2049, 384)),
+                                         (64, (63, 640, 512))])
+@pytest.mark.parametrize("group_n", [128, 1, 0])
+def test_rows64_tile(dev, batch, shape, group_n):
+    M, N, K = shape
+    run(dev, shape, group_n, batch, 16, 48, -N % 4 + 4 if N % 8 else 8, True)
+    # one tile fewer than that, and 32 rows: the K-split kernel
+    assert opus_gemm.k_slices(64, 256 * 191, 1024) < 8 == opus_gemm.k_slices(64, 256 * 192, 1024)
+    assert opus_gemm.k_slices(32, 256 * 192, 1024) < 8
+
+
+# Batches: the K-split kernel only against the 128x128 tile, and only where it
+# wins by half the time of the operands' bytes.
+@pytest.mark.parametrize("batch,M,N,K,split", [(4, 96, 4096, 7168, True), (2, 128, 7168, 2048, True),
+                                               (16, 128, 1024, 4096, False),
+                                               (200, 128, 512, 512, False),
+                                               (16, 300, 7168, 512, False)])
+def test_batches_route(dev, batch, M, N, K, split):
+    assert (opus_gemm.k_slices(M, N, K, batch) < K // 128) == split
+
+
 @pytest.mark.parametrize("shape", [(1030, 384, 384), (1030, 2100, 384)])
 @pytest.mark.parametrize("group_n", [128, 1, 0])
 def test_tiles_batched_unaligned(dev, shape, group_n):
