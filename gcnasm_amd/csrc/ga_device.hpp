@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/gcnasm_amd.h"
+#include "ga_extent.hpp"
 #include <stdint.h>
 
 #include <type_traits>

@@ -59,11 +59,8 @@ void bs_rows64_kernel(ga_opus_gemm_kargs ka)
     const char* pa = (const char*)ka.ptr_a + (size_t)b * ka.stride_a_batch;
     const char* pb = (const char*)ka.ptr_b + (size_t)b * ka.stride_b_batch +
                      (size_t)n0 * ka.stride_b;
-    // up to the last row's K bytes: copies past K never leave the operands
-    const long long abytes = (long long)(M - 1) * ka.stride_a + K;
-    const long long bbytes = (long long)(N - 1 - n0) * ka.stride_b + K;
-    const auto ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
-    const auto rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+    const auto ra = make_rsrc(pa, rows_bytes(M, ka.stride_a, K));
+    const auto rb = make_rsrc(pb, rows_bytes(N - n0, ka.stride_b, K));
     // copy i covers rows 32i .. 32i + 31, 8 of them by this wave
     int row0, chunk;
     pp::copy_lane(wave, lane, row0, chunk);

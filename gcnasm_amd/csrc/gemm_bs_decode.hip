@@ -98,13 +98,10 @@ void bs_decode_kernel(ga_opus_gemm_kargs ka, int nwg, int mblocks, int ks, int g
     if (nsteps > 0) {
         const uint32_t lda = (uint32_t)ka.stride_a, ldb = (uint32_t)ka.stride_b;
         const char* pa = (const char*)ka.ptr_a + (size_t)b * ka.stride_a_batch + (size_t)m0 * lda;
-        // up to the last row's K: copies past K never leave the operands
-        const long long abytes = (long long)(M - 1) * lda + ka.k;
-        const auto ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
+        const auto ra = make_rsrc(pa, rows_bytes(M, lda, K));
         const char* pb = (const char*)ka.ptr_b + (size_t)b * ka.stride_b_batch +
                          (size_t)cg0 * 16 * ldb;
-        const long long brows = min(ng_here * 16, N - cg0 * 16);
-        const auto rb = make_rsrc(pb, (uint32_t)min((brows - 1) * ldb + ka.k, 0xFFFFFFF0ll));
+        const auto rb = make_rsrc(pb, rows_bytes(min(ng_here * 16, N - cg0 * 16), ldb, K));
         // copy h (0, 1) of a 16-row block: lane l fetches row 8h + l / 8 from
         // whole 128-byte lines into slot l % 8
         const uint32_t crow = (uint32_t)lane >> 3, cslot = lane & 7;
@@ -116,26 +113,25 @@ void bs_decode_kernel(ga_opus_gemm_kargs ka, int nwg, int mblocks, int ks, int g
 
         // scales (fp32): SFA [K/128, M], lane l row l; SFB [ceil(N/128),
         // K/128], lane l group l % NG's 128-column block, or [K/128, N], lane l
-        // column l (past N: bytes of the next row or range-checked zeros, for
-        // columns that are never stored)
+        // column l (past N: the last column's, for columns never stored)
         __amdgpu_buffer_rsrc_t rsa = ra, rsb = rb;
         uint32_t vsa = 0, vsb = 0, sa_step = 0, sb_step = 0;
         if constexpr (MODE != BD_TENSOR) {
             const float* sfa = (const float*)ka.ptr_sfa + (size_t)b * ka.stride_sfa_batch;
             const float* sfb = (const float*)ka.ptr_sfb + (size_t)b * ka.stride_sfb_batch;
-            rsa = make_rsrc(sfa, (uint32_t)G * ka.stride_sfa * 4);
+            rsa = make_rsrc(sfa, rows_bytes(G, 4ll * ka.stride_sfa, 4ll * ka.m));
             sa_step = (uint32_t)ka.stride_sfa * 4;
             vsa = ((uint32_t)gb * ka.stride_sfa + m0 + min(lane, M - 1)) * 4;
             if constexpr (MODE == BD_GROUP128) {
                 const int nblk = (N + 127) / 128;
-                rsb = make_rsrc(sfb, (uint32_t)nblk * ka.stride_sfb * 4);
+                rsb = make_rsrc(sfb, rows_bytes(nblk, 4ll * ka.stride_sfb, 4ll * G));
                 sb_step = 4;
                 vsb = ((uint32_t)min(((cg0 + lane % NG) * 16) / 128, nblk - 1) * ka.stride_sfb +
                        gb) * 4;
             } else {
-                rsb = make_rsrc(sfb, (uint32_t)G * ka.stride_sfb * 4);
+                rsb = make_rsrc(sfb, rows_bytes(G, 4ll * ka.stride_sfb, 4ll * N));
                 sb_step = (uint32_t)ka.stride_sfb * 4;
-                vsb = ((uint32_t)gb * ka.stride_sfb + cg0 * 16 + lane) * 4;
+                vsb = ((uint32_t)gb * ka.stride_sfb + min(cg0 * 16 + lane, N - 1)) * 4;
             }
         }
 

@@ -50,11 +50,8 @@ __device__ __forceinline__ void bs_load_setup(const ga_opus_gemm_kargs& ka, int 
                      (size_t)m0 * ka.stride_a;
     const char* pb = (const char*)ka.ptr_b + (size_t)b * ka.stride_b_batch +
                      (size_t)n0 * ka.stride_b;
-    // up to the last row's K bytes: copies past K never leave the operands
-    const long long abytes = (long long)(M - 1 - m0) * ka.stride_a + K;
-    const long long bbytes = (long long)(N - 1 - n0) * ka.stride_b + K;
-    L.ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
-    L.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+    L.ra = make_rsrc(pa, rows_bytes(M - m0, ka.stride_a, K));
+    L.rb = make_rsrc(pb, rows_bytes(N - n0, ka.stride_b, K));
     L.va = (uint32_t)crow * ka.stride_a + ckc * 16;
     L.vb = (uint32_t)crow * ka.stride_b + ckc * 16;
     L.a_hstep = 64 * (uint32_t)ka.stride_a;
@@ -67,7 +64,7 @@ __device__ __forceinline__ void bs_load_setup(const ga_opus_gemm_kargs& ka, int 
             // SFA [K/128, M]: LDS position w*64 + l holds row
             // w*64 + (l%4)*16 + l/4 (rows past M clamp to M-1)
             const float* sfa = (const float*)ka.ptr_sfa + (size_t)b * ka.stride_sfa_batch;
-            L.rs = make_rsrc(sfa, (uint32_t)ngroups * ka.stride_sfa * 4);
+            L.rs = make_rsrc(sfa, rows_bytes(ngroups, 4ll * ka.stride_sfa, 4ll * M));
             const int row = min(m0 + wave * 64 + (lane & 3) * 16 + (lane >> 2), M - 1);
             L.vs = (uint32_t)row * 4;
             L.s_kstep = (uint32_t)ka.stride_sfa * 4;
@@ -78,13 +75,13 @@ __device__ __forceinline__ void bs_load_setup(const ga_opus_gemm_kargs& ka, int 
                 // SFB [ceil(N/128), K/128]: positions 0 and 1 hold the
                 // tile's two 128-column blocks
                 const int nblk = (N + 127) / 128;
-                L.rs = make_rsrc(sfb, (uint32_t)nblk * ka.stride_sfb * 4);
+                L.rs = make_rsrc(sfb, rows_bytes(nblk, 4ll * ka.stride_sfb, 4ll * ngroups));
                 const int nb = min(n0 / 128 + (pos & 1), nblk - 1);
                 L.vs = (uint32_t)nb * ka.stride_sfb * 4;
                 L.s_kstep = 4;
             } else {
                 // SFB [K/128, N]: position c holds column n0 + c
-                L.rs = make_rsrc(sfb, (uint32_t)ngroups * ka.stride_sfb * 4);
+                L.rs = make_rsrc(sfb, rows_bytes(ngroups, 4ll * ka.stride_sfb, 4ll * N));
                 const int col = min(n0 + pos, N - 1);
                 L.vs = (uint32_t)col * 4;
                 L.s_kstep = (uint32_t)ka.stride_sfb * 4;

@@ -183,10 +183,8 @@ __device__ __forceinline__ BsLoad bs_load_from(const ga_opus_gemm_kargs& ka, int
     copy_lane(wave, lane, crow, ckc);
     const char* pa = (const char*)ka.ptr_a + (size_t)m0 * ka.stride_a;
     const char* pb = (const char*)ka.ptr_b + (size_t)n0 * ka.stride_b;
-    const long long abytes = (long long)(M - m0) * ka.stride_a;
-    const long long bbytes = (long long)(N - n0) * ka.stride_b;
-    L.ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
-    L.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+    L.ra = make_rsrc(pa, rows_bytes(M - m0, ka.stride_a, K));
+    L.rb = make_rsrc(pb, rows_bytes(N - n0, ka.stride_b, K));
     L.va = (uint32_t)crow * ka.stride_a + ckc * 16 + (uint32_t)g0 * 128;
     L.vb = (uint32_t)crow * ka.stride_b + ckc * 16 + (uint32_t)g0 * 128;
     L.a_hstep = 64 * (uint32_t)ka.stride_a;
@@ -197,7 +195,7 @@ __device__ __forceinline__ BsLoad bs_load_from(const ga_opus_gemm_kargs& ka, int
         const int ngroups = K / 128;
         if (wave < 4) {
             const float* sfa = (const float*)ka.ptr_sfa;
-            L.rs = make_rsrc(sfa, (uint32_t)ngroups * ka.stride_sfa * 4);
+            L.rs = make_rsrc(sfa, rows_bytes(ngroups, 4ll * ka.stride_sfa, 4ll * M));
             const int row = min(m0 + wave * 64 + (lane & 3) * 16 + (lane >> 2), M - 1);
             L.s_kstep = (uint32_t)ka.stride_sfa * 4;
             L.vs = (uint32_t)row * 4 + (uint32_t)g0 * L.s_kstep;
@@ -206,12 +204,12 @@ __device__ __forceinline__ BsLoad bs_load_from(const ga_opus_gemm_kargs& ka, int
             const int pos = (wave - 4) * 64 + lane;
             if (MODE == PS_GROUP128) {
                 const int nblk = (N + 127) / 128;
-                L.rs = make_rsrc(sfb, (uint32_t)nblk * ka.stride_sfb * 4);
+                L.rs = make_rsrc(sfb, rows_bytes(nblk, 4ll * ka.stride_sfb, 4ll * ngroups));
                 const int nb = min(n0 / 128 + (pos & 1), nblk - 1);
                 L.s_kstep = 4;
                 L.vs = (uint32_t)nb * ka.stride_sfb * 4 + (uint32_t)g0 * 4;
             } else {
-                L.rs = make_rsrc(sfb, (uint32_t)ngroups * ka.stride_sfb * 4);
+                L.rs = make_rsrc(sfb, rows_bytes(ngroups, 4ll * ka.stride_sfb, 4ll * N));
                 const int col = min(n0 + pos, N - 1);
                 L.s_kstep = (uint32_t)ka.stride_sfb * 4;
                 L.vs = (uint32_t)col * 4 + (uint32_t)g0 * L.s_kstep;

@@ -44,13 +44,23 @@ def padded(x, ld, dev):
     return torch.from_numpy(out).to(dev)
 
 
-def run(dev, shape, group_n, batch, pad_a, pad_b, pad_c, whole_k=False):
+def strided(x, pad, dev):
+    """x [batch, rows, cols] on the device as a view whose rows are `pad` NaNs
+    apart and whose storage ends with its last element; the strides with it."""
+    b, r, c = x.shape
+    flat = torch.full((b * r * (c + pad) - pad,), float("nan"), dtype=torch.float32, device=dev)
+    view = flat.as_strided((b, r, c), (r * (c + pad), c + pad, 1))
+    view.copy_(torch.from_numpy(x))
+    return view
+
+
+def run(dev, shape, group_n, batch, pad_a, pad_b, pad_c, whole_k=False, pad_s=0):
     M, N, K = shape
     qa, qb, sfa, sfb = problem(batch, M, N, K, group_n or 128, M + N + K)
     gps = opus_gemm.k_slices(M, N, K, batch)
     assert not whole_k or gps == K // 128
     A, B = padded(qa, K + pad_a, dev), padded(qb, K + pad_b, dev)
-    SA, SB = torch.from_numpy(sfa).to(dev), torch.from_numpy(sfb).to(dev)
+    SA, SB = strided(sfa, pad_s, dev), strided(sfb, pad_s, dev)
     rows = np.unique(np.r_[np.arange(min(M, 48)), np.arange(max(0, M - 20), M)])
     want, absdot = [], []
     for b in range(batch):
@@ -70,6 +80,9 @@ def run(dev, shape, group_n, batch, pad_a, pad_b, pad_c, whole_k=False):
         ka.stride_a, ka.stride_b, ka.stride_c = K + pad_a, K + pad_b, N + pad_c
         ka.stride_a_batch, ka.stride_b_batch = M * ka.stride_a, N * ka.stride_b
         ka.stride_c_batch = M * ka.stride_c
+        if group_n:
+            (ka.stride_sfa_batch, ka.stride_sfa), (ka.stride_sfb_batch, ka.stride_sfb) = (
+                SA.stride()[:2], SB.stride()[:2])
         out = _lib.GA_DTYPE_F32 if dtype == torch.float32 else _lib.GA_DTYPE_BF16
         print("fp32 scales", shape, group_n, dtype, "groups per slice", gps, flush=True)
         if group_n:
@@ -123,6 +136,17 @@ def test_rows64_tile(dev, batch, shape, group_n):
     # one tile fewer than that, and 32 rows: the K-split kernel
     assert opus_gemm.k_slices(64, 256 * 191, 1024) < 8 == opus_gemm.k_slices(64, 256 * 192, 1024)
     assert opus_gemm.k_slices(32, 256 * 192, 1024) < 8
+
+
+@pytest.mark.parametrize("shape,batch", [((5, 40, 256), 2), ((30, 1000, 384), 1), ((64, 2113, 1152), 1),
+                                         ((40, 49157, 128), 1), ((1026, 200, 256), 1),
+                                         ((1030, 2100, 384), 3), ((1100, 7700, 128), 1)])
+@pytest.mark.parametrize("group_n", [128, 1])
+def test_strided_scales(dev, shape, batch, group_n):
+    """Scale matrices with NaNs between their rows and nothing behind the last
+    one: the K-split kernel's wave tiles, the 64x256, 128x128, 128x256 and 256x256
+    tiles (the copies of the groups past K and the columns past N are not used)."""
+    run(dev, shape, group_n, batch, 0, 16, 0, pad_s=5)
 
 
 # Batches: the K-split kernel only against the 128x128 tile, and only where it
