@@ -274,8 +274,7 @@ void mx_gemm_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
     MxState<C> st;
     {
         const char* pa = (const char*)args.ptr_A + (size_t)m0 * lda;
-        long long abytes = (long long)(M - m0) * lda;
-        st.ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
+        st.ra = make_rsrc(pa, rows_bytes(M - m0, lda, Kb));
         // row-major operands: copy i covers rows 32i .. 32i+31 (wave w: 8
         // whole 128-byte rows) of the swizzled LDS image
         int row0, chunk;
@@ -285,8 +284,7 @@ void mx_gemm_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
             st.voff_a[i] = (uint32_t)(i * 32 + row0) * lda + chunk * 16;
         if (C::BPS) {
             const char* pb = (const char*)args.ptr_B + (size_t)(n0 / 16) * Kb * 16;
-            long long bbytes = (long long)(N - n0) * Kb;
-            st.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+            st.rb = make_rsrc(pb, rows_bytes(N - n0, Kb, Kb));
             st.b_kstride = 128 * 16;
 #pragma unroll
             for (int i = 0; i < C::B_LOADS; i++) {
@@ -296,8 +294,7 @@ void mx_gemm_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
             }
         } else {
             const char* pb = (const char*)args.ptr_B + (size_t)n0 * ldb;
-            long long bbytes = (long long)(N - n0) * ldb;
-            st.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+            st.rb = make_rsrc(pb, rows_bytes(N - n0, ldb, Kb));
             st.b_kstride = 128;
 #pragma unroll
             for (int i = 0; i < C::B_LOADS; i++)
@@ -533,8 +530,7 @@ void mx_bstream_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
     MbState<C> st;
     {
         const char* pa = (const char*)args.ptr_A + (size_t)m0 * lda;
-        long long abytes = (long long)(M - m0) * lda;
-        st.ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
+        st.ra = make_rsrc(pa, rows_bytes(M - m0, lda, Kb));
         int row0, chunk;
         pp::copy_lane(wave, lane, row0, chunk);
 #pragma unroll
@@ -543,8 +539,7 @@ void mx_bstream_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
         // preshuffled B: 16-row group g of the tile holds its K steps as
         // consecutive 2 KB blocks; rows past N read as zero
         const char* pb = (const char*)args.ptr_B + (size_t)(n0 / 16) * Kb * 16;
-        long long bbytes = (long long)(N - n0) * Kb;
-        st.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+        st.rb = make_rsrc(pb, rows_bytes(N - n0, Kb, Kb));
         st.gstride = (uint32_t)Kb * 16;
         st.vb = (uint32_t)(wave * C::TN) * st.gstride + (uint32_t)lane * 16;
         const int sma = (M + 31) / 32 * 32, smb = (N + 31) / 32 * 32;

@@ -271,8 +271,7 @@ void mx_decode_kernel(ga_f4gemm_kargs args, int nwg, int ks, float* __restrict__
 
     const int r = lane & 15, g = lane >> 4;
     const uint32_t lda = args.stride_A0 / kEPB; // bytes
-    const long long abytes = (long long)M * lda;
-    const auto ra = make_rsrc(args.ptr_A, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
+    const auto ra = make_rsrc(args.ptr_A, rows_bytes(M, lda, Kb));
     // A: lane 16g + r reads row 16i + r, K chunks g and g + 4 of the step
     const uint32_t va = (uint32_t)r * lda + g * 16 + (uint32_t)kbb;
     if constexpr (LA) {
@@ -315,7 +314,7 @@ void mx_decode_kernel(ga_f4gemm_kargs args, int nwg, int ks, float* __restrict__
         } else {
             const uint32_t ldb = args.stride_B0 / kEPB; // bytes
             const char* pb = (const char*)args.ptr_B + (size_t)cg0 * 16 * ldb;
-            rbuf = make_rsrc(pb, (uint32_t)ng_here * 16 * ldb);
+            rbuf = make_rsrc(pb, rows_bytes(ng_here * 16, ldb, Kb));
             vb = (uint32_t)r * ldb + g * 16 + (uint32_t)kbb;
             b_step = 128;
             b_hi = 64;
@@ -706,8 +705,7 @@ __global__ __launch_bounds__(64 * W) void mx_decode_la_kernel(ga_f4gemm_kargs ar
     if (nsteps > 0) {
         const int r = lane & 15, g = lane >> 4;
         const uint32_t lda = args.stride_A0 / kEPB; // bytes
-        const long long abytes = (long long)M * lda;
-        const auto ra = make_rsrc(args.ptr_A, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
+        const auto ra = make_rsrc(args.ptr_A, rows_bytes(M, lda, Kb));
         // A of a step in LDS: rows 16i .. 16i + 15 as 128-byte rows at byte
         // i * 2048 of the slot, K chunk c of row 16i + t at slot
         // c ^ ((t >> 1) & 7). Copy (i, h) writes rows 16i + 8h .. + 7 from
@@ -730,7 +728,7 @@ __global__ __launch_bounds__(64 * W) void mx_decode_la_kernel(ga_f4gemm_kargs ar
         } else {
             const uint32_t ldb = args.stride_B0 / kEPB; // bytes
             const char* pb = (const char*)args.ptr_B + (size_t)(live ? cg0 : 0) * 16 * ldb;
-            rbuf = make_rsrc(pb, (uint32_t)ngb * 16 * ldb);
+            rbuf = make_rsrc(pb, ngb > 0 ? rows_bytes(ngb * 16, ldb, Kb) : 0u);
             vb = (uint32_t)r * ldb + g * 16 + (uint32_t)kbb;
             b_step = 128;
             b_hi = 64;

@@ -99,9 +99,7 @@ void mx_ksplit_kernel(ga_f4gemm_kargs args, int nwg, int mblocks, int ks, int kp
     if (nsteps > 0) {
         const uint32_t lda = args.stride_A0 / kEPB, ldb = args.stride_B0 / kEPB; // bytes
         const char* pa = (const char*)args.ptr_A + (size_t)m0 * lda;
-        // up to the last row's K: copies past K never leave the operands
-        const long long abytes = (long long)(M - 1) * lda + Kb;
-        const auto ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
+        const auto ra = make_rsrc(pa, rows_bytes(M, lda, Kb));
         // copy h (0, 1) of a row-major block: lane l fetches row 8h + l / 8
         // from whole 128-byte lines into slot l % 8
         const uint32_t crow = (uint32_t)lane >> 3, cslot = lane & 7;
@@ -120,7 +118,7 @@ void mx_ksplit_kernel(ga_f4gemm_kargs args, int nwg, int mblocks, int ks, int kp
             b_grp = (uint32_t)Kb * 16;
         } else {
             rb = make_rsrc((const char*)args.ptr_B + (size_t)cg0 * 16 * ldb,
-                           ((uint32_t)ng_here * 16 - 1) * ldb + (uint32_t)Kb);
+                           rows_bytes(ng_here * 16, ldb, Kb));
             vb0 = crow * ldb + c0 + (uint32_t)kbb;
             vb1 = (crow + 8) * ldb + c1 + (uint32_t)kbb;
             b_step = 128;

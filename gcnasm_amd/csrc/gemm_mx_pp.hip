@@ -307,8 +307,7 @@ __device__ __forceinline__ void pp_tile(const PpArgs& args, float* __restrict__ 
         copy_lane(wave, lane, crow, ckc);
         {
             const char* pa = (const char*)args.ptr_A + (size_t)m0 * lda;
-            long long abytes = (long long)(M - m0) * lda;
-            L.ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
+            L.ra = make_rsrc(pa, rows_bytes(M - m0, lda, Kb));
             L.va = (uint32_t)crow * lda + ckc * 16 + (uint32_t)kbb;
             L.a_hstep = 64 * lda;
             if (BPS) {
@@ -316,16 +315,14 @@ __device__ __forceinline__ void pp_tile(const PpArgs& args, float* __restrict__ 
                 // [Kb/16][16 rows][16 B]; one K step is 2 KB of it. Copy c of
                 // half h: groups h*8 + c*4 + wave/2, bytes (wave&1)*1024 + lane*16.
                 const char* pb = (const char*)args.ptr_B + (size_t)(n0 / 16) * Kb * 16;
-                long long bbytes = (long long)(N - n0) * Kb;
-                L.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+                L.rb = make_rsrc(pb, rows_bytes(N - n0, Kb, Kb));
                 L.b_kstep = 2048;
                 L.b_hstep = 4 * (uint32_t)Kb * 16;
                 L.vb = (uint32_t)(wave >> 1) * (uint32_t)Kb * 16 + (wave & 1) * 1024 +
                        lane * 16 + (uint32_t)kbb * 16;
             } else {
                 const char* pb = (const char*)args.ptr_B + (size_t)n0 * ldb;
-                long long bbytes = (long long)(N - n0) * ldb;
-                L.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+                L.rb = make_rsrc(pb, rows_bytes(N - n0, ldb, Kb));
                 L.b_kstep = 128;
                 L.b_hstep = 64 * ldb;
                 L.vb = (uint32_t)crow * ldb + ckc * 16 + (uint32_t)kbb;
@@ -678,24 +675,20 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
         copy_lane(wave, lane, crow, ckc);
         {
             const char* pa = (const char*)args.ptr_A + (size_t)m0 * lda;
-            // up to the last row's K: copies past K never leave the operands
-            long long abytes = (long long)(M - 1 - m0) * lda + Kb;
-            L.ra = make_rsrc(pa, (uint32_t)(abytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : abytes));
+            L.ra = make_rsrc(pa, rows_bytes(M - m0, lda, Kb));
             L.va = (uint32_t)crow * lda + ckc * 16 + (uint32_t)kbb;
             L.a_hstep = 64 * lda;
             if (BPS) {
                 // copy c (64 columns): groups 4c + wave/2, bytes (wave&1)*1024 + lane*16
                 const char* pb = (const char*)args.ptr_B + (size_t)(n0 / 16) * Kb * 16;
-                long long bbytes = (long long)(N - n0) * Kb;
-                L.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+                L.rb = make_rsrc(pb, rows_bytes(N - n0, Kb, Kb));
                 L.b_kstep = 2048;
                 L.b_hstep = 4 * (uint32_t)Kb * 16;
                 L.vb = (uint32_t)(wave >> 1) * (uint32_t)Kb * 16 + (wave & 1) * 1024 +
                        lane * 16 + (uint32_t)kbb * 16;
             } else {
                 const char* pb = (const char*)args.ptr_B + (size_t)n0 * ldb;
-                long long bbytes = (long long)(N - 1 - n0) * ldb + Kb;
-                L.rb = make_rsrc(pb, (uint32_t)(bbytes > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : bbytes));
+                L.rb = make_rsrc(pb, rows_bytes(N - n0, ldb, Kb));
                 L.b_kstep = 128;
                 L.b_hstep = 64 * ldb;
                 L.vb = (uint32_t)crow * ldb + ckc * 16 + (uint32_t)kbb;

@@ -16,7 +16,17 @@ NAMES = {(8, 1): "ga_mxfp8_bf16_BpreShuffle_256x256", (8, 0): "ga_mxfp8_bf16_noB
          (4, 1): "ga_mxfp4_bf16_BpreShuffle_256x256", (4, 0): "ga_mxfp4_bf16_noBpreShuffle_256x256"}
 
 
-def run(dev, M, N, K, elem, bps, fa=0, fb=0, l2=0, alpha=1.0, beta=0.0, pad_d=0, seed=1):
+def padded(q, pad, dev):
+    """Codes q [rows, bytes] on the device with rows `pad` bytes of 0x7F (an E4M3
+    NaN) apart, in storage that ends with the last one; the tensor and its stride."""
+    rows, n = q.shape
+    flat = torch.full((rows * (n + pad) - pad,), 0x7F, dtype=torch.uint8, device=dev)
+    flat.as_strided((rows, n), (n + pad, 1)).copy_(torch.from_numpy(np.ascontiguousarray(q)))
+    return flat, n + pad
+
+
+def run(dev, M, N, K, elem, bps, fa=0, fb=0, l2=0, alpha=1.0, beta=0.0, pad_d=0, seed=1, pad_a=0,
+        pad_b=0):
     xa = oracle.gen_mx_input(M, K, seed, 1.0, 4)
     xb = oracle.gen_mx_input(N, K, seed + 1, 1.0, 4)
     if elem == 4:
@@ -25,8 +35,9 @@ def run(dev, M, N, K, elem, bps, fa=0, fb=0, l2=0, alpha=1.0, beta=0.0, pad_d=0,
         (qa, sa), (qb, sb) = oracle.quant_mx8(xa, fa), oracle.quant_mx8(xb, fb)
     sh = f4gemm.Shape(M, N, K, elem_bits=elem)
     t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)  # noqa: E731
-    A = t(qa)
-    B = t(f4gemm.shuffle_weight_16x16(qb, N, sh.Kp()) if bps else qb)
+    A, lda = padded(qa, pad_a, dev)
+    B, ldb = (t(f4gemm.shuffle_weight_16x16(qb, N, sh.Kp())), sh.Kp()) if bps else padded(
+        qb, pad_b, dev)
     SA = t(f4gemm.shuffle_scale(sa, M, K // 32, sh.scale_a_rows(), sh.scale_cols()))
     SB = t(f4gemm.shuffle_scale(sb, N, K // 32, sh.scale_b_rows(), sh.scale_cols()))
     ldd = N + pad_d
@@ -38,6 +49,7 @@ def run(dev, M, N, K, elem, bps, fa=0, fb=0, l2=0, alpha=1.0, beta=0.0, pad_d=0,
     ld = f4gemm.make_launch(cfg, M, N, K, l2)
     args = f4gemm.fill_args(D, C, A, B, SA, SB, M, N, K, ldd, sh.scale_cols(),
                             sh.scale_cols(), alpha, beta, ld.log2_k_split)
+    args.stride_A0, args.stride_B0 = lda * 8 // elem, ldb * 8 // elem
     kern = f4gemm.Kernel().load(None, cfg)
     need = kern.workspace_bytes(ld, M, N) // 4
     # past the bytes the call may use: two slices that no kernel writes
@@ -164,6 +176,20 @@ def test_shape_tile(dev, M, N, K):
     if K % 256 == 0:
         p = run(dev, M, N, 2 * K, 4, 1, alpha=0.5, beta=2.0, seed=K)
         assert p.kernel == _lib.GA_MX_RUNS_SHAPE_TILE
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (12, 8208, 5120, _lib.GA_MX_RUNS_FEW_ROWS), (24, 12288, 8448, _lib.GA_MX_RUNS_FEW_ROWS),
+    (48, 20496, 5120, _lib.GA_MX_RUNS_FEW_ROWS_SHARED_A), (40, 272, 768, _lib.GA_MX_RUNS_K_SPLIT),
+    (300, 784, 1536, _lib.GA_MX_RUNS_K_SPLIT), (1000, 2064, 2048, _lib.GA_MX_RUNS_TILE128),
+    (1000, 8192, 512, _lib.GA_MX_RUNS_TILE128), (5290, 368, 1024, _lib.GA_MX_RUNS_SHAPE_TILE),
+    (2100, 4368, 512, _lib.GA_MX_RUNS_ENTRY)])
+@pytest.mark.parametrize("elem,bps", [(8, 1), (8, 0), (4, 1), (4, 0)])
+def test_strided_operands(dev, M, N, K, kernel, elem, bps):
+    """A and row-major B with NaN codes between their rows and nothing behind the
+    last one, every kernel (row-major B runs some of the shapes on another)."""
+    p = run(dev, M, N, K, elem, bps, seed=K, pad_a=16, pad_b=48)
+    assert elem == 4 or bps == 0 or p.kernel == kernel
 
 
 @pytest.mark.parametrize("elem", [8, 4])

@@ -62,10 +62,10 @@ def descriptors(path):
 
 # Sizes that are no strided rows: MX scales (padded and shuffled, a dense matrix),
 # preshuffled B (16-row groups of K * 16 contiguous bytes) and stream-K's slots.
-DENSE = [r"\(uint32_t\)\(+[()\w ]*M \+ 31\) / 32 \* 32\) \* sna", r"\(uint32_t\)sma \* sna",
+DENSE = [r"\(uint32_t\)\(+(\(int\)args\.)?M \+ 31\) / 32 \* 32\) \* sna", r"\(uint32_t\)sma \* sna",
          r"\(uint32_t\)\(+N \+ 31\) / 32 \* 32\) \* snb", r"\(uint32_t\)smb \* snb",
          r"\(uint32_t\)(ng_here|ngb) \* \(uint32_t\)Kb \* 16", r"kSkSlotFloats \* 4"]
-SOURCES = sorted(glob.glob(os.path.join(CSRC, "gemm_bs*.hip")))
+SOURCES = sorted(glob.glob(os.path.join(CSRC, "gemm_[bm]*.hip")))
 
 
 @pytest.mark.parametrize("path", SOURCES, ids=[os.path.basename(p) for p in SOURCES])
@@ -73,5 +73,6 @@ def test_descriptors_end_with_the_rows(path):
     found = descriptors(path)
     assert all(len(a) == 2 for a in found)
     for _, size in found:
-        assert size.startswith("rows_bytes(") or any(re.fullmatch(d, size) for d in DENSE), size
+        assert re.match(r"(ngb > 0 \? )?rows_bytes\(", size) or any(
+            re.fullmatch(d, size) for d in DENSE), size
     assert found
