@@ -206,3 +206,21 @@ def test_kargs_keep_their_tensors_alive():
         del ka
         gc.collect()
         assert all(r() is None for r in refs)
+
+
+@pytest.mark.parametrize("missing", ["_cuda_getCurrentRawStream", "_cuda_getDevice"])
+def test_stream_handle_without_torchs_raw_stream(monkeypatch, missing):
+    """A torch without the private names the call takes its stream through: the
+    public Stream object's handle."""
+    import torch
+
+    from gcnasm_amd import f4gemm
+
+    class Stream:
+        cuda_stream = 0x5EED
+
+    monkeypatch.delattr(torch._C, missing, raising=False)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream)
+    assert f4gemm._stream_handle(None) == 0x5EED
+    assert f4gemm._stream_handle(Stream) == 0x5EED and f4gemm._stream_handle(7) == 7
