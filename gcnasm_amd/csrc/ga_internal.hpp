@@ -79,9 +79,9 @@ void mx_ksplit_cut(const ga_f4gemm_kargs& args, bool fp4, int gdz, int num_cu, i
 void launch_mx_ksplit(const ga_f4gemm_kargs& args, int gdz, bool bps, bool fp4, int fmt,
                       const ga_splitk_ws_handle* wsh, int num_cu, hipStream_t stream);
 // 128x256 (halves 2) and 128x128 (1) eight-wave kernels, any MX element format,
-// grid of their own tiles.
-void launch_mx_pp_half(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh,
-                       int gdz, bool bps, bool fp4, int fmt, int halves, hipStream_t stream);
+// one K slice, grid of their own tiles.
+void launch_mx_pp_half(const ga_f4gemm_kargs& args, bool bps, bool fp4, int fmt, int halves,
+                       hipStream_t stream);
 
 // Compute units of the current device (queried once per device).
 ga_status device_cu_count(int* num_cu);

@@ -257,15 +257,13 @@ void bs_decode_kernel(ga_opus_gemm_kargs ka, int nwg, int mblocks, int ks, int g
     // tiles shared out over its waves: wave z of the ks sums and stores tiles
     // z, z + ks, ...
     constexpr int NT = NG * TM;
-    if (ks > 1) {
-        float* mine = (float*)ring;
+    float* mine = (float*)ring;
 #pragma unroll
-        for (int c = 0; c < NG; c++)
+    for (int c = 0; c < NG; c++)
 #pragma unroll
-            for (int i = 0; i < TM; i++)
-                *(v4f*)(mine + (i * NG + c) * 256 + lane * 4) = acc[c][i];
-        __syncthreads();
-    }
+        for (int i = 0; i < TM; i++)
+            *(v4f*)(mine + (i * NG + c) * 256 + lane * 4) = acc[c][i];
+    __syncthreads();
     if (!live)
         return;
 
@@ -306,14 +304,6 @@ void bs_decode_kernel(ga_opus_gemm_kargs ka, int nwg, int mblocks, int ks, int g
             }
         }
     };
-    if (ks == 1) {
-#pragma unroll
-        for (int c = 0; c < NG; c++)
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-                store(c, i, acc[c][i]);
-        return;
-    }
     const char* part = smem + tl * ks * Cfg::kWave + lane * 16;
     for (int f = slice; f < NT; f += ks) {
         v4f t = *(const v4f*)(part + f * 1024);

@@ -1240,8 +1240,7 @@ static ga_status kernel_launch(int idx, const ga_f4gemm_kargs* args, int gdx, in
         return GA_OK;
     }
     if (route == MX_ROUTE_HALF || route == MX_ROUTE_QUARTER)
-        launch_mx_pp_half(*args, ws, nullptr, gdz, bps, fp4, fmt, route == MX_ROUTE_HALF ? 2 : 1,
-                          s);
+        launch_mx_pp_half(*args, bps, fp4, fmt, route == MX_ROUTE_HALF ? 2 : 1, s);
     else if (split_groups > 0)
         launch_mx_decode_split(*args, gdz, phys, split_groups, bps, fp4, fmt, ws, wsh, num_cu, s);
     else if (route == MX_ROUTE_SHAPE)

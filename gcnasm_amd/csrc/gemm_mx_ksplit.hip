@@ -50,7 +50,7 @@ struct KsCfg {
 
 __device__ __forceinline__ uint32_t ks_uni(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 
-// Column share wx of nwg, row block mb of mblocks; ks slices of kpt elements
+// Column share wx of nwg, row block mb of mblocks; ks (2, 4 or 8) slices of kpt elements
 // (a multiple of 256) each.
 template <int TM, int NG, bool BPS, bool FP4, int F>
 __global__ __attribute__((amdgpu_flat_work_group_size(64, 512), amdgpu_waves_per_eu(1, 2)))
@@ -250,15 +250,13 @@ void mx_ksplit_kernel(ga_f4gemm_kargs args, int nwg, int mblocks, int ks, int kp
     // K slices summed in slice order: wave z of a task's ks sums and stores
     // its 16x16 tiles z, z + ks, ...
     constexpr int NT = NG * TM;
-    if (ks > 1) {
-        float* mine = (float*)ring;
+    float* mine = (float*)ring;
 #pragma unroll
-        for (int c = 0; c < NG; c++)
+    for (int c = 0; c < NG; c++)
 #pragma unroll
-            for (int i = 0; i < TM; i++)
-                *(v4f*)(mine + (i * NG + c) * 256 + lane * 4) = acc[c][i];
-        __syncthreads();
-    }
+        for (int i = 0; i < TM; i++)
+            *(v4f*)(mine + (i * NG + c) * 256 + lane * 4) = acc[c][i];
+    __syncthreads();
     if (!live)
         return;
     // lane holds C[m][n .. n+3], m = 16i + lane%16, n = 16cg + 4(lane/16); the
@@ -286,14 +284,6 @@ void mx_ksplit_kernel(ga_f4gemm_kargs args, int nwg, int mblocks, int ks, int kp
         pk.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
         *(uint2*)((uint16_t*)args.ptr_D + off) = pk;
     };
-    if (ks == 1) {
-#pragma unroll
-        for (int c = 0; c < NG; c++)
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-                store(c, i, acc[c][i]);
-        return;
-    }
     const char* part = smem + tl * ks * Cfg::kWave + lane * 16;
     for (int f = slice; f < NT; f += ks) {
         v4f t = *(const v4f*)(part + f * 1024);

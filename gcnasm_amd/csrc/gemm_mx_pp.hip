@@ -637,26 +637,17 @@ __device__ __forceinline__ void issue_hs(const PpLoad& L, char* smem, int pair, 
 }
 
 template <int NB, bool BPS, bool FP4, int F>
-__device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restrict__ ws,
-                                             char* smem, int tile_m, int tile_n)
+__device__ __forceinline__ void pp_half_tile(const PpArgs& args, char* smem, int tile_m,
+                                             int tile_n)
 {
     using H = HalfCfg<NB, FP4>;
     constexpr int kEPB = FP4 ? 2 : 1;
-    constexpr int kStepK = 128 * kEPB;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2, simd = wave & 3;
     const int M = (int)args.M, N = (int)args.N, K = (int)args.K;
     const int m0 = tile_m * 128, n0 = tile_n * 128 * NB;
-
-    const int z = blockIdx.z, gdz = gridDim.z;
-    int kpt = K;
-    if (gdz > 1)
-        kpt = ((K >> args.log2_k_split) + 255) / 256 * 256;
-    const int kb = z * kpt;
-    const int ke = min(K, kb + kpt);
-    const int nsteps = (ke - kb) / kStepK;
-    const int kbb = kb / kEPB;
+    const int nsteps = K / (128 * kEPB);
 
     v4f acc[2][4][2]; // [1] is unused with one half
 #pragma unroll
@@ -676,7 +667,7 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
         {
             const char* pa = (const char*)args.ptr_A + (size_t)m0 * lda;
             L.ra = make_rsrc(pa, rows_bytes(M - m0, lda, Kb));
-            L.va = (uint32_t)crow * lda + ckc * 16 + (uint32_t)kbb;
+            L.va = (uint32_t)crow * lda + ckc * 16;
             L.a_hstep = 64 * lda;
             if (BPS) {
                 // copy c (64 columns): groups 4c + wave/2, bytes (wave&1)*1024 + lane*16
@@ -685,21 +676,20 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
                 L.b_kstep = 2048;
                 L.b_hstep = 4 * (uint32_t)Kb * 16;
                 L.vb = (uint32_t)(wave >> 1) * (uint32_t)Kb * 16 + (wave & 1) * 1024 +
-                       lane * 16 + (uint32_t)kbb * 16;
+                       lane * 16;
             } else {
                 const char* pb = (const char*)args.ptr_B + (size_t)n0 * ldb;
                 L.rb = make_rsrc(pb, rows_bytes(N - n0, ldb, Kb));
                 L.b_kstep = 128;
                 L.b_hstep = 64 * ldb;
-                L.vb = (uint32_t)crow * ldb + ckc * 16 + (uint32_t)kbb;
+                L.vb = (uint32_t)crow * ldb + ckc * 16;
             }
             const uint32_t sna = args.stride_ScaleA0, snb = args.stride_ScaleB0;
             L.rsa = make_rsrc(args.ptr_ScaleA, (uint32_t)((M + 31) / 32 * 32) * sna);
             L.rsb = make_rsrc(args.ptr_ScaleB, (uint32_t)((N + 31) / 32 * 32) * snb);
-            L.vsa = ((uint32_t)(m0 / 32 + (wave & 3)) * (sna / 8) + (uint32_t)(kb / 256)) * 256 +
+            L.vsa = (uint32_t)(m0 / 32 + (wave & 3)) * (sna / 8) * 256 + lane * 4;
+            L.vsb = (uint32_t)(n0 / 32 + (NB == 2 ? wave : wave & 3)) * (snb / 8) * 256 +
                     lane * 4;
-            L.vsb = ((uint32_t)(n0 / 32 + (NB == 2 ? wave : wave & 3)) * (snb / 8) +
-                     (uint32_t)(kb / 256)) * 256 + lane * 4;
         }
 
         ReadBase rb;
@@ -814,7 +804,7 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
     const int ldd = (int)args.stride_C0;
     const float alpha = args.alpha, beta = args.beta;
     const bool use_c = beta != 0.0f && args.ptr_C != nullptr;
-    const bool staged = gdz == 1 && !use_c && m0 + 128 <= M && n0 + 128 * NB <= N &&
+    const bool staged = !use_c && m0 + 128 <= M && n0 + 128 * NB <= N &&
                         (ldd & 7) == 0 && ((uintptr_t)args.ptr_D & 15) == 0;
     if (staged) {
         wait_vmcnt<0>();
@@ -857,44 +847,37 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, float* __restri
                 if (m >= M || n >= N)
                     continue;
                 const v4f v = acc[q][i][t];
-                if (gdz > 1) {
-                    *(v4f*)(ws + ((size_t)z * M + m) * N + n) = v;
-                } else {
-                    uint16_t o[4];
-                    const uint16_t* cin =
-                        use_c ? (const uint16_t*)args.ptr_C + (size_t)m * ldd + n : nullptr;
+                uint16_t o[4];
+                const uint16_t* cin =
+                    use_c ? (const uint16_t*)args.ptr_C + (size_t)m * ldd + n : nullptr;
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        float x = alpha * v[j];
-                        if (use_c)
-                            x = x + beta * bf16_to_f32(cin[j]);
-                        o[j] = f32_to_bf16(x);
-                    }
-                    uint2 pk;
-                    pk.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
-                    pk.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
-                    *(uint2*)((uint16_t*)args.ptr_D + (size_t)m * ldd + n) = pk;
+                for (int j = 0; j < 4; j++) {
+                    float x = alpha * v[j];
+                    if (use_c)
+                        x = x + beta * bf16_to_f32(cin[j]);
+                    o[j] = f32_to_bf16(x);
                 }
+                uint2 pk;
+                pk.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
+                pk.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
+                *(uint2*)((uint16_t*)args.ptr_D + (size_t)m * ldd + n) = pk;
             }
         }
 }
 
 template <int NB, bool BPS, bool FP4, int F = 0>
 __global__ __attribute__((amdgpu_flat_work_group_size(kNT, kNT), amdgpu_waves_per_eu(2, 2)))
-void mx_pp_half_kernel(ga_f4gemm_kargs args, float* __restrict__ ws,
-                       const ga_splitk_ws_handle* __restrict__ wsh, int tiles_x, int tiles_y)
+void mx_pp_half_kernel(ga_f4gemm_kargs args, int tiles_x, int tiles_y)
 {
     __shared__ __attribute__((aligned(1024))) char smem[HalfCfg<NB, FP4>::kLds];
-    if (wsh && !(ws = resolve_ws(wsh, gridDim.z, args.M, args.N)))
-        return; // workspace slot shorter than the split-K layout: write nothing
     const PpArgs a = uni_args(args);
     const int ntiles = tiles_x * tiles_y;
     for (int lin = blockIdx.x; lin < ntiles; lin += gridDim.x) {
         int tile_m, tile_n;
         map_tile_lin(lin, tiles_x, tiles_y, kHGroupM, tile_m, tile_n);
-        pp_half_tile<NB, BPS, FP4, F>(a, ws, smem, tile_m, tile_n);
+        pp_half_tile<NB, BPS, FP4, F>(a, smem, tile_m, tile_n);
     }
-    wait_vmcnt<0>(); // copies of steps past the last slice land before exit
+    wait_vmcnt<0>(); // copies of steps past K land before exit
 }
 
 } // namespace
@@ -973,40 +956,38 @@ void launch_mx_pp_fmt(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws
 namespace {
 
 template <int NB, bool BPS, bool FP4, int F>
-void launch_half_n(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh, int gdz,
-                   hipStream_t stream)
+void launch_half_n(const ga_f4gemm_kargs& args, hipStream_t stream)
 {
     const int gdx = ((int)args.N + 128 * NB - 1) / (128 * NB), gdy = ((int)args.M + 127) / 128;
-    hipLaunchKernelGGL((mx_pp_half_kernel<NB, BPS, FP4, F>), dim3(pp_grid(gdx * gdy), 1, gdz),
-                       dim3(kNT), 0, stream, args, ws, wsh, gdx, gdy);
+    hipLaunchKernelGGL((mx_pp_half_kernel<NB, BPS, FP4, F>), dim3(pp_grid(gdx * gdy)), dim3(kNT),
+                       0, stream, args, gdx, gdy);
 }
 
 template <bool FP4, int F>
-void launch_half(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh, int gdz,
-                 bool bps, int halves, hipStream_t stream)
+void launch_half(const ga_f4gemm_kargs& args, bool bps, int halves, hipStream_t stream)
 {
     if (halves == 2)
-        bps ? launch_half_n<2, true, FP4, F>(args, ws, wsh, gdz, stream)
-            : launch_half_n<2, false, FP4, F>(args, ws, wsh, gdz, stream);
+        bps ? launch_half_n<2, true, FP4, F>(args, stream)
+            : launch_half_n<2, false, FP4, F>(args, stream);
     else
-        bps ? launch_half_n<1, true, FP4, F>(args, ws, wsh, gdz, stream)
-            : launch_half_n<1, false, FP4, F>(args, ws, wsh, gdz, stream);
+        bps ? launch_half_n<1, true, FP4, F>(args, stream)
+            : launch_half_n<1, false, FP4, F>(args, stream);
 }
 
 } // namespace
 
-void launch_mx_pp_half(const ga_f4gemm_kargs& args, float* ws, const ga_splitk_ws_handle* wsh,
-                       int gdz, bool bps, bool fp4, int fmt, int halves, hipStream_t stream)
+void launch_mx_pp_half(const ga_f4gemm_kargs& args, bool bps, bool fp4, int fmt, int halves,
+                       hipStream_t stream)
 {
     if (fp4) {
-        launch_half<true, 0>(args, ws, wsh, gdz, bps, halves, stream);
+        launch_half<true, 0>(args, bps, halves, stream);
         return;
     }
     switch (fmt) {
-    case 1: launch_half<false, 1>(args, ws, wsh, gdz, bps, halves, stream); break;
-    case 2: launch_half<false, 2>(args, ws, wsh, gdz, bps, halves, stream); break;
-    case 3: launch_half<false, 3>(args, ws, wsh, gdz, bps, halves, stream); break;
-    default: launch_half<false, 0>(args, ws, wsh, gdz, bps, halves, stream); break;
+    case 1: launch_half<false, 1>(args, bps, halves, stream); break;
+    case 2: launch_half<false, 2>(args, bps, halves, stream); break;
+    case 3: launch_half<false, 3>(args, bps, halves, stream); break;
+    default: launch_half<false, 0>(args, bps, halves, stream); break;
     }
 }
 
