@@ -112,6 +112,8 @@ def test_heuristic_sweep(dev, shape):
 
 @pytest.mark.parametrize("name", [c.knl_name for c in f4gemm.manifest()])
 def test_every_kernel(dev, name):
+    """Each entry on one slice at 300 rows, where the shape rule picks the kernel
+    (test_every_entry_past_one_round has each entry's own)."""
     M, N, K = 300, 2048, 1024
     cfg = cfg_named(name)
     qa, sa, qb, sb = mx_operands(M, N, K, seed=3)
@@ -123,8 +125,9 @@ def test_every_kernel(dev, name):
 @pytest.mark.parametrize("shape", [(300, 2048, 1024), (520, 784, 1536), (256, 256, 128),
                                    (1, 256, 256), (777, 1040, 2048)])
 def test_large_tiles_edge_shapes(dev, name, shape):
-    """Large tiles (in the manifest or found by name only) on shapes with
-    partial M and N tiles, a single K step and a single row."""
+    """Large tiles' entries (in the manifest or found by name only) on shapes with
+    partial M and N tiles, a single K step and a single row: what the shape rule
+    runs for them."""
     M, N, K = shape
     cfg = cfg_named(name)
     assert (cfg in f4gemm.manifest()) == (name not in NAMED_ONLY)
@@ -214,9 +217,11 @@ def test_one_call_mxfp8_gemm_from_float(dev):
           oracle.mx_absdot(qa, sa, qb, sb))
 
 
-# Small-M streaming path of the 256x256 kernels: every M row tile count
-# (M = 1, 16, 17, 33, 64), odd 16-column group counts (N = 784 -> 49 groups),
-# K not a multiple of 256, and each split factor the path handles in-kernel.
+# Up to 64 rows through the 256x256 entries: every M row tile count (M = 1, 16,
+# 17, 33, 64), odd 16-column group counts (N = 784 -> 49 groups), K not a
+# multiple of 256, and each split factor. These weights are small, so the shape
+# rule gives them to the K-split kernel but for 1-16 rows with a split
+# (test_gpu_mx_routes.py has every few-row kernel, with the kernel asserted).
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
 @pytest.mark.parametrize("NKL", [(784, 1152, 0), (784, 1152, 1), (4096, 2048, 0),
                                  (4096, 2048, 1), (4096, 2048, 2), (4096, 2048, 3),
@@ -249,7 +254,8 @@ def test_decode_sequential_slices(dev, M, NKL):
           (M, N, K, ld.gdz), oracle.mx_absdot(qa, sa, qb, sb))
 
 
-# 9-16 rows with at least four 16-column groups per CU and K <= 8192: the
+# 9-16 rows with at least four 16-column groups per CU and K <= 8192 (but
+# (20480, 1152, 0), whose 22 MB of weights the K-split kernel takes): the
 # workgroup's A panel (16 rows x K) is copied into LDS once and the waves read
 # their A fragments there. K = 8192 fills the 128 KB panel; K = 1152 is 9
 # steps; N = 20480 gives five groups per CU; N = 16384 + 64 gives 4 or 5
@@ -271,9 +277,8 @@ def test_decode_a_panel_in_lds(dev, M, NKL):
 @pytest.mark.parametrize("MNK", [(40, 8192, 8192), (64, 8192, 8192), (64, 16384, 1024),
                                  (48, 4096, 2048), (24, 8192, 8192)])
 def test_decode_64_rows_paths(dev, MNK):
-    """17-64 rows in the decode kernel: more steps in flight with one two-group
-    task per CU and long K (N = 8192, K = 8192), eight waves of two groups
-    (N = 16384), one group per wave (N = 4096)."""
+    """17-64 rows of weights up to 96 MB on one slice, long K, many and few
+    columns: the K-split kernel."""
     M, N, K = MNK
     cfg = cfg_named("ga_mxfp8_bf16_BpreShuffle_256x128_splitK")
     qa, sa, qb, sb = mx_operands(M, N, K, seed=M + N, std_b=0.02)
@@ -286,9 +291,8 @@ def test_decode_64_rows_paths(dev, MNK):
 @pytest.mark.parametrize("name", ["ga_mxfp8_bf16_BpreShuffle_256x128_splitK",
                                   "ga_mxfp8_bf16_BpreShuffle_32x512_splitK"])
 def test_few_rows_wide_n(dev, M, name):
-    """33-64 rows over N wide enough for 32x256 B-streaming tiles on 3/4 of
-    the CUs (the path ga_kernel_launch takes there instead of the decode
-    kernel), N not a multiple of 256."""
+    """33-64 rows over wide N that is not a multiple of 256, by two entries: the
+    K-split kernel, whichever tile is named."""
     N, K = 28672 - 16, 512
     cfg = cfg_named(name)
     qa, sa, qb, sb = mx_operands(M, N, K, seed=M + 3, std_b=0.02)
@@ -332,9 +336,9 @@ def test_persistent_many_tiles(dev, name):
 @pytest.mark.parametrize("MNKL", [(64, 8192, 28672, 1), (64, 8192, 32768, 2),
                                   (24, 8192, 16384, 1)])
 def test_decode_deep_k_split(dev, MNKL):
-    """The decode kernel's four-steps-in-flight variant with K split across
-    the waves of a workgroup (2 or 4 slices of at least 64 steps each), for
-    the 33-64-row and 17-32-row instantiations."""
+    """Weights from memory with a caller's 2 or 4 slices of at least 64 steps
+    each, for the 33-64-row and 17-32-row instantiations: slices over
+    workgroups."""
     M, N, K, l2 = MNKL
     cfg = cfg_named("ga_mxfp8_bf16_BpreShuffle_256x128_splitK")
     qa, sa, qb, sb = mx_operands(M, N, K, seed=M + l2, std_b=0.02)
@@ -344,8 +348,11 @@ def test_decode_deep_k_split(dev, MNKL):
           (M, N, K, ld.gdz), oracle.mx_absdot(qa, sa, qb, sb))
 
 
-# (N, K, log2 split) -> 16-column groups per wave on 256 CUs, slices: every
-# groups-per-wave instantiation, ragged last waves, whole rounds of waves.
+# (N, K, log2 split): slices over workgroups, ragged last waves, whole rounds of
+# waves. The comments give the few-row split kernel's 16-column groups per wave on
+# 256 CUs; weights this small run there only for wide N with several slices, the
+# others on the K-split kernel (the plans are asserted in test_gpu_mx_routes.py,
+# which has each number of groups).
 SPLIT_DECODE_SHAPES = [
     (1040, 4096, 2),        # 65 groups x 4 slices: 2 groups, last wave holds one
     (8192 + 48, 2048, 3),   # 515 groups x 8: 6 groups, three rounds
@@ -366,10 +373,9 @@ SPLIT_DECODE_SHAPES = [
 @pytest.mark.parametrize("bps", [True, False])
 @pytest.mark.parametrize("NKL", SPLIT_DECODE_SHAPES)
 def test_decode_split_across_workgroups(dev, M, bps, NKL):
-    """17-64 rows with each wave over several 16-column groups and one K
-    slice, the slices in separate workgroups: partials summed by the split-K
-    reduce in slice order, or with one slice the epilogue in the kernel;
-    preshuffled and row-major B."""
+    """17-64 rows in a caller's slices or one: partials of separate workgroups
+    summed by the split-K reduce in slice order, or the slices summed in a
+    workgroup; preshuffled and row-major B."""
     N, K, l2 = NKL
     name = ("ga_mxfp8_bf16_BpreShuffle_256x256_splitK" if bps else
             "ga_mxfp8_bf16_noBpreShuffle_128x128_splitK")
@@ -381,8 +387,10 @@ def test_decode_split_across_workgroups(dev, M, bps, NKL):
           ("bps" if bps else "plain", M, N, K, ld.gdz), oracle.mx_absdot(qa, sa, qb, sb))
 
 
-# 33-64 rows at one slice over wide N: the shared-A variant (A through an LDS
-# ring). (M, N, K, preshuffled B): eight waves of one group (shares of 6, 5
+# 33-64 rows at one slice over wide N. The shapes are those of the shared-A variant
+# (A through an LDS ring), which takes such N from 96 MB of weights on
+# (test_gpu_mx_routes.py); here the K-split kernel runs them. (M, N, K,
+# preshuffled B): eight waves of one group (shares of 6, 5
 # and 7 groups: waves without a group) with the ring (6 steps) longer than the
 # slice (5 steps), 33 rows; 9 steps (one pass of the main loop and a three-step
 # tail); 7 groups per workgroup as at N = 28672; four waves of 4 groups (N >

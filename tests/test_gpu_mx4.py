@@ -169,8 +169,8 @@ def test_fp4_splitk(dev, l2, name):
 @pytest.mark.parametrize("NKL", [(784, 1280, 0), (784, 1280, 1), (4096, 2048, 0),
                                  (4096, 2048, 2), (1808, 3072, 3)])
 def test_fp4_decode_path(dev, M, NKL):
-    """M <= 64 runs the streaming decode kernel (K slices summed in the
-    workgroup in slice order); results follow the same fp32 step chain."""
+    """Up to 64 rows, K slices summed in slice order: the few-row kernel for 1-16
+    rows with a split, the K-split kernel for the rest of these small weights."""
     N, K, l2 = NKL
     qa, sa, qb, sb = mx4_operands(M, N, K, seed=M * 31 + N + l2)
     name = ("ga_mxfp4_bf16_BpreShuffle_256x256_splitK" if l2 else
@@ -194,8 +194,7 @@ def test_fp4_decode_sequential_slices(dev, M, NKL):
 
 
 def test_fp4_decode_deep(dev):
-    """33-64 rows, one two-group task per CU and long K: the decode kernel
-    with four steps in flight."""
+    """33-64 rows of 64 MB of weights and long K: the K-split kernel."""
     M, N, K = 40, 8192, 16384
     qa, sa, qb, sb = mx4_operands(M, N, K, seed=77)
     got = run_mx4(dev, qa, sa, qb, sb, cfg4("ga_mxfp4_bf16_BpreShuffle_256x128_splitK"), 0)
@@ -205,8 +204,7 @@ def test_fp4_decode_deep(dev):
 @pytest.mark.parametrize("MNKL", [(64, 8192, 32768, 1), (64, 8192, 65536, 2),
                                   (24, 8192, 32768, 1)])
 def test_fp4_decode_deep_k_split(dev, MNKL):
-    """The four-steps-in-flight decode variant with K split across the waves
-    of a workgroup (2 or 4 slices of at least 64 steps each)."""
+    """Weights from memory in a caller's 2 or 4 slices of at least 64 steps each."""
     M, N, K, l2 = MNKL
     qa, sa, qb, sb = mx4_operands(M, N, K, seed=M + l2)
     got = run_mx4(dev, qa, sa, qb, sb, cfg4("ga_mxfp4_bf16_BpreShuffle_256x128_splitK"), l2)
@@ -229,8 +227,7 @@ def test_fp4_persistent_many_tiles(dev, name):
 
 @pytest.mark.parametrize("M", [33, 64])
 def test_fp4_few_rows_wide_n(dev, M):
-    """33-64 rows over wide N run 32x256 B-streaming tiles instead of the
-    decode kernel."""
+    """33-64 rows over wide N that is not a multiple of 256."""
     N, K = 28672 - 16, 512
     qa, sa, qb, sb = mx4_operands(M, N, K, seed=M + 5)
     got = run_mx4(dev, qa, sa, qb, sb, cfg4("ga_mxfp4_bf16_BpreShuffle_256x128_splitK"), 0)
@@ -250,9 +247,7 @@ def test_fp4_decode_plain_b(dev):
                                  (28672 - 16, 512, 0), (28672 - 16, 1024, 1),
                                  (19216, 2048, 2)])
 def test_fp4_decode_split_across_workgroups(dev, M, bps, NKL):
-    """17-64 rows with each wave over several 16-column groups and one K
-    slice, slices in separate workgroups (partials summed by the split-K
-    reduce), or one slice with the epilogue in the kernel."""
+    """17-64 rows in a caller's slices or one, ragged columns."""
     N, K, l2 = NKL
     qa, sa, qb, sb = mx4_operands(M, N, K, seed=M + 9)
     name = ("ga_mxfp4_bf16_BpreShuffle_256x256_splitK" if bps else
@@ -264,11 +259,9 @@ def test_fp4_decode_split_across_workgroups(dev, M, bps, NKL):
 @pytest.mark.parametrize("MNKB", [(64, 32784, 1792, True), (40, 20480, 2304, False),
                                   (33, 24576, 1280, True)])
 def test_fp4_decode_shared_a(dev, MNKB):
-    """33-64 rows at one slice over wide N: the shared-A variant with four
-    waves of 4 groups (N > 32768; 7 steps: a five-step ring and a two-step
-    tail) and eight waves of one group (9 steps against a six-step ring;
-    5 steps, shorter than the ring), MXFP4 operands (one scale dword per
-    step)."""
+    """33-64 rows at one slice over wide N, 5 to 9 steps, at the shapes of the
+    shared-A variant, which takes such N from 96 MB of weights on
+    (test_gpu_mx_routes.py)."""
     M, N, K, bps = MNKB
     qa, sa, qb, sb = mx4_operands(M, N, K, seed=M + K)
     name = ("ga_mxfp4_bf16_BpreShuffle_256x256" if bps else

@@ -75,8 +75,9 @@ def check(got, qa, sa, qb, sb, fa, fb, l2, label, rows=None):
                                      ("ga_mxfp8_bf16_noBpreShuffle_256x256", 0),
                                      ("ga_mxfp8_bf16_noBpreShuffle_128x128_splitK", 1)])
 def test_formats_large_m(dev, fa, fb, name, l2):
-    """More than 64 rows: the 256x256 kernel with the requested formats,
-    partial tiles in M and N, whatever tile the index names."""
+    """More than 64 rows with the requested formats, partial tiles in M and N,
+    whatever tile the index names: the K-split kernel on one slice, the 256x256
+    kernel on more."""
     M, N, K = 300, 784, 1536
     qa, sa, qb, sb = operands(M, N, K, fa, fb, seed=11 + 2 * fa + fb)
     got, ld = run_fmt(dev, qa, sa, qb, sb, cfg_named(name), l2, fa, fb)
@@ -88,9 +89,9 @@ def test_formats_large_m(dev, fa, fb, name, l2):
 @pytest.mark.parametrize("NKL", [(1040, 2048, 0), (1040, 2048, 2), (28672 - 16, 512, 0),
                                  (8192, 2048, 3)])
 def test_formats_decode(dev, fa, fb, M, NKL):
-    """1-64 rows: the decode kernels with the requested formats (in-workgroup
-    at 1-16 rows and narrow N, the split variant at 17-64 rows with a split or
-    over wide N), preshuffled B."""
+    """1-64 rows with the requested formats, preshuffled B: the few-row kernel at
+    1-16 rows with a split, else the K-split kernel (the other few-row kernels:
+    test_few_rows_formats)."""
     N, K, l2 = NKL
     name = "ga_mxfp8_bf16_BpreShuffle_256x256" + ("_splitK" if l2 else "")
     qa, sa, qb, sb = operands(M, N, K, fa, fb, seed=M + N + 3 * fa + fb, std_b=0.02)
@@ -156,13 +157,15 @@ def test_default_formats_equal_plain_launch(dev):
 
 
 @pytest.mark.parametrize("l2", [0, 1])
-def test_every_tile_writes_the_same_bits(dev, l2):
+@pytest.mark.parametrize("M,N,K", [(300, 784, 1536), (520, 13328, 384)])
+def test_every_tile_writes_the_same_bits(dev, l2, M, N, K):
     """Above the decode path every MXFP8 kernel (all tiles, preshuffled and
     row-major B) chains the same 128-K MFMA steps per K slice from zero, so
     the bf16 output is bit-identical whichever entry runs; this is what lets
     ga_kernel_launch_fmt run the 256x256 kernel for any index. Checked over
-    the whole manifest (split entries at l2 = 1), and against the oracle."""
-    M, N, K = 300, 784, 1536
+    the whole manifest (split entries at l2 = 1), and against the oracle. On one
+    slice the small shape runs the K-split kernel for every entry, the large one
+    each entry's own."""
     qa, sa, qb, sb = operands(M, N, K, 0, 0, seed=31 + l2)
     cfgs = [c for c in f4gemm.manifest() if l2 == 0 or c.splitK]
     outs = [run_fmt(dev, qa, sa, qb, sb, c, l2, 0, 0)[0] for c in cfgs]
