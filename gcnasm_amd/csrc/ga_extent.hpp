@@ -24,13 +24,11 @@ constexpr GA_HOST_DEVICE uint32_t rows_bytes(long long rows, long long ld, long 
     return (uint32_t)(n > 0xFFFFFFF0ll ? 0xFFFFFFF0ll : n);
 }
 
-// The same in 32 bits, for rows that the host has checked to lie within 4 GiB
-// (the fp32 scale matrices): a few scalar instructions less before a kernel's
-// first copy, which the 128x256 block-scale tile shows (2048x2560x8192 57.5 us
-// instead of 58.6).
-constexpr GA_HOST_DEVICE uint32_t rows_bytes32(uint32_t rows, uint32_t ld, uint32_t used)
+// The same for fp32 scale matrices, ld and used in floats, in 32 bits: the host
+// has checked that they lie within 4 GiB.
+constexpr GA_HOST_DEVICE uint32_t rows_bytes_f32(uint32_t rows, uint32_t ld, uint32_t used)
 {
-    return (rows - 1) * ld + used;
+    return ((rows - 1) * ld + used) * 4u;
 }
 
 } // namespace ga

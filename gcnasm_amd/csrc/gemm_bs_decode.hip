@@ -119,17 +119,17 @@ void bs_decode_kernel(ga_opus_gemm_kargs ka, int nwg, int mblocks, int ks, int g
         if constexpr (MODE != BD_TENSOR) {
             const float* sfa = (const float*)ka.ptr_sfa + (size_t)b * ka.stride_sfa_batch;
             const float* sfb = (const float*)ka.ptr_sfb + (size_t)b * ka.stride_sfb_batch;
-            rsa = make_rsrc(sfa, rows_bytes32(G, 4u * ka.stride_sfa, 4u * ka.m));
+            rsa = make_rsrc(sfa, rows_bytes_f32(G, ka.stride_sfa, ka.m));
             sa_step = (uint32_t)ka.stride_sfa * 4;
             vsa = ((uint32_t)gb * ka.stride_sfa + m0 + min(lane, M - 1)) * 4;
             if constexpr (MODE == BD_GROUP128) {
                 const int nblk = (N + 127) / 128;
-                rsb = make_rsrc(sfb, rows_bytes32(nblk, 4u * ka.stride_sfb, 4u * G));
+                rsb = make_rsrc(sfb, rows_bytes_f32(nblk, ka.stride_sfb, G));
                 sb_step = 4;
                 vsb = ((uint32_t)min(((cg0 + lane % NG) * 16) / 128, nblk - 1) * ka.stride_sfb +
                        gb) * 4;
             } else {
-                rsb = make_rsrc(sfb, rows_bytes32(G, 4u * ka.stride_sfb, 4u * N));
+                rsb = make_rsrc(sfb, rows_bytes_f32(G, ka.stride_sfb, N));
                 sb_step = (uint32_t)ka.stride_sfb * 4;
                 vsb = ((uint32_t)gb * ka.stride_sfb + min(cg0 * 16 + lane, N - 1)) * 4;
             }

@@ -64,7 +64,7 @@ __device__ __forceinline__ void bs_load_setup(const ga_opus_gemm_kargs& ka, int 
             // SFA [K/128, M]: LDS position w*64 + l holds row
             // w*64 + (l%4)*16 + l/4 (rows past M clamp to M-1)
             const float* sfa = (const float*)ka.ptr_sfa + (size_t)b * ka.stride_sfa_batch;
-            L.rs = make_rsrc(sfa, rows_bytes32(ngroups, 4u * ka.stride_sfa, 4u * M));
+            L.rs = make_rsrc(sfa, rows_bytes_f32(ngroups, ka.stride_sfa, M));
             const int row = min(m0 + wave * 64 + (lane & 3) * 16 + (lane >> 2), M - 1);
             L.vs = (uint32_t)row * 4;
             L.s_kstep = (uint32_t)ka.stride_sfa * 4;
@@ -75,13 +75,13 @@ __device__ __forceinline__ void bs_load_setup(const ga_opus_gemm_kargs& ka, int 
                 // SFB [ceil(N/128), K/128]: positions 0 and 1 hold the
                 // tile's two 128-column blocks
                 const int nblk = (N + 127) / 128;
-                L.rs = make_rsrc(sfb, rows_bytes32(nblk, 4u * ka.stride_sfb, 4u * ngroups));
+                L.rs = make_rsrc(sfb, rows_bytes_f32(nblk, ka.stride_sfb, ngroups));
                 const int nb = min(n0 / 128 + (pos & 1), nblk - 1);
                 L.vs = (uint32_t)nb * ka.stride_sfb * 4;
                 L.s_kstep = 4;
             } else {
                 // SFB [K/128, N]: position c holds column n0 + c
-                L.rs = make_rsrc(sfb, rows_bytes32(ngroups, 4u * ka.stride_sfb, 4u * N));
+                L.rs = make_rsrc(sfb, rows_bytes_f32(ngroups, ka.stride_sfb, N));
                 const int col = min(n0 + pos, N - 1);
                 L.vs = (uint32_t)col * 4;
                 L.s_kstep = (uint32_t)ka.stride_sfb * 4;

@@ -195,7 +195,7 @@ __device__ __forceinline__ BsLoad bs_load_from(const ga_opus_gemm_kargs& ka, int
         const int ngroups = K / 128;
         if (wave < 4) {
             const float* sfa = (const float*)ka.ptr_sfa;
-            L.rs = make_rsrc(sfa, rows_bytes32(ngroups, 4u * ka.stride_sfa, 4u * M));
+            L.rs = make_rsrc(sfa, rows_bytes_f32(ngroups, ka.stride_sfa, M));
             const int row = min(m0 + wave * 64 + (lane & 3) * 16 + (lane >> 2), M - 1);
             L.s_kstep = (uint32_t)ka.stride_sfa * 4;
             L.vs = (uint32_t)row * 4 + (uint32_t)g0 * L.s_kstep;
@@ -204,12 +204,12 @@ __device__ __forceinline__ BsLoad bs_load_from(const ga_opus_gemm_kargs& ka, int
             const int pos = (wave - 4) * 64 + lane;
             if (MODE == PS_GROUP128) {
                 const int nblk = (N + 127) / 128;
-                L.rs = make_rsrc(sfb, rows_bytes32(nblk, 4u * ka.stride_sfb, 4u * ngroups));
+                L.rs = make_rsrc(sfb, rows_bytes_f32(nblk, ka.stride_sfb, ngroups));
                 const int nb = min(n0 / 128 + (pos & 1), nblk - 1);
                 L.s_kstep = 4;
                 L.vs = (uint32_t)nb * ka.stride_sfb * 4 + (uint32_t)g0 * 4;
             } else {
-                L.rs = make_rsrc(sfb, rows_bytes32(ngroups, 4u * ka.stride_sfb, 4u * N));
+                L.rs = make_rsrc(sfb, rows_bytes_f32(ngroups, ka.stride_sfb, N));
                 const int col = min(n0 + pos, N - 1);
                 L.s_kstep = (uint32_t)ka.stride_sfb * 4;
                 L.vs = (uint32_t)col * 4 + (uint32_t)g0 * L.s_kstep;

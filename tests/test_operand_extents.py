@@ -1,6 +1,7 @@
 """What the GEMM kernels may read of a strided operand or scale matrix (CPU only):
-rows_bytes and rows_bytes32, the extent of a buffer descriptor, against the bytes that the rows
-use, and every kernel's descriptors, which must be built with it."""
+rows_bytes and rows_bytes_f32, the extent of a buffer descriptor, against the
+bytes that the rows use, and every kernel's descriptors, which must be built with
+them."""
 import glob
 import os
 import re
@@ -25,7 +26,7 @@ int main()
             for (long long pad : pad_of) {
                 const long long ld = used + pad, storage = (rows - 1) * ld + used;
                 bad += (long long)ga::rows_bytes(rows, ld, used) != storage;
-                bad += (long long)ga::rows_bytes32(rows, ld, used) != storage;
+                bad += (long long)ga::rows_bytes_f32(rows, ld / 4, used / 4) != storage;
             }
     // at most 4 GiB less 16 bytes
     bad += ga::rows_bytes(256, 1ll << 26, 1ll << 26) != 0xFFFFFFF0u;
@@ -74,6 +75,6 @@ def test_descriptors_end_with_the_rows(path):
     found = descriptors(path)
     assert all(len(a) == 2 for a in found)
     for _, size in found:
-        assert re.match(r"(ngb > 0 \? )?rows_bytes(32)?\(", size) or any(
+        assert re.match(r"(ngb > 0 \? )?rows_bytes(_f32)?\(", size) or any(
             re.fullmatch(d, size) for d in DENSE), size
     assert found
