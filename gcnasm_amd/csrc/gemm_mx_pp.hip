@@ -833,7 +833,6 @@ __device__ __forceinline__ void pp_half_tile(const PpArgs& args, char* smem, int
             *(v4i*)(dst + (size_t)row * ldd + col) =
                 *(const v4i*)(smem + row * kStagePitch + col * 2);
         }
-        barrier_lds(); // staged rows read before the LDS takes the next tile's copies
         return;
     }
 #pragma unroll
@@ -870,13 +869,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kNT, kNT), amdgpu_waves_pe
 void mx_pp_half_kernel(ga_f4gemm_kargs args, int tiles_x, int tiles_y)
 {
     __shared__ __attribute__((aligned(1024))) char smem[HalfCfg<NB, FP4>::kLds];
+    // A workgroup per tile: the rule that picks these tiles has them fit on the
+    // CUs in one round. alpha and beta are fetched with the other arguments, not
+    // in a fetch of their own that the tile's first copies wait for.
     const PpArgs a = uni_args(args);
-    const int ntiles = tiles_x * tiles_y;
-    for (int lin = blockIdx.x; lin < ntiles; lin += gridDim.x) {
-        int tile_m, tile_n;
-        map_tile_lin(lin, tiles_x, tiles_y, kHGroupM, tile_m, tile_n);
-        pp_half_tile<NB, BPS, FP4, F>(a, smem, tile_m, tile_n);
-    }
+    asm volatile("" ::"v"(a.alpha), "v"(a.beta));
+    int tile_m, tile_n;
+    map_tile_lin(blockIdx.x, tiles_x, tiles_y, kHGroupM, tile_m, tile_n);
+    pp_half_tile<NB, BPS, FP4, F>(a, smem, tile_m, tile_n);
     wait_vmcnt<0>(); // copies of steps past K land before exit
 }
 
@@ -959,8 +959,8 @@ template <int NB, bool BPS, bool FP4, int F>
 void launch_half_n(const ga_f4gemm_kargs& args, hipStream_t stream)
 {
     const int gdx = ((int)args.N + 128 * NB - 1) / (128 * NB), gdy = ((int)args.M + 127) / 128;
-    hipLaunchKernelGGL((mx_pp_half_kernel<NB, BPS, FP4, F>), dim3(pp_grid(gdx * gdy)), dim3(kNT),
-                       0, stream, args, gdx, gdy);
+    hipLaunchKernelGGL((mx_pp_half_kernel<NB, BPS, FP4, F>), dim3(gdx * gdy), dim3(kNT), 0,
+                       stream, args, gdx, gdy);
 }
 
 template <bool FP4, int F>
