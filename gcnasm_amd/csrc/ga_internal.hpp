@@ -92,7 +92,7 @@ void launch_bs_pp(const ga_opus_gemm_kargs& ka, int mode, int out_dtype, hipStre
 void launch_bs_half(const ga_opus_gemm_kargs& ka, int mode, int out_dtype, int halves,
                     hipStream_t stream);
 // The 256x256 kernel's stream-K form (batch 1): workgroups it would use on
-// num_cu CUs (0: the whole-tile form is the better one), its workspace
+// num_cu CUs (0: not this form), its workspace
 // (per-tile counters, zero between calls, then 2 * nwg fp32 partial tiles),
 // the counters' share of it, and the launch.
 int bs_sk_workgroups(const ga_opus_gemm_kargs& ka, int num_cu);

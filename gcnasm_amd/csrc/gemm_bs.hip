@@ -239,8 +239,8 @@ static BsPath bs_path(const ga_opus_gemm_kargs& ka, int num_cu)
     // instead of 64, counts for more than the split (K-split / 64x256, 64 rows:
     // 40960x4096 29.9 / 31.2 us, 57344x4096 42.9 / 37.9, 129280x7168 229 / 174,
     // 16 batches of 4096x7168 139 / 89, 24 of 2048x2048 25.4 / 23.5).
-    // More rows: the smallest tile whose
-    // tiles fit on the CUs in one round (128x128, 128x256), else 256x256
+    // More rows: the smallest tile whose tiles fit on the CUs in one round
+    // (128x128, 128x256), else 256x256
     // (measured on MI355X, GROUP_N 128, bf16 C, 128x128 / 128x256 / 256x256:
     // 512x8192x8192 45.4 / 59.0 / 85.8 us, 1000x8192x8192 87.3 / 71.9 / 88.7,
     // 2048x8192x8192 177 / 147 / 118), and up to 1024 rows, as far as it was
@@ -362,7 +362,7 @@ static ga_status check_blockscale(const ga_opus_gemm_kargs* kargs, int group_n, 
 }
 
 // Workgroups of the stream-K form for these kargs on this device (0: the
-// call runs whole tiles).
+// call runs as without a workspace).
 static ga_status bs_stream_k_plan(const ga_opus_gemm_kargs& ka, int* nwg)
 {
     int num_cu = 0;

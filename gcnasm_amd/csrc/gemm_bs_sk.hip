@@ -1,6 +1,7 @@
 // gemm_bs_sk.hip -- stream-K form of the 256x256 fp32-scaled FP8 GEMM
 // (DeepSeek block scale, batch 1), for long-K problems whose 256x256 tiles
-// keep few CUs busy (2048 x 2560 x 8192: 80 tiles on 256 CUs).
+// keep few CUs busy (2048 x 2560 x 8192: 80 tiles on 256 CUs) and whose caller
+// passes a workspace.
 //
 // With T = tiles * G iterations (G = K / 128 groups per tile) and P
 // workgroups (one per CU), virtual workgroup v computes iterations
@@ -572,15 +573,15 @@ int bs_sk_workgroups(const ga_opus_gemm_kargs& ka, int num_cu)
         return 0;
     const long long tiles = (long long)((ka.n + 255) / 256) * ((ka.m + 255) / 256);
     const long long iters = tiles * (ka.k / 128);
-    // Worth it only when whole tiles would keep at most 40 % of the CUs busy
-    // in their one round, with at least 16 128-K groups per workgroup
-    // (measured on MI355X, bf16 C, best of 3 x 100 calls: 80 tiles on 256
-    // CUs, K = 8192: 103.1 -> 83.9 us; 99 tiles: 80.0 -> 78.1; 112 tiles:
-    // 80.6 -> 81.3; 144 tiles, K = 7168: 94.7 -> 96.9; 448 tiles: 72.3 ->
-    // 82.6): the partial tiles' device-coherent traffic and the last
-    // arrival's sum cost about as much as a third of the CUs idling.
-    // (256x256 whole tiles. A call without a workspace runs 128x256 or 128x128
-    // tiles here, which are faster: 80 tiles, K = 8192, 67 against 92 us.)
+    // Only where 256x256 tiles would keep at most 40 % of the CUs busy in their
+    // one round, with at least 16 128-K groups per workgroup: with more tiles the
+    // partial tiles' device-coherent traffic and the last arrival's sum cost more
+    // than the idle CUs (MI355X, bf16 C, whole 256x256 tiles / this form: 80 tiles
+    // on 256 CUs, K = 8192, 103.1 / 83.9 us; 99 tiles 80.0 / 78.1; 112 tiles
+    // 80.6 / 81.3; 144 tiles, K = 7168, 94.7 / 96.9; 448 tiles 72.3 / 82.6).
+    // A call without a workspace runs 128x256 tiles on these shapes, which are
+    // faster than either (80 tiles, K = 8192, on other data, 57 us, this form 94):
+    // the form is what a caller asks for with a workspace, not a gain.
     if (tiles * 5 > 2ll * nwg || iters < 16ll * nwg)
         return 0;
     return nwg;

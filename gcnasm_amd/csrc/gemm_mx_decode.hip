@@ -1,8 +1,9 @@
 // gemm_mx_decode.hip -- MXFP8 GEMM for small M (decode), HBM-streaming.
 //
 // Used by every manifest kernel for M <= 64 rows where the weights are large
-// enough to come from HBM (the K-split kernel of gemm_mx_ksplit.hip takes the
-// smaller ones; mx_route in gemm_mx.hip has the line). With so few rows the
+// enough to come from HBM, or the caller's split suits it better than the
+// K-split kernel of gemm_mx_ksplit.hip, which takes the rest
+// (mx_few_rows_ksplit in gemm_mx.hip has the lines). With so few rows the
 // GEMM is a stream over B (N x K bytes), so the design is about keeping HBM
 // busy:
 //  * one wave per NG 16-column groups of B and one K slice; B's 2 KB per

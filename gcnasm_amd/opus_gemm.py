@@ -89,7 +89,7 @@ def workspace_bytes(kargs):
 
 def stream_k_workgroups(m, n, k, batch=1):
     """Workgroups of the stream-K form ga_gemm_a8w8_blockscale_ws runs for
-    these sizes on the current device (0: whole tiles)."""
+    these sizes on the current device (0: as without a workspace)."""
     ka = opus_gemm_kargs()
     ka.m, ka.n, ka.k, ka.batch = m, n, k, batch
     w = ctypes.c_int(0)

@@ -424,8 +424,9 @@ ga_status ga_kernel_launch_fmt(int idx, const ga_f4gemm_kargs* args, int gdx, in
                                void* stream);
 
 /* One-call MXFP8 GEMM: select_kernel + make_launch + fill_args + launch.
- * log2_k_split as in ga_select_kernel. Writes the chosen kernel index and
- * launch into *chosen / *ld_out when non-NULL. */
+ * log2_k_split as in ga_select_kernel. Writes the manifest entry that it
+ * chooses and its launch into *chosen / *ld_out when non-NULL; the kernel that
+ * such a launch runs depends on the shape (ga_kernel_plan). */
 ga_status ga_mxfp8_gemm(void* d_D, const void* d_A, const void* d_B,
                         const void* d_ScaleA, const void* d_ScaleB, int M, int N, int K,
                         int stride_D0, int bpreshuffle, int log2_k_split, int num_cu,
@@ -464,29 +465,30 @@ ga_status ga_fp8_gemm_per_tensor(const ga_opus_gemm_kargs* kargs, int out_dtype,
  * chain. Lets a caller (or a test) reproduce the rounding exactly. */
 ga_status ga_blockscale_k_slices(const ga_opus_gemm_kargs* kargs, int* groups_per_slice);
 
-/* ga_gemm_a8w8_blockscale with a caller workspace, which lets long-K
- * problems whose 256x256 tiles would keep few CUs busy (batch 1, more than
- * 64 rows, tiles for at most 40 % of the CUs, at least 16 128-K groups per
- * CU; e.g. 2048x2560x8192: 80 tiles on 256 CUs, 103 -> 84 us on MI355X)
- * run in stream-K form: every CU takes an equal share of the tiles' 128-K
- * groups, and a tile cut between CUs is summed from fp32 partials in K
- * order by the last CU to finish it (the DeepSeek configuration shapes are
- * not among them: their partial traffic costs as much as the balance
- * gains). The reference's kernel has no split, and its cross-workgroup
+/* ga_gemm_a8w8_blockscale with a caller workspace, which makes long-K
+ * problems with few tiles (batch 1, more than 64 rows, 256x256 tiles for at
+ * most 40 % of the CUs, 128x128 tiles for more than one round, at least 16
+ * 128-K groups per CU; e.g. 2048x2560x8192) run in stream-K form: every CU
+ * takes an equal share of the 256x256 tiles' 128-K groups, and a tile cut
+ * between CUs is summed from fp32 partials in K order by the last CU to
+ * finish it. It is kept for callers that want that form and its K cuts, not
+ * for speed: without a workspace these calls run 128x256 tiles, which are
+ * faster (MI355X, bf16 C, stream-K / without: 2048x2560x8192 94 / 57 us,
+ * 1280x4096x8192 91 / 57, 2304x2816x8192 106 / 58, 1100x4000x28672 247 / 182).
+ * The reference's kernel has no split, and its cross-workgroup
  * counter (wmma_opus_rdna4/opus/opus.hpp:1296-1304) spins, where here nobody
  * waits. workspace: ga_blockscale_workspace_bytes bytes (up to about 128
  * MiB), zero-filled before its first use (on the call's stream, or waited
  * for before the call: a hipMemset queues on the null stream, which does not
  * order against non-blocking streams) and left zero-filled by every call;
  * calls that overlap in time must not share it. workspace NULL,
- * or a shape the whole-tile kernel suits, runs exactly
- * ga_gemm_a8w8_blockscale; a workspace that is too small is
+ * or any other shape, runs exactly ga_gemm_a8w8_blockscale; a workspace that is too small is
  * GA_ERR_WORKSPACE. Summation order: ga_blockscale_stream_k. */
 ga_status ga_gemm_a8w8_blockscale_ws(const ga_opus_gemm_kargs* kargs, int group_n, int out_dtype,
                                      void* workspace, size_t workspace_bytes, void* stream);
 
 /* Workspace ga_gemm_a8w8_blockscale_ws can use for these kargs on the
- * current device (0: it runs the whole-tile kernel). */
+ * current device (0: it runs ga_gemm_a8w8_blockscale). */
 ga_status ga_blockscale_workspace_bytes(const ga_opus_gemm_kargs* kargs, size_t* bytes);
 
 /* No counterpart in the reference (whose cross-workgroup counter has no
@@ -502,7 +504,8 @@ ga_status ga_blockscale_workspace_check(const ga_opus_gemm_kargs* kargs, void* w
                                         size_t workspace_bytes, void* stream);
 
 /* Stream-K plan of ga_gemm_a8w8_blockscale_ws (given a workspace) on the
- * current device: *workgroups = P, or 0 when that call runs whole tiles.
+ * current device: *workgroups = P, or 0 when that call runs
+ * ga_gemm_a8w8_blockscale.
  * With G = K/128 and T = tiles * G, iteration t*G + g is 128-K group g of
  * tile t, and workgroup v computes iterations [floor(v*T/P),
  * floor((v+1)*T/P)). Tiles are numbered in bands of four tile rows, column
