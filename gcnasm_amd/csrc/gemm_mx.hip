@@ -43,6 +43,7 @@
 #include "ga_internal.hpp"
 #include "ga_pp.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstring>
@@ -1057,17 +1058,21 @@ static MxRoute mx_route(const ga_f4gemm_kargs& a, bool fp4, bool bps, int fmt, i
     MxRoute tile = one ? MX_ROUTE_QUARTER : MX_ROUTE_HALF;
     float ksplit_us = mx_ksplit_estimate_us(a, fp4, num_cu);
     if (M > 1024) {
-        // Past the rows its estimate was fitted on (1000), the K-split kernel takes
-        // up to 1.3 times as long (2048x512x8192: estimate 19.0, measured 24.5).
-        // And where at most half the CUs have a 128x128 tile, and N has 256
-        // columns, the four-wave tiles of twice as many workgroups are faster
-        // (4096x512x8192 30.8 us, 128x128 34.3, K-split 41.4; 3000x512x4096 17.3 /
-        // 20.4 / 21.5, MXFP4 4096x512x4096 11.9 / 14.6 / 12.9; 16384x128x8192 40.4 /
-        // 34.4 / 42.0).
-        ksplit_us *= 1.2f;
-        if (bps && fmt == 0 && 2 * quarters <= num_cu && N >= 256) {
+        // Past the rows its estimate was fitted on (1000) the K-split kernel takes
+        // longer with more row blocks, up to 1.3 times from 2304 rows on, where K
+        // is not short (1500x512x8192: estimate 19.0, measured 20.7; 2048x512x8192
+        // 19.0 / 24.5; 2564x640x7168 29.4 / 36.5; but 2862x368x2048 11.5 / 10.9).
+        if (K >= (fp4 ? 4096 : 3072))
+            ksplit_us *= 1.0f + 0.2f * std::min(1.0f, std::max(0.0f, (float)(M - 1152) / 1152.0f));
+        // And where at most half the CUs have a 128x128 tile, and N has 256 columns,
+        // the four-wave tiles of 32 rows are faster than it (4096x512x8192 30.8 us,
+        // 128x128 34.3, K-split 41.4; 3000x512x4096 17.3 / 20.4 / 21.5, MXFP4
+        // 4096x512x4096 11.9 / 14.6 / 12.9; 16384x128x8192 40.4 / 34.4 / 42.0), while
+        // they are one round (1737x1040x4096, 275 of them, 31.4 / 21.2).
+        if (bps && fmt == 0 && 2 * quarters <= num_cu && N >= 256 &&
+            (M + 31) / 32 * ((N + 255) / 256) <= num_cu) {
             tile = MX_ROUTE_SHAPE;
-            tile_us = 5.4f + 0.38f * steps;
+            tile_us = 5.8f + (fp4 ? 0.42f : 0.39f) * steps;
         }
     }
     return ksplit_us < tile_us ? MX_ROUTE_KSPLIT : tile;

@@ -64,6 +64,12 @@ ROUTES = [
     (P8, 32, 1024, 12288, 3, SPLIT), (P8, 32, 2048, 12288, 3, KSPLIT),
     # more rows: the K-split kernel up to a quarter of the CUs with a 128x128 tile,
     # the shape's four-wave tile up to half, 128x128, 128x256, the entry's own
+    # (the four-wave tile for one round of 32x256 and long K only)
+    (P8, 1536, 1040, 4096, 0, SHAPE), (P8, 1737, 1040, 4096, 0, KSPLIT),
+    (P8, 2865, 592, 4096, 0, TILE128), (P8, 2564, 640, 7168, 0, SHAPE),
+    (P8, 2815, 560, 1536, 0, KSPLIT), (P8, 1700, 1120, 512, 0, KSPLIT),
+    (P8, 1100, 1040, 2048, 0, KSPLIT), (P8, 3204, 464, 1536, 0, KSPLIT),
+    (P4, 4812, 288, 3072, 0, KSPLIT), (P4, 1991, 768, 3072, 0, KSPLIT),
     (P8, 1000, 512, 8192, 0, KSPLIT), (P8, 2048, 512, 8192, 0, KSPLIT), (P8, 3000, 512, 8192, 0, SHAPE),
     (P8, 8192, 256, 4096, 0, SHAPE), (P4, 4096, 512, 4096, 0, SHAPE), (P8, 1500, 1040, 8192, 0, SHAPE),
     (P8, 16384, 128, 8192, 0, TILE128), (P8R, 4096, 512, 8192, 0, TILE128),
