@@ -5,7 +5,8 @@
 One "step" is one MXFP8 GEMM D[8192, 8192] bf16 = A[8192, 8192] * B[8192, 8192]^T
 (E4M3 operands, E8M0 scale per 1x32 K-block, B 16x16-preshuffled, scales
 padded + shuffled), inputs resident in HBM, launched through the library's
-C ABI (select_kernel -> make_launch -> fill_args -> kernel launch). Inputs are
+C ABI (select_kernel -> make_launch -> fill_args -> kernel launch; "kernel"
+names the manifest entry chosen, ga_kernel_plan tells the kernel it runs). Inputs are
 synthetic: N(0,1) values scaled by 2^u per 1x32 block (u uniform in [-4, 4]),
 quantised on the GPU by the library's MX quantiser (scale rule floor(log2(amax/448))).
 
