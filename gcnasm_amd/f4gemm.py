@@ -206,13 +206,14 @@ def shuffle_scale(src, rows, cols, sm, sn):
 def _stream_handle(stream):
     if stream is None:
         import torch
-        # the current stream's handle without the Stream object around it: 0.2 us
-        # a call instead of 2.8, of the 20 of a small layer. The two names are
-        # torch's own, so a version may come without them.
-        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-        device = getattr(torch._C, "_cuda_getDevice", None)
-        if raw is not None and device is not None and torch.cuda.is_initialized():
-            return raw(device())
+        if torch.cuda.is_initialized():
+            # the current stream's handle without the Stream object around it:
+            # 0.2 us a call instead of 2.8, of the 20 of a small layer. The two
+            # names are torch's own, so a version may come without them.
+            try:
+                return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+            except AttributeError:
+                pass
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, int):
         return stream
